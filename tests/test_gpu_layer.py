@@ -219,6 +219,25 @@ def test_argmax_reference_cases_and_full_vocab(vo, gpu_backend):
     assert np.array_equal(gpu_backend.argmax(_dev(b16, torch.bfloat16)), orc.argmax(b16))
 
 
+@pytest.mark.parametrize("cols", [1, 255, 1020, 1023, 1024, 4096, 4100, 8191, 8200, 32772, 65544])
+@pytest.mark.parametrize("bf16", [False, True])
+def test_argmax_row_widths(vo, gpu_backend, cols, bf16):
+    """Rows that are and are not whole 16-byte words, below, at and past one
+    pass of the workgroup; the maximum in the first, the last and a middle
+    column, twice, -inf everywhere, and a NaN in the last column."""
+    import torch
+    _say(f"argmax {cols} {'bf16' if bf16 else 'f32'}")
+    x = W.round_bf16(np.random.default_rng(cols).uniform(-1, 1, (6, cols)).astype(np.float32))
+    x[0, 0] = x[1, cols - 1] = x[2, cols // 2] = 7.0
+    x[3, cols // 3] = x[3, cols - 1] = 7.0
+    x[4] = -np.inf
+    dt = torch.bfloat16 if bf16 else torch.float32
+    assert np.array_equal(gpu_backend.argmax(_dev(x, dt)), orc.argmax(x))
+    x[5, cols - 1] = np.nan
+    with pytest.raises(vo.NaNError):
+        gpu_backend.argmax(_dev(x, dt))
+
+
 def test_embed_exact_and_vocab_check(vo, gpu_backend):
     import torch
     _say("embed")

@@ -266,36 +266,67 @@ __device__ __forceinline__ float load_logit(const void *p, uint64_t k, bool f32)
 
 // Backend::argmax: ids[r] = first index of row r's maximum, or 0xffffffff
 // when the row holds a NaN (EngineError::NaN, reported by the host).  One
-// workgroup per row; each thread scans its columns in increasing order with
-// a strict '>', then the (value, index) pairs merge by `beats`.  V4: f32
-// rows read as 16-byte words (cols % 4 == 0).
-template <bool F32, bool V4>
-__global__ __launch_bounds__(kThreads) void argmax_kernel(const void *__restrict__ logits,
-                                                          uint32_t cols,
-                                                          uint32_t *__restrict__ ids) {
-    __shared__ float lds_v[4];
-    __shared__ uint32_t lds_i[4];
-    __shared__ int lds_nan[4];
+// workgroup of T threads per row; a thread reads VPL values at a time (16
+// bytes: f32 with V = 4, bf16 with V = 8; V = 1 where the row is no whole
+// number of such words), U of them before it looks at the first, and keeps
+// the first maximum of its own columns, which it sees in increasing order
+// (strict '>'); the (value, index) pairs then merge by `beats`.
+//
+// Bound: how much one CU keeps in flight, since a greedy step has few rows
+// and each is one workgroup's (a second level over several workgroups would
+// need a workspace, which the op's callers do not give).  With 256 threads
+// and one load in flight a 128256-column f32 row took 42 us (12 GB/s) and 40
+// rows 60 us; with 1024 threads and eight loads each (128 KiB in flight) 9 us
+// for 1 to 40 rows, 23 us for 256 (131 MB, 5.8 TB/s).
+template <bool F32, int V, int T>
+__global__ __launch_bounds__(T) void argmax_kernel(const void *__restrict__ logits, uint32_t cols,
+                                                   uint32_t *__restrict__ ids) {
+    constexpr int U = V == 1 ? 4 : 8;
+    constexpr int W = T / 64;
+    __shared__ float lds_v[W];
+    __shared__ uint32_t lds_i[W];
+    __shared__ int lds_nan[W];
     const uint32_t r = blockIdx.x;
     const uint64_t base = static_cast<uint64_t>(r) * cols;
     ArgBest b{-__builtin_inff(), 0xffffffffu};
     bool nan = false;
-    if constexpr (F32 && V4) {
-        const floatx4 *row = reinterpret_cast<const floatx4 *>(static_cast<const float *>(logits) + base);
-        for (uint32_t q = threadIdx.x; q < cols / 4; q += kThreads) {
-            const floatx4 v = row[q];
+    auto take = [&](float v, uint32_t c) {
+        nan |= v != v;
+        if (b.i == 0xffffffffu || v > b.v) b = ArgBest{v, c};
+    };
+    // The values at word q of the row (V columns from V q on).
+    auto words = [&](const u32x4 &w, uint32_t q) {
+        if constexpr (F32) {
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                nan |= v[k] != v[k];
-                const ArgBest o{v[k], 4 * q + k};
-                if (b.i == 0xffffffffu || o.v > b.v) b = o;
-            }
+            for (int k = 0; k < 4; ++k) take(__uint_as_float(w[k]), 4 * q + k);
+        } else {
+            float f[8];
+            unpack8(w, f);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) take(f[k], 8 * q + k);
         }
-    } else {
-        for (uint32_t c = threadIdx.x; c < cols; c += kThreads) {
-            const float v = load_logit(logits, base + c, F32);
-            nan |= v != v;
-            if (b.i == 0xffffffffu || v > b.v) b = ArgBest{v, c};
+    };
+    const uint32_t n = cols / V;  // words of the row
+    const uint32_t passes = n / (U * T) + (n % (U * T) != 0);
+    for (uint32_t p = 0; p < passes; ++p) {
+        // Words past the row load its last one and are not looked at.
+        const uint32_t q0 = p * (U * T) + threadIdx.x;
+        if constexpr (V > 1) {
+            const u32x4 *row = reinterpret_cast<const u32x4 *>(
+                static_cast<const uint8_t *>(logits) + base * (F32 ? 4 : 2));
+            u32x4 w[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) w[u] = row[min(q0 + u * T, n - 1)];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (q0 + u * T < n) words(w[u], q0 + u * T);
+        } else {
+            float w[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) w[u] = load_logit(logits, base + min(q0 + u * T, n - 1), F32);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (q0 + u * T < n) take(w[u], q0 + u * T);
         }
     }
 #pragma unroll
@@ -313,13 +344,14 @@ __global__ __launch_bounds__(kThreads) void argmax_kernel(const void *__restrict
     __syncthreads();
     if (threadIdx.x == 0) {
         ArgBest t{lds_v[0], lds_i[0]};
-        int n = lds_nan[0];
-        for (int k = 1; k < 4; ++k) {
+        int any = lds_nan[0];
+#pragma unroll
+        for (int k = 1; k < W; ++k) {
             const ArgBest x{lds_v[k], lds_i[k]};
             if (beats(x, t)) t = x;
-            n |= lds_nan[k];
+            any |= lds_nan[k];
         }
-        ids[r] = n ? 0xffffffffu : t.i;
+        ids[r] = any ? 0xffffffffu : t.i;
     }
 }
 
@@ -494,16 +526,26 @@ hipError_t launch_argmax(const void *logits, bool f32, uint32_t rows, uint32_t c
                          hipStream_t stream) {
     if (rows == 0) return hipSuccess;
     KernelTimer timer("argmax", stream);
-    const bool v4 = f32 && cols % 4 == 0;
-    if (f32 && v4)
-        hipLaunchKernelGGL((argmax_kernel<true, true>), dim3(rows), dim3(kThreads), 0, stream, logits,
-                           cols, ids);
-    else if (f32)
-        hipLaunchKernelGGL((argmax_kernel<true, false>), dim3(rows), dim3(kThreads), 0, stream,
-                           logits, cols, ids);
-    else
-        hipLaunchKernelGGL((argmax_kernel<false, false>), dim3(rows), dim3(kThreads), 0, stream,
-                           logits, cols, ids);
+    // 16-byte reads where every row starts on a 16-byte boundary; 1024 threads
+    // once a row has a word for each.
+    const uint32_t per_word = f32 ? 4 : 8;
+    const bool wide = cols % per_word == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0;
+#define VO_ARGMAX(F32, V, T) \
+    hipLaunchKernelGGL((argmax_kernel<F32, V, T>), dim3(rows), dim3(T), 0, stream, logits, cols, ids)
+    if (wide) {
+        const bool large = cols / per_word >= 1024;
+        if (f32 && large) VO_ARGMAX(true, 4, 1024);
+        else if (f32) VO_ARGMAX(true, 4, 256);
+        else if (large) VO_ARGMAX(false, 8, 1024);
+        else VO_ARGMAX(false, 8, 256);
+    } else {
+        const bool large = cols >= 1024;
+        if (f32 && large) VO_ARGMAX(true, 1, 1024);
+        else if (f32) VO_ARGMAX(true, 1, 256);
+        else if (large) VO_ARGMAX(false, 1, 1024);
+        else VO_ARGMAX(false, 1, 256);
+    }
+#undef VO_ARGMAX
     return hipGetLastError();
 }
 
