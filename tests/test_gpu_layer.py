@@ -81,8 +81,8 @@ def test_matmul_reference_shape_generic_kernel(vo, gpu_backend):
                                       (16, 1024, 14336), (300, 1024, 14336), (1280, 512, 4096),
                                       (4, 1024, 256), (17, 512, 4096)])
 def test_matmul_vs_float64(vo, gpu_backend, rows, n, k):
-    """Up to 4 rows run on the weight-streaming kernel (K a multiple of
-    2048), the rest on hipBLASLt."""
+    """Up to 16 rows (64 where K is at most twice the outputs) run on the
+    weight-streaming kernels (K a multiple of 512), the rest on hipBLASLt."""
     import torch
     _say(f"matmul {rows}x{k} . {n}x{k}^T")
     rng = np.random.default_rng(rows + n + k)
@@ -105,6 +105,33 @@ def test_matmul_vs_float64(vo, gpu_backend, rows, n, k):
     acc = _dev(base, torch.float32)
     gpu_backend.matmul(xd, wd, out=acc, accumulate=True)
     assert orc.max_rel_diff(_np(acc), base.astype(np.float64) + want) < 1e-5
+
+
+@pytest.mark.parametrize("rows", [1, 4, 5, 16, 17, 33, 48, 49, 64, 65])
+@pytest.mark.parametrize("n,k", [(16, 512), (4112, 1024), (5136, 1536), (8208, 512), (24592, 512),
+                                 (65552, 512), (512, 4608)])
+def test_streaming_matmul_shapes(vo, gpu_backend, rows, n, k):
+    """Each workgroup shape of the weight-streaming kernel, with output
+    columns that are no whole number of its weight tiles, batches at and past
+    each of its 16-row tiles, one chunk and several; a 512 x 4608 weight goes
+    to the library past 16 rows, and 65 rows do everywhere.  f32 sums of k
+    products in any order: below 1e-5 of the largest output (measured 3e-7)."""
+    import torch
+    _say(f"streaming matmul {rows}x{k} . {n}x{k}^T")
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows + n + k)
+    x = torch.randn((rows, k), generator=gen, device="cuda:0").to(torch.bfloat16)
+    w = (0.02 * torch.randn((n, k), generator=gen, device="cuda:0")).to(torch.bfloat16)
+    want = x.double() @ w.double().T
+    bound = 1e-5 * want.abs().max()
+    got = gpu_backend.matmul(x, w, out_dtype=torch.float32)
+    assert (got - want).abs().max() < bound
+    acc = torch.ones_like(got)
+    gpu_backend.matmul(x, w, out=acc, accumulate=True)
+    assert (acc - 1 - want).abs().max() < bound + 2 ** -22 * (1 + want.abs().max())
+    b16 = gpu_backend.matmul(x, w)
+    if rows <= 16 or (rows <= 64 and k <= 2 * n):  # the same sums, rounded once
+        assert torch.equal(b16, got.to(torch.bfloat16))
 
 
 def test_skinny_matmul_rows_independent_of_batch(vo, gpu_backend):

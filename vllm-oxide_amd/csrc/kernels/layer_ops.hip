@@ -380,20 +380,42 @@ __global__ __launch_bounds__(kThreads) void matmul_generic_kernel(
     }
 }
 
-// Backend::matmul for 1..4 rows (small decode batches): streaming the
-// weight is the whole cost.  A workgroup owns 16 weight rows (outputs) and
-// splits K over its 8 wavefronts; each wavefront runs
-// v_mfma_f32_16x16x32_bf16 with A = 16 weight rows x 32 k (one non-temporal
-// 16-byte load per lane) and B = x^T (the batch rows in columns 0..rows-1;
-// columns past the batch repeat its last row and are not stored, so no lane
-// branches), 8 steps of loads issued before their MFMAs.  The 8 partial
-// tiles are summed through LDS in wavefront order, so an output depends
-// only on its own row of x, whatever the batch size.  Beyond 4 rows the
-// repeated x reads (every workgroup reads all of x) make hipBLASLt faster.
-// MODE 0: bf16 out, 1: f32 out, 2: f32 out += .
+// Four consecutive outputs of one row.  MODE 0: bf16, 1: f32, 2: f32 +=.
+template <int MODE>
+__device__ __forceinline__ void store_out4(void *out, uint64_t o, floatx4 t) {
+    if constexpr (MODE == 0) {
+        u32x2 p;
+        p[0] = static_cast<uint32_t>(f32_to_bf16_bits(t[0])) |
+               (static_cast<uint32_t>(f32_to_bf16_bits(t[1])) << 16);
+        p[1] = static_cast<uint32_t>(f32_to_bf16_bits(t[2])) |
+               (static_cast<uint32_t>(f32_to_bf16_bits(t[3])) << 16);
+        *reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(out) + o) = p;
+    } else {
+        floatx4 *d = reinterpret_cast<floatx4 *>(static_cast<float *>(out) + o);
+        if constexpr (MODE == 2) t += *d;
+        *d = t;
+    }
+}
+
+// Backend::matmul for 1..4 rows and a small weight (up to 2^24 values):
+// streaming the weight is the whole cost.  A workgroup owns 16 weight rows
+// (outputs) and splits K over its 8 wavefronts; each wavefront runs
+// v_mfma_f32_16x16x32_bf16 with A = 16 weight rows x 32 k (one 16-byte load
+// per lane) and B = x^T (the batch rows in columns 0..rows-1; columns past
+// the batch repeat its last row and are not stored, so no lane branches), 8
+// steps of loads issued before their MFMAs.  The 8 partial tiles are summed
+// through LDS in wavefront order, so an output depends only on its own row of
+// x, whatever the batch size.  Ordinary loads: a step reads 64 bytes of each
+// weight row, half a cache line, and the next step the other half;
+// non-temporal loads measured 10-15% slower (the line is fetched twice).
+// Here, in the order of one launch and one round of loads, it beats
+// stream_gemm_kernel below (a weight of 3072 x 2048, 4 rows: 5.1 against
+// 5.8 us; 4096 x 4096: 8.7 against 9.4); on larger weights, or with more
+// rows, every workgroup's reads of x from L2 make it the slower one.
 constexpr int kSkinnyWaves = 8;
 constexpr int kSkinnyU = 8;     // 32-k steps per load batch
 constexpr int kSkinnyRows = 4;  // largest batch the kernel is used for
+constexpr uint64_t kSkinnyWeight = 1ull << 24;  // largest weight
 
 template <int MODE>
 __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(
@@ -414,7 +436,7 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(
         u32x4 a[U], b[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            a[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(wp + kk + 32 * u));
+            a[u] = *reinterpret_cast<const u32x4 *>(wp + kk + 32 * u);
             b[u] = *reinterpret_cast<const u32x4 *>(xp + kk + 32 * u);
         }
 #pragma unroll
@@ -430,19 +452,200 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(
 #pragma unroll
     for (int v = 1; v < kSkinnyWaves; ++v) t += part[v][lane];
     // Lane l holds outputs n0 + 4 (l / 16) + e, e = 0..3, of batch row l % 16.
-    if (!live) return;
-    const uint64_t o = static_cast<uint64_t>(r) * n + n0 + 4 * kg;
-    if constexpr (MODE == 0) {
-        u32x2 p;
-        p[0] = static_cast<uint32_t>(f32_to_bf16_bits(t[0])) |
-               (static_cast<uint32_t>(f32_to_bf16_bits(t[1])) << 16);
-        p[1] = static_cast<uint32_t>(f32_to_bf16_bits(t[2])) |
-               (static_cast<uint32_t>(f32_to_bf16_bits(t[3])) << 16);
-        *reinterpret_cast<u32x2 *>(static_cast<uint16_t *>(out) + o) = p;
+    if (live) store_out4<MODE>(out, static_cast<uint64_t>(r) * n + n0 + 4 * kg, t);
+}
+
+// Backend::matmul for up to 64 rows: HBM, the weight read once.  MT = tiles
+// of 16 batch rows.  A workgroup owns NW tiles of 16 weight rows, one to a
+// wavefront, and splits K over KG groups of NW wavefronts.  A wavefront
+// loads its 16 x KC piece of the weight straight into registers, one chunk
+// ahead of the MFMAs (KC / 32 loads of 16 bytes per lane in flight while it
+// computes), and each group stages the KC columns of x that its wavefronts
+// all need in LDS by LDS DMA, through a ring of three stages, two chunks
+// ahead: read from L2 once per NW weight tiles and not once per tile, since
+// with x loaded by every wavefront the kernel slows in proportion to the
+// batch (a 28672 x 4096 weight: 40 us for 1 row, 63 for 16).  The KG partial
+// tiles of an output are summed through LDS in group order.
+//
+// LDS: row r's 16-byte unit c sits at unit c ^ (r % 16) (mod the row's
+// units), so the 16 lanes that read one unit of 16 rows hit 16 different
+// 4-bank groups; the DMA, whose lanes write in order, applies the same map to
+// its sources.
+//
+// Workgroup b starts its walk over K at chunk b mod (chunks), so that the
+// workgroups do not all read the same lines of x, or the same columns of
+// their weight rows, at once; the order in which an output's products are
+// added depends on the shape and the output's column only.  Weight loads
+// are ordinary ones (see skinny_gemm_kernel).
+//
+// Measured, rows 16 / 40 / 64, against the library product it stands in for:
+// 28672 x 4096: 42.6 / 49.1 / 47.7 us, library 59.6 / 51.1 / 52.2 (5.5 TB/s
+// at 16 rows); 128256 x 2048: 94.8 / 99.9 / 110 us, library 117 / 124 / 130;
+// 6144 x 4096: 13.3 / 16.4 / 18.7 us, library 14.1 / 16.8 / 17.3.
+template <int MODE, int MT, int NW, int KG, int KC>
+__global__ __launch_bounds__(64 * NW * KG) void stream_gemm_kernel(
+    const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, uint32_t rows, uint32_t n,
+    uint32_t k, void *__restrict__ out) {
+    constexpr int W = NW * KG;
+    constexpr int U = KC / 32;              // weight loads per chunk
+    constexpr uint32_t UPR = KC / 8;        // 16-byte units of a staged row
+    constexpr uint32_t SWZ = UPR < 16 ? UPR - 1 : 15;
+    constexpr int XI = 16 * MT * UPR / 64;  // DMA instructions per chunk and group
+    constexpr int ND = XI / NW;
+    constexpr uint32_t XB = 16 * MT * KC * 2;  // bytes of a group's stage
+    static_assert(XI % NW == 0 && ND + U <= 63, "chunk DMA split");
+    static_assert(KG == 1 || W * MT * 64 * 16 <= XB * KG, "the partial tiles fit a stage");
+    __shared__ __align__(1024) uint8_t st0[XB * KG];
+    __shared__ __align__(1024) uint8_t st1[XB * KG];
+    __shared__ __align__(1024) uint8_t st2[XB * KG];
+
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t nw = wave % NW, grp = wave / NW;
+    const uint32_t r = lane & 15, kg = lane >> 4;
+    // A tile past the last one (n is a multiple of 16, not of 16 NW) reads
+    // the last one and stores nothing.
+    const uint32_t n0 = (blockIdx.x * NW + nw) * 16;
+    const uint32_t nr = min(n0, n - 16);
+    const uint32_t kslice = k / KG, k0 = grp * kslice, nch = kslice / KC;
+    const uint32_t rot = blockIdx.x % nch;
+    auto chunk_at = [&](uint32_t c) {  // c < nch
+        c += rot;
+        return c >= nch ? c - nch : c;
+    };
+    const uint16_t *wp = w + static_cast<uint64_t>(nr + r) * k + k0 + 8 * kg;
+    const auto x_rsrc = buffer_rsrc(x, rows * k * 2);
+    uint32_t x_off[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+        const uint32_t u = (i * NW + nw) * 64 + lane;
+        const uint32_t row = u / UPR, c = (u % UPR) ^ (row & SWZ);
+        x_off[i] = (min(row, rows - 1) * k + k0 + 8 * c) * 2;
+    }
+    auto dma = [&](uint8_t *st, uint32_t c) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+            dma16_at(x_rsrc, st + grp * XB + (i * NW + nw) * 1024, x_off[i], chunk_at(c) * (KC * 2));
+    };
+    auto load_w = [&](u32x4 (&a)[U], uint32_t c) __attribute__((always_inline)) {
+        const uint16_t *p = wp + static_cast<uint64_t>(chunk_at(c)) * KC;
+#pragma unroll
+        for (int u = 0; u < U; ++u) a[u] = *reinterpret_cast<const u32x4 *>(p + 32 * u);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    floatx4 acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // Chunk c: issue the weight loads of chunk c + 1, wait for chunk c's
+    // (older, as is this wavefront's share of its x), meet the other
+    // wavefronts, refill the stage they read last with x of chunk c + 2.
+    // Every step issues its loads (past the last chunk the last one's), so
+    // that the wait count stays uniform.
+    auto step = [&](u32x4 (&a)[U], u32x4 (&an)[U], const uint8_t *__restrict__ cur,
+                    uint8_t *__restrict__ nxt, uint32_t c) __attribute__((always_inline)) {
+        load_w(an, min(c + 1, nch - 1));
+        wait_barrier<ND + U>();
+        dma(nxt, min(c + 2, nch - 1));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const uint32_t row = 16 * m + r;
+                const bf16x8 b = *reinterpret_cast<const bf16x8 *>(
+                    cur + grp * XB + (row * UPR + ((4 * u + kg) ^ (row & SWZ))) * 16);
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[u]),
+                                                                 b, acc[m], 0, 0, 0);
+            }
+    };
+    u32x4 a0[U], a1[U];
+    dma(st0, 0);
+    load_w(a0, 0);
+    dma(st1, min(1u, nch - 1));
+    for (uint32_t c = 0;;) {
+        step(a0, a1, st0, st2, c);
+        if (++c >= nch) break;
+        step(a1, a0, st1, st0, c);
+        if (++c >= nch) break;
+        step(a0, a1, st2, st1, c);
+        if (++c >= nch) break;
+        step(a1, a0, st0, st2, c);
+        if (++c >= nch) break;
+        step(a0, a1, st1, st0, c);
+        if (++c >= nch) break;
+        step(a1, a0, st2, st1, c);
+        if (++c >= nch) break;
+    }
+    // The DMA past the last chunk must land before the stages are reused or
+    // the workgroup's LDS is released.
+    __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
+
+    // Lane l holds outputs n0 + 4 (l / 16) + e, e = 0..3, of batch row 16 m +
+    // l % 16.
+    if constexpr (KG == 1) {
+        if (n0 >= n) return;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const uint32_t row = 16 * m + r;
+            if (row < rows)
+                store_out4<MODE>(out, static_cast<uint64_t>(row) * n + n0 + 4 * kg, acc[m]);
+        }
     } else {
-        floatx4 *d = reinterpret_cast<floatx4 *>(static_cast<float *>(out) + o);
-        if constexpr (MODE == 2) t += *d;
-        *d = t;
+        __syncthreads();
+        floatx4 *part = reinterpret_cast<floatx4 *>(st0);  // [W][MT][64]
+#pragma unroll
+        for (int m = 0; m < MT; ++m) part[(wave * MT + m) * 64 + lane] = acc[m];
+        __syncthreads();
+        for (uint32_t t = wave; t < NW * MT; t += W) {
+            const uint32_t tn = t % NW, m = t / NW;
+            floatx4 sum = part[(tn * MT + m) * 64 + lane];
+#pragma unroll
+            for (int g = 1; g < KG; ++g) sum += part[((g * NW + tn) * MT + m) * 64 + lane];
+            const uint32_t row = 16 * m + r, nt = (blockIdx.x * NW + tn) * 16;
+            if (row < rows && nt < n)
+                store_out4<MODE>(out, static_cast<uint64_t>(row) * n + nt + 4 * kg, sum);
+        }
+    }
+}
+
+template <int MT, int NW, int KG, int KC>
+void launch_stream(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n, uint32_t k,
+                   void *out, int mode, hipStream_t stream) {
+    const dim3 grid((n + 16 * NW - 1) / (16 * NW)), block(64 * NW * KG);
+#define VO_STREAM(MODE)                                                                        \
+    hipLaunchKernelGGL((stream_gemm_kernel<MODE, MT, NW, KG, KC>), grid, block, 0, stream, x, \
+                       w, rows, n, k, out)
+    if (mode == 0) VO_STREAM(0);
+    else if (mode == 1) VO_STREAM(1);
+    else VO_STREAM(2);
+#undef VO_STREAM
+}
+
+// The workgroup's shape, by how many 16-row weight tiles there are: enough
+// workgroups for the 256 CUs, then as many tiles to a workgroup as that
+// leaves (each shares x once more).  Measured over 2048 .. 128256 weight rows:
+// 4 tiles with 256-column chunks from 8192 rows on (the narrower splits of K
+// lose 1-5% there, and 8 tiles leave CUs idle below 24576: 20.9 against 15.6
+// us at 16384 x 2048, 40 rows); 8 tiles for a vocabulary's worth of rows and
+// more than one batch tile (99.9 against 114 us at 128256 x 2048, 40 rows)
+// and for 4 batch tiles from 24576 on (47.7 against 55.2 us at 28672 x
+// 4096); 2 tiles and 4 groups from 5120 on (13.3 against 18.3 us at 6144 x
+// 4096, 16 rows); below that 1 tile and 8 groups, with 2 and 4 where the
+// stages of 3 or 4 batch tiles would not fit.
+template <int MT>
+void launch_stream_rows(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
+                        uint32_t k, void *out, int mode, hipStream_t stream) {
+    if (n >= 8192) {
+        if constexpr (MT > 1)
+            if (n >= 65536) return launch_stream<MT, 8, 1, 256>(x, w, rows, n, k, out, mode, stream);
+        if constexpr (MT == 4)
+            if (n >= 24576) return launch_stream<MT, 8, 1, 128>(x, w, rows, n, k, out, mode, stream);
+        return launch_stream<MT, 4, 1, 256>(x, w, rows, n, k, out, mode, stream);
+    }
+    if constexpr (MT <= 2) {
+        if (n >= 5120) return launch_stream<MT, 2, 4, 128>(x, w, rows, n, k, out, mode, stream);
+        return launch_stream<MT, 1, 8, 64>(x, w, rows, n, k, out, mode, stream);
+    } else {
+        return launch_stream<MT, 2, 4, 64>(x, w, rows, n, k, out, mode, stream);
     }
 }
 
@@ -578,9 +781,14 @@ hipError_t launch_matmul_generic(const uint16_t *x, const uint16_t *w, uint32_t 
 namespace vo {
 namespace kernels {
 
+// The weight-streaming kernels take up to 64 rows.  Past 16 rows a weight
+// with more than twice as many columns as rows stays with the library: each
+// workgroup then reads more of x than of the weight (4096 x 14336: 32.5 / 49 us at
+// 32 / 40 rows, library 30.7 / 35.3; at 16 rows 26.5 against 25.9, and the
+// call costs the host 6 us less).
 bool skinny_gemm_supported(uint64_t rows, uint64_t n, uint64_t k) {
-    return rows >= 1 && rows <= kSkinnyRows && n % 16 == 0 &&
-           k % (kSkinnyWaves * 32 * kSkinnyU) == 0 && n / 16 <= 0x7fffffffull;
+    return rows >= 1 && rows <= 64 && n >= 16 && n % 16 == 0 && k >= 512 && k % 512 == 0 &&
+           k <= (1u << 24) && n / 16 <= 0x7fffffffull && (rows <= 16 || k <= 2 * n);
 }
 
 hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
@@ -588,13 +796,24 @@ hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t row
                               hipStream_t stream) {
     if (!skinny_gemm_supported(rows, n, k)) return hipErrorInvalidValue;
     KernelTimer timer("matmul_skinny", stream);
-    const dim3 grid(n / 16), block(64 * kSkinnyWaves);
-    if (!out_f32)
-        hipLaunchKernelGGL((skinny_gemm_kernel<0>), grid, block, 0, stream, x, w, rows, n, k, out);
-    else if (!accumulate)
-        hipLaunchKernelGGL((skinny_gemm_kernel<1>), grid, block, 0, stream, x, w, rows, n, k, out);
-    else
-        hipLaunchKernelGGL((skinny_gemm_kernel<2>), grid, block, 0, stream, x, w, rows, n, k, out);
+    const int mode = !out_f32 ? 0 : (accumulate ? 2 : 1);
+    if (rows <= kSkinnyRows && k % (kSkinnyWaves * 32 * kSkinnyU) == 0 &&
+        static_cast<uint64_t>(n) * k <= kSkinnyWeight) {
+        const dim3 grid(n / 16), block(64 * kSkinnyWaves);
+        if (mode == 0)
+            hipLaunchKernelGGL((skinny_gemm_kernel<0>), grid, block, 0, stream, x, w, rows, n, k, out);
+        else if (mode == 1)
+            hipLaunchKernelGGL((skinny_gemm_kernel<1>), grid, block, 0, stream, x, w, rows, n, k, out);
+        else
+            hipLaunchKernelGGL((skinny_gemm_kernel<2>), grid, block, 0, stream, x, w, rows, n, k, out);
+        return hipGetLastError();
+    }
+    switch ((rows + 15) / 16) {
+        case 1: launch_stream_rows<1>(x, w, rows, n, k, out, mode, stream); break;
+        case 2: launch_stream_rows<2>(x, w, rows, n, k, out, mode, stream); break;
+        case 3: launch_stream_rows<3>(x, w, rows, n, k, out, mode, stream); break;
+        default: launch_stream_rows<4>(x, w, rows, n, k, out, mode, stream); break;
+    }
     return hipGetLastError();
 }
 
