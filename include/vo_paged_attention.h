@@ -329,8 +329,9 @@ int32_t vo_step_meta_unfix_launch(vo_step_meta *meta);
  * reference, whose CPU backend has no launch plan): work items launched per
  * KV head, split-K partials (one per (row, split)), and the row-packing
  * factor P -- with P > 1, full splits of up to P rows that read the same
- * physical blocks (a shared prefix) run as one work item.  VO_ERR_ARGUMENT
- * when the last upload planned no decode rows. */
+ * physical blocks (a shared prefix) run as one work item.  A split that a
+ * small step runs as several workgroups per KV head counts as one item.
+ * VO_ERR_ARGUMENT when the last upload planned no decode rows. */
 int32_t vo_step_meta_decode_plan(const vo_step_meta *meta, uint64_t *work_items,
                                  uint64_t *partials, uint32_t *pack);
 

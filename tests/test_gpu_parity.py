@@ -517,6 +517,46 @@ def test_decode_attention_write_kv_full_size(vo, name):
     _assert_close(got.float().cpu().numpy(), oracle_want, name)
 
 
+@pytest.mark.parametrize("hd,heads,kvh", [(128, 32, 8), (64, 32, 8), (128, 8, 8), (64, 16, 1),
+                                          (128, 64, 8)])
+def test_decode_small_steps_bitwise(vo, monkeypatch, hd, heads, kvh):
+    """A step with few rows splits the rows past 1024 keys over more
+    workgroups (one state of a split each) and merges the partials in the
+    launch.  Rows at the edges of a chunk, a run, a state and a split are, in
+    the mixed step and alone, bitwise what whole splits (VO_DECODE_FINE=0)
+    and the reduce kernel (VO_DECODE_ARRIVE=0) give, on repeated launches too
+    (the arrival counters return to zero), as the one call with write_kv; and
+    within tolerance of the oracle."""
+    _say(f"decode small steps hd={hd} heads={heads} kvh={kvh}")
+    ctx = [1023, 1024, 1055, 2046, 2047, 2048, 2079, 4095, 4196, 16, 5000][: 11 if kvh == 1 else 8]
+    backend = vo.HipBackend(device=0, max_seqs=16, max_rows=W.FILL_ROWS, max_table_entries=8192,
+                            max_query_heads=heads)
+    wl = W.build(vo, backend, kind="decode", heads=heads, kv_heads=kvh, head_dim=hd, block_size=16,
+                 num_blocks=2500, context_lens=ctx, seed=hd + heads)
+    outs = {}
+    for fine in ("0", "160"):
+        for arrive in ("0", "1"):
+            monkeypatch.setenv("VO_DECODE_FINE", fine)
+            monkeypatch.setenv("VO_DECODE_ARRIVE", arrive)
+            outs[fine, arrive] = _bits(_out_replanned(wl, backend))
+            for _ in range(3):
+                assert np.array_equal(_bits(_out(wl, backend)), outs[fine, arrive])
+    monkeypatch.delenv("VO_DECODE_FINE")
+    monkeypatch.delenv("VO_DECODE_ARRIVE")
+    want = outs["0", "0"]
+    for key, got in outs.items():
+        assert np.array_equal(got, want), key
+    backend.step_meta(wl.pool).holds = None
+    fused = backend.decode_attention_write_kv(wl.q, wl.k_new, wl.v_new, wl.pool, 0, wl.meta)
+    assert np.array_equal(_bits(fused), want)
+    for s_ in range(len(ctx)):
+        one = vo.DecodeMeta.new([vo.DecodeSeq(ctx[s_], wl.tables[s_])], 16)
+        alone = backend.decode_attention(wl.q[s_:s_ + 1].contiguous(), wl.pool, 0, one)
+        assert np.array_equal(_bits(alone)[0], want[s_]), ctx[s_]
+    got = backend.decode_attention(wl.q, wl.pool, 0, wl.meta).float().cpu().numpy()
+    _assert_close(got, W.oracle_attention(orc, wl), f"small steps hd={hd} H={heads}")
+
+
 def test_decode_batch_invariance_bitwise(vo, gpu_backend):
     """A row's output is identical alone or in a batch (the reference's
     batch-invariance invariant, CLAUDE.md; model.rs:539-584)."""

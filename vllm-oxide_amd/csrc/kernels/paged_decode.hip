@@ -15,7 +15,10 @@
 // byte is read from HBM once: the algorithmic minimum.  An item is one
 // 16-byte record (row, split, where the split's block ids start, keys), so
 // the workgroup starts its loads after one dependent read.  Its W wavefronts
-// take the split's 32-key chunks round robin; block ids are wave-uniform and
+// take the split's 32-key chunks round robin: chunk c goes to state c % W,
+// wavefront c % W's.  A state folds its chunks kSubChunks at a time: each run
+// of kSubChunks chunks is an online softmax of its own, and the runs are
+// merged in order (fold_state).  Block ids are wave-uniform and
 // come from scalar loads.  Each wavefront issues all 16 loads of its next
 // chunk before it waits for the current one (two register buffers), so two
 // chunks are in flight per wavefront.  The wavefronts merge through LDS at
@@ -24,10 +27,28 @@
 // fp32 partial (m, l, acc[head_dim]) per head, and decode_reduce_kernel
 // merges them:
 //   M = max_i m_i,  out = sum_i 2^(m_i-M) acc_i / sum_i 2^(m_i-M) l_i.
-// (Merging in the last workgroup to finish a row instead needs an
-// agent-scope release/acquire per workgroup; on gfx950 that is an L2
-// writeback and invalidate each time, which measured 5-9x slower than the
-// separate launch.)
+//
+// Few rows.  A step whose splits are fewer than the CUs runs the longer rows
+// one state of a split per workgroup (a "fine" item; W = 4): wavefront s
+// takes run s of the state, so that a wavefront walks at most kSubChunks
+// chunks in a row and four times the workgroups share the reads; the runs
+// are folded through LDS, the partial is the state's, and the merge at the
+// end first merges the four states of a split, then the splits.  Operation for
+// operation that is what a whole item does, so a row gets the same bits
+// either way and batch invariance holds.  Bound: a wavefront's chain of
+// chunks (over 1 us each from HBM) and the number of CUs that read at all.
+// Two rows of 5000-8100 keys of 8 KV heads of 128 dims are 64 whole items: 25.5 us,
+// and 13.8 as 220 fine ones, of a 53 MB read; one row of 8000 keys 27 and
+// 13.8 us a call.
+//
+// The merge.  In a plan without packs the last workgroup of a row (and KV
+// head) to finish merges the row's partials: they are written and read with
+// agent-scope accesses and counted with a relaxed atomic, and no reduce
+// launch follows (3 us of GPU time, and 2.5 us of the host's in a small
+// call: 13.8 -> 11.1 us for one row of 8000 keys of 64 dims).  (A release and an acquire fence
+// per workgroup instead are an L2 writeback and invalidate each time, which
+// measured 5-9x slower than the separate launch.)  Plans with packs and
+// fixed launches keep the reduce kernel.
 // Workgroups are numbered KV head fastest, so the KV heads of one block are
 // read at about the same time.
 //
@@ -81,6 +102,7 @@ namespace {
 
 constexpr int kBS = 16;     // block size of the MFMA path
 constexpr int kChunk = 32;  // keys per wavefront iteration
+constexpr uint32_t kSubChunks = 4;  // chunks of one run of a state (see fold_state)
 
 __device__ __forceinline__ floatx4 mfma16x16x32(bf16x8 a, bf16x8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -101,6 +123,19 @@ __device__ __forceinline__ bf16x8 load_kv(const uint16_t *p) {
         return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load(v));
     else
         return __builtin_bit_cast(bf16x8, *v);
+}
+
+// Max of x over the four lanes l % 16 + 16 g of a column: the row and the
+// half-wave swaps of gfx950 hand each lane the other row's (half's) value in
+// registers.  (__shfl_xor goes through the LDS permute unit and its latency,
+// twice in every chunk's chain.)
+__device__ __forceinline__ float column_max(float x) {
+    const uint32_t w = __float_as_uint(x);
+    const auto r = __builtin_amdgcn_permlane16_swap(w, w, false, false);
+    const float y = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    const uint32_t v = __float_as_uint(y);
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
 }
 
 // One chunk's K and V operands, in registers.
@@ -206,7 +241,7 @@ __device__ __forceinline__ void mask_tail_v(bf16x8 (&va)[HD / 16], int nv) {
         va[dt] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, va[dt]) & mask);
 }
 
-template <int HD>
+template <int HD, bool FIRST = false>
 __device__ __forceinline__ void chunk_update(const floatx4 &s0, const floatx4 &s1,
                                              const bf16x8 (&va)[HD / 16], bool tail, int nv,
                                              float scale_log2, float &m_run, float &l_run,
@@ -215,8 +250,8 @@ __device__ __forceinline__ void chunk_update(const floatx4 &s0, const floatx4 &s
     float sc[8];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        sc[i] = s0[i] * scale_log2;
-        sc[4 + i] = s1[i] * scale_log2;
+        sc[i] = s0[i];
+        sc[4 + i] = s1[i];
     }
     if (tail) {
 #pragma unroll
@@ -225,9 +260,9 @@ __device__ __forceinline__ void chunk_update(const floatx4 &s0, const floatx4 &s
     float mt = sc[0];
 #pragma unroll
     for (int i = 1; i < 8; ++i) mt = fmaxf(mt, sc[i]);
-    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
-    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
-    const float m_new = fmaxf(m_run, mt);  // finite: every chunk has a valid key
+    mt = column_max(mt);
+    // finite: every chunk has a valid key (and the scale is positive)
+    const float m_new = fmaxf(m_run, mt * scale_log2);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     // P goes to the MFMA as two bf16 parts, hi = bf16(p) and lo = bf16(p - hi),
     // so the probabilities keep ~16 significant bits instead of bf16's 8;
@@ -237,7 +272,7 @@ __device__ __forceinline__ void chunk_update(const floatx4 &s0, const floatx4 &s
     bf16x8 pb_hi, pb_lo;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-        const float p = __builtin_amdgcn_exp2f(sc[i] - m_new);
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], scale_log2, -m_new));
         ps += p;
         const __bf16 hi = static_cast<__bf16>(p);
         pb_hi[i] = hi;
@@ -247,8 +282,10 @@ __device__ __forceinline__ void chunk_update(const floatx4 &s0, const floatx4 &s
     m_run = m_new;
 #pragma unroll
     for (int dt = 0; dt < HD / 16; ++dt) {
-        acc[dt] *= alpha;
-        acc[dt] = mfma16x16x32(va[dt], pb_lo, acc[dt]);
+        if constexpr (FIRST)
+            acc[dt] = mfma16x16x32(va[dt], pb_lo, floatx4{0.f, 0.f, 0.f, 0.f});
+        else
+            acc[dt] = mfma16x16x32(va[dt], pb_lo, acc[dt] * alpha);
         acc[dt] = mfma16x16x32(va[dt], pb_hi, acc[dt]);
     }
 }
@@ -263,6 +300,87 @@ __device__ __forceinline__ void compute_chunk(Chunk<HD> &r, const bf16x8 (&qv)[H
     chunk_update<HD>(s0, s1, r.va, tail, nv, scale_log2, m_run, l_run, acc);
 }
 
+// (mf, lf, accf) := (mf, lf, accf) merged with the run (m, l, acc) after it.
+// Every run holds a chunk, so both maxima are finite.
+template <int HD>
+__device__ __forceinline__ void fold_state(float &mf, float &lf, floatx4 (&accf)[HD / 16], float m,
+                                           float l, const floatx4 (&acc)[HD / 16]) {
+#pragma clang fp contract(off)
+    const float mx = fmaxf(mf, m);
+    const float ef = __builtin_amdgcn_exp2f(mf - mx);
+    const float e = __builtin_amdgcn_exp2f(m - mx);
+    lf = lf * ef + l * e;
+    mf = mx;
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) accf[dt][j] = __builtin_fmaf(accf[dt][j], ef, acc[dt][j] * e);
+}
+
+// One state's run in progress (m, l, acc) and the merge of the runs before
+// it.  `flush` ends a run; `finish` leaves the state in (m, l, acc).  With a
+// wavefront's LDS given to flush and finish (room for DT * 64 floatx4), the
+// merged accumulators live there between runs, not in registers: 32
+// registers at head_dim 128, which the two chunks in flight need.
+template <int HD>
+struct RunState {
+    static constexpr int DT = HD / 16;
+    float m, l, mf, lf;
+    floatx4 acc[DT], accf[DT];
+
+    __device__ __forceinline__ void reset_run() {
+        m = -INFINITY;
+        l = 0.0f;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    // In registers; `first`: nothing in accf yet.
+    __device__ __forceinline__ void flush(bool first) {
+        if (first) {
+            mf = m;
+            lf = l;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) accf[dt] = acc[dt];
+        } else {
+            fold_state<HD>(mf, lf, accf, m, l, acc);
+        }
+        reset_run();
+    }
+    __device__ __forceinline__ void finish(bool first) {
+        if (first) return;
+        fold_state<HD>(mf, lf, accf, m, l, acc);
+        m = mf;
+        l = lf;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = accf[dt];
+    }
+    // The same with accf in lds[dt * 64 + lane]; `first`: nothing there yet.
+    __device__ __forceinline__ void flush(floatx4 *lds, int lane, bool first) {
+        merge(lds, lane, first);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) lds[dt * 64 + lane] = acc[dt];
+        mf = m;
+        lf = l;
+        reset_run();
+    }
+    // (m, l, acc) := the runs before it (none if `first`) merged with it.
+    __device__ __forceinline__ void merge(const floatx4 *lds, int lane, bool first) {
+#pragma clang fp contract(off)
+        if (first) return;
+        const float mx = fmaxf(mf, m);
+        const float ef = __builtin_amdgcn_exp2f(mf - mx);
+        const float e = __builtin_amdgcn_exp2f(m - mx);
+        l = lf * ef + l * e;
+        m = mx;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) {
+            const floatx4 f = lds[dt * 64 + lane];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[dt][j] = __builtin_fmaf(f[j], ef, acc[dt][j] * e);
+        }
+    }
+};
+
 // Keeps the scheduler from moving instructions across this point: the next
 // chunk's loads are all issued before the current chunk's first wait.
 __device__ __forceinline__ void issue_fence() { __builtin_amdgcn_sched_barrier(0); }
@@ -276,9 +394,10 @@ __device__ __forceinline__ void issue_fence() { __builtin_amdgcn_sched_barrier(0
 // global address, through a ring of four stages; the workgroup takes one
 // chunk per barrier while the next three load.  The wavefronts then read their operands from LDS at
 // the positions the register path loads from the pool and run its
-// compute_chunk; chunk c updates state c % W, the state the register path's
-// wavefront c % W keeps, and the W states are merged as that path merges its
-// wavefronts, so every column's result is the register path's, bit for bit.
+// compute_chunk.  The chunks of state 0 (c % W == 0) come first, then those
+// of state 1 and so on, each in the register path's runs, and the W states
+// are merged as that path merges its wavefronts, so every column's result is
+// the register path's, bit for bit.
 //
 // LDS bank spread: within a tile, 16-byte unit x sits at unit swz(x).  K
 // unit x = 64 kk + 4 key + j (dims 8 j.. of 32-dim chunk kk): j ^= 2 (key >>
@@ -326,7 +445,7 @@ __device__ __forceinline__ void shared_split(
     constexpr uint32_t KIB_PER_TILE = S::TB / 1024;
 
     const uint32_t row = uniform_u32(rec[0]);
-    const uint32_t split = uniform_u32(rec[1]);
+    const uint32_t split = uniform_u32(rec[1]);  // a pack is never a fine item
     const uint32_t *table = tables + uniform_u32(rec[2]);
     const uint32_t nchunks = split_keys / kChunk;  // a full split
     // The split's block ids (at most kMaxSplitKeys / 16 = 256), 64 per
@@ -420,21 +539,12 @@ __device__ __forceinline__ void shared_split(
     const uint32_t vx = 2 * m + static_cast<uint32_t>(g & 1);
     const uint32_t v_rd = (2 + vb_hi) * S::TB + 16 * S::swz_v(vx);
 
-    // Chunk c goes to state c % W: the (m, l, acc) the register path's
-    // wavefront c % W keeps, in the same order, merged at the end as that
-    // path merges its wavefronts.  So a row's bits do not depend on whether
-    // it was packed.
+    // State w: the (m, l, acc) the register path's wavefront w keeps, in the
+    // same order, merged at the end as that path merges its wavefronts.  So a
+    // row's bits do not depend on whether it was packed.
     float ms[W], ls[W];
     floatx4 as[W][DT];
-#pragma unroll
-    for (int w = 0; w < W; ++w) {
-        ms[w] = -INFINITY;
-        ls[w] = 0.0f;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) as[w][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
 
-    // Chunk c (stage c % 4) updates state c % 4.
     auto read_k = [&](const uint8_t *cur, bf16x8 (&ka)[KK], bf16x8 (&kb)[KK])
         __attribute__((always_inline)) {
 #pragma unroll
@@ -447,38 +557,57 @@ __device__ __forceinline__ void shared_split(
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) va[dt] = *reinterpret_cast<const bf16x8 *>(cur + v_rd + 512 * dt);
     };
-    // One chunk per step: step c waits for chunk c (the DMA of chunks c + 1
-    // and c + 2 may fly on) and for every wavefront to be done with chunk
-    // c - 1, refills that stage with chunk c + 3 and computes chunk c into
-    // state c % 4.  Every step issues its DMA (past the last chunk the block
-    // ids repeat the split's last blocks), so the wait count stays uniform.
-    auto one = [&](auto s_c, uint32_t c) __attribute__((always_inline)) {
-        constexpr int sidx = decltype(s_c)::value;
-        uint8_t *__restrict__ cur = sidx == 0 ? st0 : sidx == 1 ? st1 : sidx == 2 ? st2 : st3;
-        uint8_t *__restrict__ nxt = sidx == 0 ? st3 : sidx == 1 ? st0 : sidx == 2 ? st1 : st2;
-        wait_barrier<2 * NI>();
-        dma_chunk(nxt, min(c + 3, nchunks - 1));
-        if (!wave_live) return;
-        bf16x8 ka[KK], kb[KK], va[DT];
-        floatx4 sa0, sa1;
-        read_k(cur, ka, kb);
-        chunk_qk<HD>(ka, kb, qv, sa0, sa1);
-        read_v(cur, va);
-        chunk_update<HD>(sa0, sa1, va, false, 8, scale_log2, ms[sidx], ls[sidx], as[sidx]);
+    // Step t stages chunk chunk_of(t): `per` steps for each state, padded to
+    // the four stages (steps without a chunk stage the last one and compute
+    // nothing).
+    const uint32_t per = (nchunks + 4 * W - 1) / (4 * W) * 4;
+    auto chunk_of = [&](uint32_t t) { return (t % per) * W + t / per; };
+    auto staged = [&](uint32_t t) { return min(chunk_of(min(t, W * per - 1)), nchunks - 1); };
+    static_assert(W == 4, "four stages");
+    dma_chunk(st0, staged(0));
+    dma_chunk(st1, staged(1));
+    dma_chunk(st2, staged(2));
+    auto state = [&](auto w_c) __attribute__((always_inline)) {
+        constexpr int w = decltype(w_c)::value;
+        RunState<HD> rs;
+        rs.reset_run();
+        // One chunk per step: step t waits for its chunk (the DMA of the next
+        // two may fly on) and for every wavefront to be done with the step
+        // before, refills that stage with the chunk three steps on and
+        // computes.  Every step issues its DMA, so the wait count stays
+        // uniform.
+        auto one = [&](auto s_c, uint32_t k) __attribute__((always_inline)) {
+            constexpr int sidx = decltype(s_c)::value;
+            uint8_t *__restrict__ cur = sidx == 0 ? st0 : sidx == 1 ? st1 : sidx == 2 ? st2 : st3;
+            uint8_t *__restrict__ nxt = sidx == 0 ? st3 : sidx == 1 ? st0 : sidx == 2 ? st1 : st2;
+            wait_barrier<2 * NI>();
+            dma_chunk(nxt, staged(w * per + k + 3));
+            if (!wave_live || k * W + w >= nchunks) return;
+            if (sidx == 0 && k != 0) rs.flush(k == kSubChunks);  // runs of kSubChunks == 4 chunks
+            bf16x8 ka[KK], kb[KK], va[DT];
+            floatx4 sa0, sa1;
+            read_k(cur, ka, kb);
+            chunk_qk<HD>(ka, kb, qv, sa0, sa1);
+            read_v(cur, va);
+            chunk_update<HD>(sa0, sa1, va, false, 8, scale_log2, rs.m, rs.l, rs.acc);
+        };
+        static_assert(kSubChunks == 4, "a run is one turn of the stages");
+        for (uint32_t k = 0; k < per; k += 4) {
+            one(std::integral_constant<int, 0>{}, k);
+            one(std::integral_constant<int, 1>{}, k + 1);
+            one(std::integral_constant<int, 2>{}, k + 2);
+            one(std::integral_constant<int, 3>{}, k + 3);
+        }
+        if (wave_live) rs.finish(nchunks <= W * kSubChunks + w);  // at most one run
+        ms[w] = rs.m;
+        ls[w] = rs.l;
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) as[w][dt] = rs.acc[dt];
     };
-    static_assert(W == 4, "state index = stage index");
-    dma_chunk(st0, 0);
-    dma_chunk(st1, min(1u, nchunks - 1));
-    dma_chunk(st2, min(2u, nchunks - 1));
-    for (uint32_t c = 0; c < nchunks; c += 4) {
-        one(std::integral_constant<int, 0>{}, c);
-        if (c + 1 >= nchunks) break;
-        one(std::integral_constant<int, 1>{}, c + 1);
-        if (c + 2 >= nchunks) break;
-        one(std::integral_constant<int, 2>{}, c + 2);
-        if (c + 3 >= nchunks) break;
-        one(std::integral_constant<int, 3>{}, c + 3);
-    }
+    state(std::integral_constant<int, 0>{});
+    state(std::integral_constant<int, 1>{});
+    state(std::integral_constant<int, 2>{});
+    state(std::integral_constant<int, 3>{});
     // The DMA past the last chunk must land before the workgroup's LDS is
     // released.
     __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
@@ -532,9 +661,10 @@ __device__ __forceinline__ void shared_split(
 // four softmax states as shared_split, but each 16-column tile has two
 // wavefronts: the one of parity 0 keeps states 0 and 2 (chunks 4k and
 // 4k + 2), the one of parity 1 states 1 and 3 (chunks 4k + 1, 4k + 3).  One
-// step stages two chunks (2j in stage 2(j % 2), 2j + 1 in the next) and each
+// step stages two chunks and each
 // wavefront of a pair computes one of them, so a wavefront walks half of the
-// split's chunks.  The workgroup holds W / 2 tiles, so a pack has W / 2 *
+// split's chunks: first the chunks of states 0 and 1 (4k, 4k + 1), then those of states
+// 2 and 3, so that a wavefront has one run in progress.  The workgroup holds W / 2 tiles, so a pack has W / 2 *
 // (16 / G) rows.  Every state still takes its chunks in increasing order,
 // and the four states are merged in the order 0..3 with the register path's
 // arithmetic, so a row's bits are the register path's, as in shared_split.
@@ -568,7 +698,7 @@ __device__ __forceinline__ void shared_split_pairs(
     __builtin_amdgcn_s_setprio(3);
 
     const uint32_t row = uniform_u32(rec[0]);
-    const uint32_t split = uniform_u32(rec[1]);
+    const uint32_t split = uniform_u32(rec[1]);  // a pack is never a fine item
     const uint32_t *table = tables + uniform_u32(rec[2]);
     const uint32_t nchunks = split_keys / kChunk;  // a full split
     constexpr int TV = kMaxSplitKeys / kBS / 64;
@@ -579,15 +709,6 @@ __device__ __forceinline__ void shared_split_pairs(
         const uint32_t i = 64 * k + static_cast<uint32_t>(threadIdx.x & 63);
         tv[k] = i < nblk ? table[i] : 0u;
     }
-    auto block_id = [&](uint32_t i) {  // i < nblk, wave-uniform
-        uint32_t b = __builtin_amdgcn_readlane(tv[0], i & 63);
-#pragma unroll
-        for (int k = 1; k < TV; ++k) {
-            const uint32_t bk = __builtin_amdgcn_readlane(tv[k], i & 63);
-            b = (i >> 6) == static_cast<uint32_t>(k) ? bk : b;
-        }
-        return b;
-    };
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int h = lane & 15;
@@ -631,7 +752,16 @@ __device__ __forceinline__ void shared_split_pairs(
         dma_off[i] = 16 * (t < 2 ? S::swz_k(u, t) : S::swz_v(u));
     }
     const uint64_t block_stride = static_cast<uint64_t>(kv_heads) * kTile;
-    auto dma_chunk = [&](uint8_t *stage, uint32_t c) {
+    auto block_id = [&](uint32_t i) {  // i < nblk, wave-uniform
+        uint32_t b = __builtin_amdgcn_readlane(tv[0], i & 63);
+#pragma unroll
+        for (int k = 1; k < TV; ++k) {
+            const uint32_t bk = __builtin_amdgcn_readlane(tv[k], i & 63);
+            b = (i >> 6) == static_cast<uint32_t>(k) ? bk : b;
+        }
+        return b;
+    };
+    auto dma_chunk = [&](uint8_t *stage, uint32_t c) __attribute__((always_inline)) {
         const uint32_t b0 = block_id(2 * c);
         const uint32_t b1 = block_id(2 * c + 1);
 #pragma unroll
@@ -657,14 +787,9 @@ __device__ __forceinline__ void shared_split_pairs(
     // Local state i is state par + 2 i.
     float ms[2], ls[2];
     floatx4 as[2][DT];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        ms[i] = -INFINITY;
-        ls[i] = 0.0f;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) as[i][dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-    auto compute = [&](const uint8_t *cur, int i) __attribute__((always_inline)) {
+    auto compute = [&](auto first_c, const uint8_t *cur, RunState<HD> &rs)
+        __attribute__((always_inline)) {
+        constexpr bool first = decltype(first_c)::value;  // of a run
         bf16x8 ka[KK], kb[KK], va[DT];
         floatx4 sa0, sa1;
 #pragma unroll
@@ -675,33 +800,65 @@ __device__ __forceinline__ void shared_split_pairs(
         chunk_qk<HD>(ka, kb, qv, sa0, sa1);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) va[dt] = *reinterpret_cast<const bf16x8 *>(cur + v_rd + 512 * dt);
-        chunk_update<HD>(sa0, sa1, va, false, 8, scale_log2, ms[i], ls[i], as[i]);
+        chunk_update<HD, first>(sa0, sa1, va, false, 8, scale_log2, rs.m, rs.l, rs.acc);
     };
-    // Step j: wait for chunks 2j and 2j + 1 (the only DMA in flight), then
-    // for every wavefront to be done with step j - 1's pair, refill that
-    // pair with chunks 2j + 2 and 2j + 3, and compute chunk 2j + par into
-    // local state j % 2 (state (2j + par) % 4).  Each stage is named in its
+    // Step t stages chunks pair_of(t) and the next: `per` steps (whole runs)
+    // for the states 0 and 1, then as many for 2
+    // and 3; a step past a state's last chunk stages the split's last one and
+    // computes nothing.
+    const uint32_t per = (nchunks + 4 * kSubChunks - 1) / (4 * kSubChunks) * kSubChunks;
+    auto pair_of = [&](uint32_t t) { return t < per ? 4 * t : 4 * (t - per) + 2; };
+    // Step t: wait for its two chunks (the only DMA in flight), then
+    // for every wavefront to be done with the step before, refill that
+    // step's stages with the next step's chunks, and compute chunk pair_of(t)
+    // + par.  Each stage is named in its
     // own branch, so that the compiler tells the stage being read from the
-    // ones the DMA fills.  Every step issues its DMA (past the last chunk
-    // the block ids repeat the split's last blocks).
-    auto step = [&](auto s_pair, uint32_t j) __attribute__((always_inline)) {
-        constexpr int sp = decltype(s_pair)::value;
-        wait_barrier<0>();
-        dma_chunk(sp ? st0 : st2, min(2 * j + 2, nchunks - 1));
-        dma_chunk(sp ? st1 : st3, min(2 * j + 3, nchunks - 1));
-        if (!wave_live || 2 * j + par >= nchunks) return;
-        if (par == 0)
-            compute(sp ? st2 : st0, sp);
-        else
-            compute(sp ? st3 : st1, sp);
-    };
-    const uint32_t nsteps = (nchunks + 1) / 2;
+    // ones the DMA fills.  Every step issues its DMA (past the last step
+    // the chunks are the split's last).
+    // The two phases run in a rolled loop, a run to a turn: the code of a
+    // chunk is large, and the instruction cache is shared with the register
+    // path's workgroups.
     dma_chunk(st0, 0);
     dma_chunk(st1, min(1u, nchunks - 1));
-    for (uint32_t j = 0; j < nsteps; j += 2) {
-        step(std::integral_constant<int, 0>{}, j);
-        if (j + 1 >= nsteps) break;
-        step(std::integral_constant<int, 1>{}, j + 1);
+#pragma unroll 1
+    for (uint32_t i = 0; i < 2; ++i) {
+        RunState<HD> rs;
+        rs.reset_run();
+        auto step = [&](auto s_run, uint32_t k) __attribute__((always_inline)) {
+            constexpr int in_run = decltype(s_run)::value;  // k % kSubChunks
+            constexpr int sp = in_run % 2;
+            using First = std::integral_constant<bool, in_run == 0>;
+            const uint32_t nx = pair_of(min(i * per + k + 1, 2 * per - 1));
+            wait_barrier<0>();
+            dma_chunk(sp ? st0 : st2, min(nx, nchunks - 1));
+            dma_chunk(sp ? st1 : st3, min(nx + 1, nchunks - 1));
+            if (!wave_live || 4 * k + 2 * i + par >= nchunks) return;
+            if (in_run == 0 && k != 0) rs.flush(k == kSubChunks);
+            if (par == 0)
+                compute(First{}, sp ? st2 : st0, rs);
+            else
+                compute(First{}, sp ? st3 : st1, rs);
+        };
+        static_assert(kSubChunks == 4, "a run's steps");
+#pragma unroll 1
+        for (uint32_t k = 0; k < per; k += 4) {
+            step(std::integral_constant<int, 0>{}, k);
+            step(std::integral_constant<int, 1>{}, k + 1);
+            step(std::integral_constant<int, 2>{}, k + 2);
+            step(std::integral_constant<int, 3>{}, k + 3);
+        }
+        if (wave_live) rs.finish(nchunks <= 4 * kSubChunks + 2 * i + par);  // at most one run
+        if (i == 0) {
+            ms[0] = rs.m;
+            ls[0] = rs.l;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) as[0][dt] = rs.acc[dt];
+        } else {
+            ms[1] = rs.m;
+            ls[1] = rs.l;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) as[1][dt] = rs.acc[dt];
+        }
     }
     // The DMA past the last chunk must land before the stages are reused.
     __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));
@@ -780,7 +937,167 @@ __device__ __forceinline__ void shared_split_pairs(
     }
 }
 
-template <int HD, int W, bool NT>
+// Split-K partials of a row are merged by the reduce kernel, or by the
+// last workgroup of the row's items to finish (`arrivals`; see decode_splitk_kernel).
+// In the second form they cross workgroups inside a launch, so they are
+// written and read with agent-scope (device-coherent) accesses.
+__device__ __forceinline__ void put_f32(float *p, float v, bool agent) {
+    if (agent)
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        *p = v;
+}
+
+__device__ __forceinline__ void put_f32x4(float *p, floatx4 v, bool agent) {
+    if (agent) {
+        typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+        const u64x2 w = __builtin_bit_cast(u64x2, v);
+        uint64_t *d = reinterpret_cast<uint64_t *>(p);
+        __hip_atomic_store(d, static_cast<uint64_t>(w[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(d + 1, static_cast<uint64_t>(w[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+        *reinterpret_cast<floatx4 *>(p) = v;
+    }
+}
+
+template <bool AGENT>
+__device__ __forceinline__ float get_f32(const float *p) {
+    if constexpr (AGENT)
+        return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        return *p;
+}
+
+template <bool AGENT>
+__device__ __forceinline__ floatx4 get_f32x4(const float *p) {
+    if constexpr (AGENT) {
+        typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+        const uint64_t *d = reinterpret_cast<const uint64_t *>(p);
+        u64x2 w;
+        w[0] = __hip_atomic_load(d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        w[1] = __hip_atomic_load(d + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return __builtin_bit_cast(floatx4, w);
+    } else {
+        return *reinterpret_cast<const floatx4 *>(p);
+    }
+}
+
+// States of a split of `keys` keys that hold keys: the fine items it has.
+__device__ __forceinline__ uint32_t split_states(uint32_t keys) {
+    return min((keys + kChunk - 1) / kChunk, static_cast<uint32_t>(kSharedWaves));
+}
+
+// Merges one row's partials for dims d .. d + 3 of query head qh and writes
+// them.  The splits are folded in order with a running max; a fine row's
+// split is first the merge of its states, as the split kernel merges its
+// wavefronts, so the result depends on the row's keys only.  Four partials
+// of a row of up to four splits, and eight of another or of a fine row, are
+// loaded before the first is used.
+template <int HD, bool AGENT>
+__device__ __forceinline__ void merge_row(const float *part_acc, const float *part_ml,
+                                          uint32_t first, uint32_t nsplit, bool fine, uint32_t nk,
+                                          uint32_t split_keys, uint32_t num_heads, uint32_t qh,
+                                          uint32_t d, uint16_t *out) {
+#pragma clang fp contract(off)
+    constexpr int W = kSharedWaves;
+    constexpr int U = 8;
+    float mx = -INFINITY, den = 0.0f;
+    floatx4 num = {0.f, 0.f, 0.f, 0.f};
+    float m[U], l[U];
+    floatx4 a[U];
+    auto load = [&](int u, uint32_t slot) {
+        const uint64_t part = static_cast<uint64_t>(slot) * num_heads + qh;
+        m[u] = get_f32<AGENT>(part_ml + 2 * part);
+        l[u] = get_f32<AGENT>(part_ml + 2 * part + 1);
+        a[u] = get_f32x4<AGENT>(part_acc + part * HD + d);
+    };
+    auto fold = [&](float mi, float li, const floatx4 &ai) {
+        const float m_new = fmaxf(mx, mi);
+        const float scale_old = __builtin_amdgcn_exp2f(mx - m_new);
+        const float e = __builtin_amdgcn_exp2f(mi - m_new);
+        den = den * scale_old + e * li;
+        num = num * scale_old + ai * e;
+        mx = m_new;
+    };
+    if (!fine) {
+        auto rounds = [&](auto r_c) __attribute__((always_inline)) {
+            constexpr uint32_t R = decltype(r_c)::value;  // splits per round
+            for (uint32_t i = 0; i < nsplit; i += R) {
+#pragma unroll
+                for (uint32_t u = 0; u < R; ++u) load(u, first + min(i + u, nsplit - 1));
+#pragma unroll
+                for (uint32_t u = 0; u < R; ++u)
+                    if (i + u < nsplit) fold(m[u], l[u], a[u]);
+            }
+        };
+        if (nsplit <= 4)
+            rounds(std::integral_constant<uint32_t, 4>{});
+        else
+            rounds(std::integral_constant<uint32_t, U>{});
+    } else {
+        constexpr int S = U / W;  // splits per round
+        for (uint32_t i = 0; i < nsplit; i += S) {
+            uint32_t states[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const uint32_t sp = min(i + s, nsplit - 1);
+                states[s] = split_states(min(nk - sp * split_keys, split_keys));
+                // Past the split's states: its first one, not used.
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    load(s * W + w, first + W * sp + (static_cast<uint32_t>(w) < states[s] ? w : 0));
+            }
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                if (i + s >= nsplit) break;
+                float ms = -INFINITY;
+#pragma unroll
+                for (int w = 0; w < W; ++w)
+                    if (static_cast<uint32_t>(w) < states[s]) ms = fmaxf(ms, m[s * W + w]);
+                float ds = 0.0f;
+                floatx4 ns = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    if (static_cast<uint32_t>(w) < states[s]) {
+                        const float e = __builtin_amdgcn_exp2f(m[s * W + w] - ms);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) ns[j] += e * a[s * W + w][j];
+                        ds += e * l[s * W + w];
+                    }
+                }
+                if (nsplit == 1) {  // as the split kernel's own output
+                    num = ns;
+                    den = ds;
+                } else {
+                    fold(ms, ds, ns);
+                }
+            }
+        }
+    }
+    u32x2 packed;
+    if (fine && nsplit == 1) {
+        packed[0] = f32_to_bf16_bits(num[0] / den) |
+                    (static_cast<uint32_t>(f32_to_bf16_bits(num[1] / den)) << 16);
+        packed[1] = f32_to_bf16_bits(num[2] / den) |
+                    (static_cast<uint32_t>(f32_to_bf16_bits(num[3] / den)) << 16);
+    } else {
+        const float inv = 1.0f / den;
+        packed[0] = f32_to_bf16_bits(num[0] * inv) |
+                    (static_cast<uint32_t>(f32_to_bf16_bits(num[1] * inv)) << 16);
+        packed[1] = f32_to_bf16_bits(num[2] * inv) |
+                    (static_cast<uint32_t>(f32_to_bf16_bits(num[3] * inv)) << 16);
+    }
+    *reinterpret_cast<u32x2 *>(out + d) = packed;
+}
+
+// The kernels of a launch: one without packs (single rows, fine items, the
+// in-launch merge) and one for each form of shared packs beside single rows,
+// so that neither carries the other's code, which would not fit half the
+// instruction cache (22 and 33 KB at head_dim 128; all in one 50 KB, and the
+// 64-row decode step 0.9% longer).
+enum PackKind : int { kNoPacks = 0, kPairPacks = 1, kSinglePacks = 2 };
+
+template <int HD, int W, bool NT, int PACKS>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(2))) void
 decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__restrict__ v_pool,
                      uint32_t kv_heads, const uint32_t *__restrict__ tables,
@@ -792,7 +1109,7 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
                      const uint32_t *__restrict__ mates, uint32_t pack, uint16_t *__restrict__ k_w,
                      uint16_t *__restrict__ v_w, const uint16_t *__restrict__ new_k,
                      const uint16_t *__restrict__ new_v, const uint32_t *__restrict__ new_slots,
-                     uint32_t num_shared, uint32_t shared_pairs) {
+                     uint32_t num_shared, uint32_t *__restrict__ arrivals) {
 #pragma clang fp contract(off)  // the wavefronts' merge rounds as a shared pack's does
     constexpr int KK = HD / 32;
     constexpr int DT = HD / 16;
@@ -810,6 +1127,7 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     __shared__ __align__(1024) uint8_t sh2[kStageBytes];
     __shared__ __align__(1024) uint8_t sh3[kStageBytes];
     __shared__ float s_ml[kStages ? 2 * W * 16 : 1];
+    __shared__ uint32_t s_last;
     static_assert(!kStages || 16 * kAccStride<HD> * 4 <= kStageBytes, "merge fits a stage");
 
     const uint32_t item = blockIdx.x / kv_heads;
@@ -820,7 +1138,7 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     const u32x4 rec = *reinterpret_cast<const u32x4 *>(work + 4 * static_cast<uint64_t>(item));
     if (item >= counts[0]) return;
     const uint32_t row = rec[0];
-    const uint32_t split = rec[1];
+    const uint32_t split = rec[1] & kSplitMask;
     const uint32_t *table = tables + rec[2];  // this split's block ids
     const uint32_t nk = rec[3];
     const uint64_t out_base = static_cast<uint64_t>(row) * num_heads * HD;
@@ -832,9 +1150,9 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
             out[out_base + static_cast<uint64_t>(kvh) * group * HD + idx] = 0;
         return;
     }
-    if constexpr (kStages) {
+    if constexpr (kStages && PACKS != kNoPacks) {
         if (item < num_shared) {
-            if (shared_pairs)
+            if constexpr (PACKS == kPairPacks)
                 shared_split_pairs<HD, W>(k_pool, v_pool, kv_heads, kvh, item, rec, tables,
                                           row_info, split_keys, q, out, part_acc, part_ml,
                                           num_heads, group, scale_log2, mates, pack, sh0, sh1,
@@ -847,7 +1165,7 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
         }
     }
     // In a plan with shared packs every item with mates is one of them.
-    if (num_shared != 0) pack = 1;
+    if constexpr (PACKS != kNoPacks) pack = 1;
 
     const uint32_t k_begin = split * split_keys;
     const uint32_t k_end = min(nk, k_begin + split_keys);
@@ -855,7 +1173,11 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     const uint32_t nchunks = (k_end - k_begin + kChunk - 1) / kChunk;
     // With new keys given, the item holding the row's last key caches it
     // and takes it from new_k / new_v (see NewKeys).
-    const bool take_new = new_k != nullptr && k_end == nk;
+    // A fine item holds the chunks c % W == part of its split only.
+    constexpr bool kFine = kStages && PACKS == kNoPacks;
+    const bool fine = kFine && (rec[1] & ~kSplitMask) != 0;
+    const uint32_t part = fine ? (rec[1] >> kPartShift) - 1 : 0u;
+    const bool take_new = new_k != nullptr && k_end == nk && (!fine || (nchunks - 1) % W == part);
     const uint16_t *nk_row = take_new ? new_k + (static_cast<uint64_t>(row) * kv_heads + kvh) * HD : nullptr;
     const uint16_t *nv_row = take_new ? new_v + (static_cast<uint64_t>(row) * kv_heads + kvh) * HD : nullptr;
 
@@ -904,6 +1226,36 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     u32x2 cinfo = {0u, 0u};
     if (head_ok) cinfo = *reinterpret_cast<const u32x2 *>(row_info + 2 * static_cast<uint64_t>(crow));
 
+    // The end of an item with a partial, when the row's last workgroup merges
+    // (a plan without packs: every column is this row's).  Each partial was
+    // written with agent-scope stores; once this wavefront's are done and the
+    // workgroup has met, one lane counts the item, and the workgroup that
+    // counts the row's last one for this KV head reads the partials back with
+    // agent-scope loads and leaves the counter at zero for the next launch.
+    // (No release or acquire fence: see the top of this file.)
+    auto arrive = [&](uint32_t first, uint32_t nsplit, bool fine_row) {
+        __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): the stores are done
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const uint32_t expected = fine_row ? W * (nk / split_keys) + split_states(nk % split_keys)
+                                               : nsplit;
+            uint32_t *const count = arrivals + static_cast<uint64_t>(row) * kv_heads + kvh;
+            const uint32_t before =
+                __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const bool last = before + 1 == expected;
+            if (last) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_last = last ? 1u : 0u;
+        }
+        __syncthreads();
+        if (s_last == 0) return;
+        constexpr uint32_t NQ = HD / 4;
+        for (uint32_t i = threadIdx.x; i < group * NQ; i += 64 * W) {
+            const uint32_t qh = kvh * group + i / NQ;
+            merge_row<HD, true>(part_acc, part_ml, first, nsplit, fine_row, nk, split_keys, num_heads,
+                                qh, 4 * (i % NQ), out + out_base + static_cast<uint64_t>(qh) * HD);
+        }
+    };
+
     // Block ids of chunk cc: wave-uniform, so scalar loads from the table
     // (no LDS copy, no VGPR).  Load order: mates, Q and column info, first
     // chunk, so that each wait for a value (vmcnt counts in issue order)
@@ -918,16 +1270,22 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
         issue_fence();
     };
     Chunk<HD> bufA, bufB;
-    // This wavefront's chunks: wave + k W for k < mine.
-    const uint32_t mine = nchunks > static_cast<uint32_t>(wave) ? (nchunks - wave + W - 1) / W : 0;
-    auto chunk = [&](uint32_t k) { return static_cast<uint32_t>(wave) + k * W; };
+    // This wavefront's chunks: state + (k0 + k) W for k < mine, where a fine
+    // item's wavefront has run `wave` of the item's state, and another
+    // item's has the whole state `wave`.
+    const uint32_t state = fine ? part : static_cast<uint32_t>(wave);
+    const uint32_t k0 = fine ? kSubChunks * static_cast<uint32_t>(wave) : 0u;
+    const uint32_t of_state = nchunks > state ? (nchunks - state + W - 1) / W : 0;
+    uint32_t mine = of_state > k0 ? of_state - k0 : 0u;
+    if (fine) mine = min(mine, kSubChunks);
+    auto chunk = [&](uint32_t k) { return state + (k0 + k) * W; };
     load(bufA, chunk(0));
 
-    float m_run = -INFINITY;
-    float l_run = 0.0f;
-    floatx4 acc[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) acc[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // Between runs the merged accumulators wait in the wavefront's stage.
+    floatx4 *const run_lds = kStages ? reinterpret_cast<floatx4 *>(
+        wave == 0 ? sh0 : (wave == 1 ? sh1 : (wave == 2 ? sh2 : sh3))) : nullptr;
+    RunState<HD> rs;
+    rs.reset_run();
 
     // A chunk computed inside the loop has a successor, so it is full: only
     // the chunks computed at the loop's exits can be the split's tail, and
@@ -938,8 +1296,16 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
             take_new_key<HD>(r, nk - 1 - j0, nk_row, nv_row, lane);
         const bool tail = may_tail && j0 + kChunk > k_end;
         const int nv = max(0, min(8, static_cast<int>(k_end) - static_cast<int>(j0 + 8 * g)));
-        compute_chunk<HD>(r, qv, tail, nv, scale_log2, m_run, l_run, acc);
+        compute_chunk<HD>(r, qv, tail, nv, scale_log2, rs.m, rs.l, rs.acc);
     };
+    // Before chunk k (even): the runs end every kSubChunks chunks.  (With
+    // another number of wavefronts than a pack's or a fine item's, a tuning
+    // setting, a state is one run.)
+    auto new_run = [&](uint32_t k) {
+        if constexpr (kStages)
+            if (k != 0 && k % kSubChunks == 0) rs.flush(run_lds, lane, k == kSubChunks);
+    };
+    static_assert(kSubChunks % 2 == 0, "runs start at the first register buffer");
 
     // Two register buffers: the loads of chunk k + 1 are all issued (the
     // fence in `load`) before the first wait for chunk k, so each wavefront
@@ -950,17 +1316,24 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     uint32_t k = 0;
     for (; k + 2 < mine; k += 2) {
         load(bufB, chunk(k + 1));
+        new_run(k);
         run(bufA, chunk(k), false);
         load(bufA, chunk(k + 2));
         run(bufB, chunk(k + 1), false);
     }
     if (k + 1 < mine) {
         load(bufB, chunk(k + 1));
+        new_run(k);
         run(bufA, chunk(k), false);
         run(bufB, chunk(k + 1), true);
     } else if (k < mine) {
+        new_run(k);
         run(bufA, chunk(k), true);
     }
+    if constexpr (kStages) rs.merge(run_lds, lane, mine <= kSubChunks);
+    float m_run = rs.m;
+    float l_run = rs.l;
+    floatx4 (&acc)[DT] = rs.acc;
 
     // Cache the new key (nothing in this launch reads its slot from the pool).
     if (take_new) {
@@ -973,6 +1346,59 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
                 *reinterpret_cast<const u32x4 *>(nk_row + d);
         }
         for (uint32_t d = threadIdx.x; d < HD; d += 64 * W) v_w[tile + d * kBS + t] = nv_row[d];
+    }
+
+    if constexpr (kFine) {
+        if (fine) {
+            // Fold the state's runs, in order, through the stages: wavefront
+            // w's run sits in stage w ([DT][64] floatx4, then m and l per
+            // lane), and wavefront w folds DT / W of the DT accumulators.
+            uint8_t *const mine_st = wave == 0 ? sh0 : (wave == 1 ? sh1 : (wave == 2 ? sh2 : sh3));
+            constexpr uint32_t ML = DT * 64 * 16;
+            static_assert(ML + 2 * 64 * 4 <= kStageBytes && DT % W == 0, "a run fits a stage");
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+                reinterpret_cast<floatx4 *>(mine_st)[dt * 64 + lane] = acc[dt];
+            reinterpret_cast<float *>(mine_st + ML)[lane] = m_run;
+            reinterpret_cast<float *>(mine_st + ML)[64 + lane] = l_run;
+            __syncthreads();
+            const uint32_t runs = (of_state + kSubChunks - 1) / kSubChunks;  // 1 .. W
+            constexpr int DW = DT / W;
+            const floatx4 *a0 = reinterpret_cast<const floatx4 *>(sh0) + (wave * DW) * 64 + lane;
+            float mf = reinterpret_cast<const float *>(sh0 + ML)[lane];
+            float lf = reinterpret_cast<const float *>(sh0 + ML)[64 + lane];
+            floatx4 af[DW];
+#pragma unroll
+            for (int i = 0; i < DW; ++i) af[i] = a0[i * 64];
+#pragma unroll
+            for (int w = 1; w < W; ++w) {
+                if (static_cast<uint32_t>(w) < runs) {
+                    const uint8_t *st = w == 1 ? sh1 : (w == 2 ? sh2 : sh3);
+                    floatx4 aw[DW];
+#pragma unroll
+                    for (int i = 0; i < DW; ++i)
+                        aw[i] = reinterpret_cast<const floatx4 *>(st)[(wave * DW + i) * 64 + lane];
+                    fold_state<16 * DW>(mf, lf, af, reinterpret_cast<const float *>(st + ML)[lane],
+                                        reinterpret_cast<const float *>(st + ML)[64 + lane], aw);
+                }
+            }
+            lf += __shfl_xor(lf, 16, 64);
+            lf += __shfl_xor(lf, 32, 64);
+            // The partial of state `part`: slot first + W split + part.
+            if (head_ok) {
+                const uint64_t slot = static_cast<uint64_t>(cinfo[0]) + static_cast<uint64_t>(W) * split + part;
+                const uint64_t at = slot * num_heads + qhead;
+                float *ap = part_acc + at * HD + 16 * DW * wave + 4 * g;
+#pragma unroll
+                for (int i = 0; i < DW; ++i) put_f32x4(ap + 16 * i, af[i], arrivals != nullptr);
+                if (wave == 0 && g == 0) {
+                    put_f32(part_ml + 2 * at, mf, arrivals != nullptr);
+                    put_f32(part_ml + 2 * at + 1, lf, arrivals != nullptr);
+                }
+            }
+            if (arrivals) arrive(uniform_u32(cinfo[0]), uniform_u32(cinfo[1]) & ~kFineRow, true);
+            return;
+        }
     }
 
     // The running sums are per lane group; the max is already per head.
@@ -1060,89 +1486,45 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
                     f32_to_bf16_bits(num / den);
             } else {
                 const uint64_t part = static_cast<uint64_t>(s_col[1][col] + split) * num_heads + qh;
-                part_acc[part * HD + d] = num;
+                put_f32(part_acc + part * HD + d, num, kFine && arrivals != nullptr);
                 if (d == 0) {
-                    part_ml[2 * part] = mx;
-                    part_ml[2 * part + 1] = den;
+                    put_f32(part_ml + 2 * part, mx, kFine && arrivals != nullptr);
+                    put_f32(part_ml + 2 * part + 1, den, kFine && arrivals != nullptr);
                 }
             }
         }
+        if constexpr (kFine)
+            if (arrivals && s_col[2][0] > 1) arrive(s_col[1][0], s_col[2][0], false);
     }
 }
 
-// Merge the split-K partials of one (row, query head) for the rows listed in
-// reduce_rows (those with more than one split; rows with one split were
-// written by the split kernel).  The 256 threads are HD/4 dim quads x P
-// split lanes: lane p folds splits p, p + P, ... with a running max (its
-// loads are independent of each other), and the P lane results are merged
-// through LDS in lane order.  The merge order depends only on the row's
-// number of splits, so the result is the same in any batch.  With P lanes a
-// 64-split row costs 8 dependent load rounds instead of 64.
+// Merges the split-K partials of the rows listed in reduce_rows (those with
+// more than one split, and those of fine items; rows with one whole split
+// were written by the split kernel), where the row's last workgroup does not:
+// plans with packs and fixed launches.  A wavefront is a workgroup and takes
+// 64 / (HD / 4) query heads of one row, a thread four dims (with four such to
+// a workgroup 65 rows of 64 heads took 5.8 us instead of 5.5).
 template <int HD>
-__global__ __launch_bounds__(256) void decode_reduce_kernel(
-    const uint32_t *__restrict__ row_info, const uint32_t *__restrict__ reduce_rows,
-    const float *__restrict__ part_acc, const float *__restrict__ part_ml,
-    uint16_t *__restrict__ out, uint32_t num_heads, const uint32_t *__restrict__ counts) {
-    constexpr int NQ = HD / 4;     // dim quads of one head
-    constexpr int P = 256 / NQ;    // split lanes
-    __shared__ float s_m[P][NQ];
-    __shared__ float s_l[P][NQ];
-    __shared__ floatx4 s_acc[P][NQ];
-
-    if (blockIdx.x / num_heads >= counts[1]) return;  // past this step's rows (fixed launch)
-    const uint32_t row = reduce_rows[blockIdx.x / num_heads];
-    const uint32_t qh = blockIdx.x % num_heads;
-    const uint32_t first = row_info[2 * row];
-    const uint32_t nsplit = row_info[2 * row + 1];
-    const uint32_t dq = threadIdx.x % NQ;
-    const uint32_t p = threadIdx.x / NQ;
-    const uint32_t d = 4 * dq;
-
-    float mx = -INFINITY, den = 0.0f;
-    floatx4 num = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-    for (uint32_t i = p; i < nsplit; i += P) {
-        const uint64_t part = static_cast<uint64_t>(first + i) * num_heads + qh;
-        const float m = part_ml[2 * part];  // finite: a split holds >= 1 key
-        const float l = part_ml[2 * part + 1];
-        const floatx4 a = *reinterpret_cast<const floatx4 *>(part_acc + part * HD + d);
-        const float m_new = fmaxf(mx, m);
-        const float scale_old = __builtin_amdgcn_exp2f(mx - m_new);
-        const float e = __builtin_amdgcn_exp2f(m - m_new);
-        den = den * scale_old + e * l;
-        num = num * scale_old + a * e;
-        mx = m_new;
-    }
-    s_m[p][dq] = mx;
-    s_l[p][dq] = den;
-    s_acc[p][dq] = num;
-    __syncthreads();
-    if (p != 0) return;
-    float M = s_m[0][dq];
-#pragma unroll
-    for (int j = 1; j < P; ++j) M = fmaxf(M, s_m[j][dq]);
-    float L = 0.0f;
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < P; ++j) {
-        const float mj = s_m[j][dq];
-        if (mj == -INFINITY) continue;  // lane j had no split
-        const float e = __builtin_amdgcn_exp2f(mj - M);
-        L += e * s_l[j][dq];
-        acc += s_acc[j][dq] * e;
-    }
-    const float inv = 1.0f / L;
-    u32x2 packed;
-    packed[0] = f32_to_bf16_bits(acc[0] * inv) |
-                (static_cast<uint32_t>(f32_to_bf16_bits(acc[1] * inv)) << 16);
-    packed[1] = f32_to_bf16_bits(acc[2] * inv) |
-                (static_cast<uint32_t>(f32_to_bf16_bits(acc[3] * inv)) << 16);
-    const uint64_t out_off = (static_cast<uint64_t>(row) * num_heads + qh) * HD + d;
-    *reinterpret_cast<u32x2 *>(out + out_off) = packed;
+__global__ __launch_bounds__(64) void decode_reduce_kernel(
+    const uint32_t *__restrict__ reduce_rows, const float *__restrict__ part_acc,
+    const float *__restrict__ part_ml, uint16_t *__restrict__ out, uint32_t num_heads,
+    const uint32_t *__restrict__ counts, uint32_t split_keys) {
+    constexpr uint32_t NQ = HD / 4;    // dim quads of one head
+    constexpr uint32_t HPW = 64 / NQ;  // heads per workgroup
+    const uint32_t groups = (num_heads + HPW - 1) / HPW;
+    // The row's whole record in one load (every launched row has a readable
+    // one), beside the step's count.
+    const u32x4 rec = *reinterpret_cast<const u32x4 *>(reduce_rows + 4 * static_cast<uint64_t>(blockIdx.x / groups));
+    if (blockIdx.x / groups >= counts[1]) return;  // past this step's rows (fixed launch)
+    const uint32_t qh = (blockIdx.x % groups) * HPW + threadIdx.x / NQ;
+    if (qh >= num_heads) return;
+    merge_row<HD, false>(part_acc, part_ml, rec[1], rec[2] & ~kFineRow, (rec[2] & kFineRow) != 0,
+                         rec[3], split_keys, num_heads, qh, 4 * (threadIdx.x % NQ),
+                         out + (static_cast<uint64_t>(rec[0]) * num_heads + qh) * HD);
 }
 
-template <int HD, int W, bool NT>
-hipError_t launch_split(const PoolLayer &pool, const MetaView &meta, const DecodePlan &plan,
+template <int HD, int W, bool NT, int PACKS>
+hipError_t launch_split_kind(const PoolLayer &pool, const MetaView &meta, const DecodePlan &plan,
                         const uint16_t *q, uint16_t *out, uint32_t num_heads, float scale_log2,
                         hipStream_t stream, const NewKeys *nkeys) {
     const uint32_t group = num_heads / pool.kv_heads;
@@ -1156,6 +1538,8 @@ hipError_t launch_split(const PoolLayer &pool, const MetaView &meta, const Decod
                         pack > shared_tiles * (16 / group) || plan.split_keys % kChunk != 0))
         return hipErrorInvalidValue;
     const uint32_t item_pack = shared ? 1u : pack;
+    static_assert(PACKS == kNoPacks || W == kSharedWaves, "packs need the stages");
+    if (plan.arrivals && (pack != 1 || W != kSharedWaves)) return hipErrorInvalidValue;
     if (item_pack * group > 16 || (pack > 1 && plan.mates == nullptr)) return hipErrorInvalidValue;
     // With 4 wavefronts (not streaming) the merge lives in the shared-pack
     // stages (at most 16 columns of HD floats per wavefront, 8 KiB at
@@ -1167,14 +1551,30 @@ hipError_t launch_split(const PoolLayer &pool, const MetaView &meta, const Decod
     const uint64_t grid = static_cast<uint64_t>(plan.launch_work) * pool.kv_heads;
     if (grid > 0x7fffffffull) return hipErrorInvalidValue;
     KernelTimer timer("decode_splitk", stream);
-    hipLaunchKernelGGL((decode_splitk_kernel<HD, W, NT>), dim3(static_cast<uint32_t>(grid)),
+    hipLaunchKernelGGL((decode_splitk_kernel<HD, W, NT, PACKS>), dim3(static_cast<uint32_t>(grid)),
                        dim3(64 * W), smem, stream, pool.k, pool.v, pool.kv_heads, meta.tables,
                        plan.work, plan.row_info,
                        plan.split_keys, q, out, plan.part_acc, plan.part_ml, num_heads, group,
                        scale_log2, plan.counts, plan.mates, pack, pool.k, pool.v,
                        nkeys ? nkeys->k : nullptr, nkeys ? nkeys->v : nullptr,
-                       nkeys ? nkeys->slots : nullptr, shared, plan.shared_pairs ? 1u : 0u);
+                       nkeys ? nkeys->slots : nullptr, shared, plan.arrivals);
     return hipGetLastError();
+}
+
+template <int HD, int W, bool NT>
+hipError_t launch_split(const PoolLayer &pool, const MetaView &meta, const DecodePlan &plan,
+                        const uint16_t *q, uint16_t *out, uint32_t num_heads, float scale_log2,
+                        hipStream_t stream, const NewKeys *nkeys) {
+    if constexpr (W == kSharedWaves) {
+        if (plan.num_shared != 0 && plan.shared_pairs)
+            return launch_split_kind<HD, W, NT, kPairPacks>(pool, meta, plan, q, out, num_heads,
+                                                            scale_log2, stream, nkeys);
+        if (plan.num_shared != 0)
+            return launch_split_kind<HD, W, NT, kSinglePacks>(pool, meta, plan, q, out, num_heads,
+                                                              scale_log2, stream, nkeys);
+    }
+    return launch_split_kind<HD, W, NT, kNoPacks>(pool, meta, plan, q, out, num_heads, scale_log2,
+                                                  stream, nkeys);
 }
 
 template <int HD>
@@ -1195,13 +1595,15 @@ hipError_t launch_hd(const PoolLayer &pool, const MetaView &meta, const DecodePl
         default: err = VO_SPLIT(4); break;
     }
 #undef VO_SPLIT
-    if (err != hipSuccess || plan.launch_reduce == 0) return err;
-    const uint64_t grid = static_cast<uint64_t>(plan.launch_reduce) * num_heads;
+    if (err != hipSuccess || plan.launch_reduce == 0 || plan.arrivals) return err;
+    constexpr uint32_t kHeadsPerGroup = 64 / (HD / 4);
+    const uint64_t grid = static_cast<uint64_t>(plan.launch_reduce) *
+                          ((num_heads + kHeadsPerGroup - 1) / kHeadsPerGroup);
     if (grid > 0x7fffffffull) return hipErrorInvalidValue;
     KernelTimer timer("decode_reduce", stream);
-    hipLaunchKernelGGL((decode_reduce_kernel<HD>), dim3(static_cast<uint32_t>(grid)), dim3(256),
-                       0, stream, plan.row_info, plan.reduce_rows, plan.part_acc, plan.part_ml,
-                       out, num_heads, plan.counts);
+    hipLaunchKernelGGL((decode_reduce_kernel<HD>), dim3(static_cast<uint32_t>(grid)), dim3(64),
+                       0, stream, plan.reduce_rows, plan.part_acc, plan.part_ml, out, num_heads,
+                       plan.counts, plan.split_keys);
     return hipGetLastError();
 }
 

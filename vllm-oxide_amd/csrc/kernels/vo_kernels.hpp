@@ -151,14 +151,27 @@ hipError_t launch_matmul_generic(const uint16_t *x, const uint16_t *w, uint32_t 
 // Largest split the decode kernel takes (its block-table slice lives in LDS).
 constexpr uint32_t kMaxSplitKeys = 4096;
 
+// A work record's split word: the split, and above it 0 for a whole split or
+// 1 + the state (0 .. 3) that a fine item computes of it.
+constexpr uint32_t kPartShift = 28;
+constexpr uint32_t kSplitMask = (1u << kPartShift) - 1;
+// In row_info's split count: the row runs as fine items, four partial slots
+// a split.
+constexpr uint32_t kFineRow = 0x80000000u;
+// Keys of a split above which fine items cannot cover a state (four
+// wavefronts of four 32-key chunks, four states).
+constexpr uint32_t kMaxFineSplit = 2048;
+
 // Split-K work plan for the MFMA decode kernel.
 struct DecodePlan {
-    const uint32_t *work;         // [num_work][4]: (row, split, index of the split's first
+    const uint32_t *work;         // [num_work][4]: (row, split word, index of the split's first
                                   // block id in `tables`, the row's keys); 16-byte aligned,
                                   // launch_work records readable; a zero-key row has one item
-    const uint32_t *row_info;     // [T][2]: (first partial index, number of splits); (0, 0) for
-                                  // rows the plan does not cover
-    const uint32_t *reduce_rows;  // [num_reduce_rows]: rows with more than one split
+    const uint32_t *row_info;     // [T][2]: (first partial index, number of splits, kFineRow);
+                                  // (0, 0) for rows the plan does not cover
+    const uint32_t *reduce_rows;  // [num_reduce_rows][4]: (row, its row_info, its keys) of the rows
+                                  // with more than one split and the fine rows; 16-byte aligned,
+                                  // launch_reduce records readable
     uint32_t num_work;
     uint32_t num_reduce_rows;
     uint32_t split_keys;          // keys per split, a multiple of 32, <= kMaxSplitKeys
@@ -184,6 +197,11 @@ struct DecodePlan {
     // each keeping two of the tile's four softmax states, so pack <= W / 2 *
     // (16 / group) and each wavefront walks half of the split's chunks.
     bool shared_pairs;
+    // With arrivals, [rows][kv_heads] counters that are zero between
+    // launches, the workgroup that finishes a row's last item for a KV head
+    // merges its partials and no reduce kernel runs; only for plans without
+    // packs, on 2 or more wavefronts.  Null: the reduce kernel.
+    uint32_t *arrivals;
 };
 
 constexpr uint32_t kNoMate = 0xffffffffu;

@@ -525,6 +525,33 @@ bool canonical_decode_rows(vo_step_meta *m) {
     return true;
 }
 
+// Fine items (one state of a split per workgroup, paged_decode.hip): for
+// plans of fewer than decode_fine_limit workgroups, the rows of more than
+// kFineMinKeys keys.  Measured a call, whole / fine: 8 rows of 1000-2000 keys
+// of 128 dims (64 workgroups) 24.2 / 17.2 us, 16 of 1500-2000 (128) 28.5 /
+// 25.5, but 24 of them (192) 32.9 / 37.1 and 16 of 1100-4000 (200) 36.0 /
+// 36.7: past five eighths of the CUs the whole items already draw what the
+// HBM gives, and the fine ones only add partials.  One row of 1100 keys:
+// 14.4 / 11.1 us at 128 dims, 11.0 / 11.2 at 64, where a split's chain of
+// chunks is as short as the merge is long.  VO_DECODE_FINE overrides the
+// limit (0: off; a tuning knob, read per plan and at creation).
+constexpr uint64_t kFineMinKeys = 1024;
+
+uint64_t decode_fine_limit(uint64_t num_cus) {
+    const int env = env_int("VO_DECODE_FINE", -1);
+    return env >= 0 ? static_cast<uint64_t>(env) : num_cus * 5 / 8;
+}
+
+// Whether the decode launch merges the partials itself (plans without packs;
+// VO_DECODE_ARRIVE=0: the reduce kernel does, a tuning knob).
+bool decode_arrive() { return env_int("VO_DECODE_ARRIVE", 1) != 0; }
+
+// States of a row that hold keys, and so its fine items: four per whole
+// split, and one per 32-key chunk of a shorter one.
+uint64_t fine_items(uint64_t keys, uint64_t L) {
+    return 4 * (keys / L) + std::min<uint64_t>(4, (keys % L + 31) / 32);
+}
+
 // Split-K plan over the rows listed in `rows` (every row of the step when
 // rows is null).  Rows outside the plan get row_info (0, 0).
 vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32_t> *rows) {
@@ -536,36 +563,56 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
     for (uint64_t i = 0; i < R; ++i) parts += row_splits(m->row_num_keys[row_at(i)], L);
     if (parts > m->max_parts) return fail_capacity("split-K partials per step", parts, m->max_parts);
 
+    const bool streaming = pk.fixed() ? m->fixed.streaming : decode_streaming(m);
+    const int waves = decode_waves();
+    // Fine items need four wavefronts, splits they can cover, partial slots,
+    // and no blocks that several rows read (packs serve those).
+    const bool fine = streaming && !pk.fixed() && waves == 4 && L % 128 == 0 &&
+                      L <= kernels::kMaxFineSplit && 4 * parts <= m->fine_slots &&
+                      parts * m->kv_heads < decode_fine_limit(m->num_cus);
+    auto fine_row = [&](uint64_t keys) { return fine && keys > kFineMinKeys; };
+    uint64_t items = 0;
+    for (uint64_t i = 0; i < R; ++i) {
+        const uint64_t nk = m->row_num_keys[row_at(i)];
+        items += fine_row(nk) ? fine_items(nk, L) : row_splits(nk, L);
+    }
+
     const uint32_t *dp;
-    uint32_t *work = pk.add(kRegWork, 4 * parts, &dp);
+    uint32_t *work = pk.add(kRegWork, 4 * items, &dp);
     m->plan.work = dp;
     uint32_t *row_info = pk.add(kRegRowInfo, 2 * T, &dp);
     m->plan.row_info = dp;
-    uint32_t *reduce_rows = pk.add(kRegReduceRows, R, &dp);
+    uint32_t *reduce_rows = pk.add(kRegReduceRows, 4 * R, &dp);
     m->plan.reduce_rows = dp;
     // Work order, longest first: every full split (L keys) in row order, then
     // each row's shorter last split by descending length.  The hardware deals
     // workgroups out in grid order as slots free up, so the short items fill
     // the gaps at the end instead of a full split starting last and running
     // alone.  Partials are addressed by (row, split), so the order changes no
-    // arithmetic.
+    // arithmetic.  Fine items, short chains of work, come last.
     if (rows) std::fill(row_info, row_info + 2 * T, 0u);
     uint64_t n = 0, nred = 0;
     for (uint64_t i = 0; i < R; ++i) {
         const uint64_t r = row_at(i);
-        const uint64_t ns = row_splits(m->row_num_keys[r], L);
+        const uint64_t nk = m->row_num_keys[r];
+        const uint64_t ns = row_splits(nk, L);
+        const bool fr = fine_row(nk);
         row_info[2 * r] = static_cast<uint32_t>(n);
-        row_info[2 * r + 1] = static_cast<uint32_t>(ns);
-        n += ns;
-        if (ns > 1) reduce_rows[nred++] = static_cast<uint32_t>(r);
+        row_info[2 * r + 1] = static_cast<uint32_t>(ns) | (fr ? kernels::kFineRow : 0u);
+        n += fr ? 4 * ns : ns;
+        if (ns > 1 || fr) {
+            uint32_t *rec = reduce_rows + 4 * nred++;
+            rec[0] = static_cast<uint32_t>(r);
+            rec[1] = row_info[2 * r];
+            rec[2] = row_info[2 * r + 1];
+            rec[3] = static_cast<uint32_t>(nk);
+        }
     }
     m->tail_items.clear();
     uint64_t f = 0;
-    const bool streaming = pk.fixed() ? m->fixed.streaming : decode_streaming(m);
     // Packing needs shared blocks, so a streaming plan never packs; a fixed
     // launch keeps one item per (row, split).
     uint32_t mode = (pk.fixed() || streaming || L % m->block_size != 0) ? kPackOff : decode_pack_mode();
-    const int waves = decode_waves();
     // Shared packs need 4 wavefronts (the kernel keeps one softmax state per
     // wavefront in registers and stages four chunks).
     if (mode == kPackShared && waves != 4) mode = kPackOneTile;
@@ -585,6 +632,7 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
         uint64_t nf = 0;
         for (uint64_t i = 0; i < R; ++i) {
             const uint64_t r = row_at(i);
+            if (fine_row(m->row_num_keys[r])) continue;
             for (uint64_t sp = 0; sp < m->row_num_keys[r] / L; ++sp, ++nf) {
                 work[4 * nf] = static_cast<uint32_t>(r);
                 work[4 * nf + 1] = static_cast<uint32_t>(sp);
@@ -596,6 +644,7 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
     for (uint64_t i = 0; i < R; ++i) {
         const uint64_t r = row_at(i);
         const uint64_t nk = m->row_num_keys[r];
+        if (fine_row(nk)) continue;
         if (nk % L != 0 || nk == 0)
             m->tail_items.push_back({static_cast<uint32_t>(nk % L), static_cast<uint32_t>(r),
                                      static_cast<uint32_t>(nk / L)});
@@ -624,23 +673,37 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
         if (P > 1) std::fill(mates + (P - 1) * f, mates + (P - 1) * (f + 1), kernels::kNoMate);
         ++f;
     }
-    const uint64_t num_work = f;  // = parts unless packed
+    for (uint64_t i = 0; fine && i < R; ++i) {
+        const uint64_t r = row_at(i);
+        const uint64_t nk = m->row_num_keys[r];
+        if (!fine_row(nk)) continue;
+        const uint64_t n_items = fine_items(nk, L);
+        for (uint64_t k = 0; k < n_items; ++k, ++f) {
+            work[4 * f] = static_cast<uint32_t>(r);
+            work[4 * f + 1] = static_cast<uint32_t>(k / 4) |
+                              static_cast<uint32_t>(k % 4 + 1) << kernels::kPartShift;
+        }
+    }
+    const uint64_t num_work = f;  // = items unless packed
     // The rest of each record: where the split's block ids start in the
     // tables, and the (leading) row's key count.
     for (uint64_t i = 0; i < num_work; ++i) {
         const uint32_t row = work[4 * i];
-        const uint64_t split = work[4 * i + 1];
+        const uint64_t split = work[4 * i + 1] & kernels::kSplitMask;
         work[4 * i + 2] =
             static_cast<uint32_t>(m->table_off[m->row_seq[row]] + split * L / m->block_size);
         work[4 * i + 3] = m->row_num_keys[row];
     }
     m->decode_parts = parts;
+    m->decode_items = num_work - items + parts;  // a split of fine items counts once
     m->plan.pack = P;
     m->plan.num_work = static_cast<uint32_t>(num_work);
     m->plan.num_reduce_rows = static_cast<uint32_t>(nred);
     m->plan.split_keys = static_cast<uint32_t>(L);
     m->plan.part_acc = m->d_part_acc;
     m->plan.part_ml = m->d_part_ml;
+    m->plan.arrivals = nullptr;
+    if (!pk.fixed() && P == 1 && waves == 4 && decode_arrive()) m->plan.arrivals = m->d_arrivals;
     m->h_counts[0] = static_cast<uint32_t>(num_work);
     m->h_counts[1] = static_cast<uint32_t>(nred);
     m->plan.counts = m->d_counts;
@@ -918,12 +981,17 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
     // keys of a step are at most entries * block_size, so rows + keys / L
     // bounds the splits (L as configured when the meta is created).
     m->max_parts = max_rows + (max_table_entries * pool->layout.block_size) / decode_split_keys();
+    // Fine items: four partial slots for each of fewer splits than make
+    // decode_fine_limit workgroups, and no more than the step can have.
+    m->fine_slots = 4 * std::min<uint64_t>(m->max_parts,
+                                           decode_fine_limit(m->num_cus) / std::max<uint64_t>(1, m->kv_heads) + 1);
+    const uint64_t slots = std::max(m->max_parts, m->fine_slots);
 
     const uint64_t u32s = (max_seqs + 1) + max_table_entries + 3 * max_rows  // offsets, tables, row arrays
                           + max_rows                                         // write slots
                           + 3 * max_rows                                     // write plan
                           + max_rows                                         // positions
-                          + 4 * m->max_parts + 3 * max_rows                  // decode plan
+                          + 4 * slots + 6 * max_rows                         // decode plan
                           + 4 * (max_rows + max_seqs)                        // prefill plan
                           + (5 + kernels::kPipeFirstWords) * (max_rows + max_seqs) + 1  // its slot plan
                           + max_seqs                                         // last rows
@@ -934,10 +1002,15 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
     if (err == hipSuccess) err = m->stage.create(m->buf_bytes);
     if (err == hipSuccess)
         err = hipMalloc(reinterpret_cast<void **>(&m->d_part_acc),
-                        m->max_parts * max_query_heads * m->head_dim * sizeof(float));
+                        slots * max_query_heads * m->head_dim * sizeof(float));
     if (err == hipSuccess)
         err = hipMalloc(reinterpret_cast<void **>(&m->d_part_ml),
-                        m->max_parts * max_query_heads * 2 * sizeof(float));
+                        slots * max_query_heads * 2 * sizeof(float));
+    if (err == hipSuccess)
+        err = hipMalloc(reinterpret_cast<void **>(&m->d_arrivals),
+                        max_rows * m->kv_heads * sizeof(uint32_t));
+    if (err == hipSuccess)
+        err = hipMemset(m->d_arrivals, 0, max_rows * m->kv_heads * sizeof(uint32_t));
     if (err == hipSuccess)
         err = hipMalloc(reinterpret_cast<void **>(&m->d_tokens), max_rows * sizeof(uint32_t));
     if (err == hipSuccess) err = m->tokens_stage.create(max_rows * sizeof(uint32_t));
@@ -961,6 +1034,7 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
         m->stage.destroy();
         if (m->d_part_acc) (void)hipFree(m->d_part_acc);
         if (m->d_part_ml) (void)hipFree(m->d_part_ml);
+        if (m->d_arrivals) (void)hipFree(m->d_arrivals);
         if (m->side) (void)hipStreamDestroy(m->side);
         if (m->fork) (void)hipEventDestroy(m->fork);
         if (m->join) (void)hipEventDestroy(m->join);
@@ -984,6 +1058,7 @@ extern "C" void vo_step_meta_destroy(vo_step_meta *m) {
     (void)hipFree(m->d_buf);
     (void)hipFree(m->d_part_acc);
     (void)hipFree(m->d_part_ml);
+    (void)hipFree(m->d_arrivals);
     if (m->side) {
         (void)hipStreamSynchronize(m->side);
         (void)hipStreamDestroy(m->side);
@@ -1177,7 +1252,7 @@ extern "C" int32_t vo_step_meta_fix_launch(vo_step_meta *m, uint64_t work_headro
     const uint64_t S = f.seqs;
     const uint64_t caps[kNumRegions] = {
         2, S + 1, f.entries_cap, S, S, f.has_positions ? S : 0, S, 3 * S,
-        4 * f.work_cap, 2 * S, S, S, 0, 0, 0};
+        4 * f.work_cap, 2 * S, 4 * S, S, 0, 0, 0};
     uint64_t off = 0;
     for (int r = 0; r < kNumRegions; ++r) {
         off = align_up(off, 256);
@@ -1206,7 +1281,7 @@ extern "C" int32_t vo_step_meta_decode_plan(const vo_step_meta *m, uint64_t *wor
                                             uint64_t *partials, uint32_t *pack) {
     if (!m || !work_items || !partials || !pack) return fail_argument("decode_plan", "null argument");
     if (!m->decode_planned) return fail_argument("decode_plan", "the last upload has no decode plan");
-    *work_items = m->plan.num_work;
+    *work_items = m->decode_items;
     *partials = m->decode_parts;
     *pack = m->plan.pack ? m->plan.pack : 1;
     clear_error();

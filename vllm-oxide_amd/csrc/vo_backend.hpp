@@ -193,6 +193,7 @@ struct vo_step_meta {
     uint64_t head_dim = 0;
 
     uint64_t max_seqs = 0, max_rows = 0, max_entries = 0, max_heads = 0, max_parts = 0;
+    uint64_t fine_slots = 0;  // partial slots of a plan of fine decode items (decode_fine_rows)
 
     vo::MetaKind kind = vo::kNone;
     uint64_t block_size = 0;
@@ -223,6 +224,9 @@ struct vo_step_meta {
     // Split-K partials (fp32).
     float *d_part_acc = nullptr;
     float *d_part_ml = nullptr;
+    // Arrival counters of the rows' work items [max_rows][kv_heads], zero
+    // between launches (the decode kernel's in-launch merge).
+    uint32_t *d_arrivals = nullptr;
 
     vo::kernels::MetaView view{};
     const uint32_t *d_write_slots = nullptr;  // slots with superseded rows = kSkipSlot
@@ -239,6 +243,7 @@ struct vo_step_meta {
     std::vector<uint64_t> seq_keys;    // scratch of plan_decode: keys read per sequence
     std::vector<uint32_t> decode_rows; // rows of a prefill step planned on the decode kernel
     uint64_t decode_parts = 0;         // split-K partials of the plan (work items before packing)
+    uint64_t decode_items = 0;         // its work items, a split of fine items counted once
     std::unordered_map<uint64_t, uint32_t> pack_open;  // scratch of plan_decode: open packs by hash
     std::vector<uint32_t> pack_fill;                   // scratch of plan_decode: rows per pack
     vo::kernels::PrefillPlan prefill_plan{};

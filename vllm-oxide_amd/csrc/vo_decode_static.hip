@@ -11,7 +11,7 @@
 // CSR table offsets [S+1], tables [entries], key counts [S] (context + 1).
 //
 // Scratch.  `scratch` holds, per call: the plan's two counts, row_info [S][2],
-// reduce_rows [S], work [cap][4] and the partials (m, l) [cap][heads][2] and
+// reduce_rows [S][4] (after the 32 MiB), work [cap][4] and the partials (m, l) [cap][heads][2] and
 // acc [cap][heads][head_dim] fp32, cap = S * ceil(max_keys / split) work
 // items.  Each GPU holds its own copy, whose address hipGetSymbolAddress
 // gives once per device (the array's name is not a device address in host
@@ -47,11 +47,12 @@ namespace {
 // at 64 heads.
 constexpr uint64_t kScratchBytes = 32ull << 20;
 constexpr uint64_t kMaxSeqs = 4096;
+constexpr uint64_t kReduceBytes = kMaxSeqs * 16;  // the rows to reduce, behind the rest
 constexpr int kMaxDevices = 64;
 
 }  // namespace
 
-static __device__ __align__(256) uint8_t scratch[kScratchBytes];
+static __device__ __align__(256) uint8_t scratch[kScratchBytes + kReduceBytes];
 
 namespace {
 
@@ -87,7 +88,8 @@ struct ScratchLayout {
         };
         counts = take(2 * 4);
         row_info = take(2 * S * 4);
-        reduce_rows = take(S * 4);
+        (void)take(S * 4);  // the limit counts four bytes a row for reduce_rows
+        reduce_rows = kScratchBytes;
         work = take(4 * cap * 4);
         part_ml = take(cap * heads * 2 * 4);
         part_acc = take(cap * heads * hd * 4);
@@ -181,7 +183,13 @@ __global__ __launch_bounds__(kPlanThreads) void decode_static_plan_kernel(
             w[2] = base + sp * blocks_per_split;
             w[3] = nk;
         }
-        if (n > 1) reduce_rows[red++] = s;
+        if (n > 1) {
+            uint32_t *rec = reduce_rows + 4 * static_cast<uint64_t>(red++);
+            rec[0] = s;
+            rec[1] = row_info[2 * s];
+            rec[2] = n;
+            rec[3] = nk;
+        }
     }
     if (tid == 0) {
         counts[0] = total_items;
