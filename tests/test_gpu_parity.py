@@ -906,6 +906,28 @@ def test_prefill_pipe_kernel_bitwise_equals_dma_kernel(vo, gpu_backend, monkeypa
     assert np.array_equal(_bits(outs["1"]), _bits(outs["0"]))
 
 
+@pytest.mark.parametrize("kvh,slots", [(8, ""), (8, "1"), (2, "3")])
+def test_prefill_pipe_kernel_eight_heads_bitwise(vo, gpu_backend, monkeypatch, kvh, slots):
+    """With 8 query heads to a KV head the pipelined kernel runs two quads of
+    heads per KV head in steps with rows past 1024 keys: bitwise the
+    8-wavefront DMA kernel, at the item lengths of the test above; and a step
+    up to 1024 keys stays with that kernel."""
+    _say(f"prefill pipelined kernel, 8 heads per KV head ({kvh} KV heads, slots {slots or 'default'})")
+    monkeypatch.setenv("VO_PREFILL_PIPE_SLOTS", slots)
+    ctx = [0, 63, 64, 127, 128, 130, 191, 192, 255, 960, 3001, 4095]
+    new = [64, 1, 65, 2, 64, 31, 33, 1, 129, 64, 77, 64]
+    for n, kernel in ((12, "prefill_pipe"), (10, "prefill_dma")):
+        wl = W.build(vo, gpu_backend, kind="prefill", heads=8 * kvh, kv_heads=kvh, head_dim=128,
+                     block_size=16, num_blocks=1200, context_lens=ctx[:n], num_new=new[:n], seed=73)
+        outs = {}
+        for pipe in ("1", "0"):
+            monkeypatch.setenv("VO_PREFILL_PIPE", pipe)
+            out, ran = _out_with_prefill_instances(vo, wl, gpu_backend)
+            assert ran == {kernel if pipe == "1" else "prefill_dma"}, ran
+            outs[pipe] = out.clone()
+        assert np.array_equal(_bits(outs["1"]), _bits(outs["0"])), n
+
+
 MIXED_CTX = [0, 1, 15, 16, 17, 63, 64, 65, 700, 1023, 1024, 1025, 3000, 0, 100, 700, 5, 2047]
 MIXED_NEW = [1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 64, 100, 200, 2, 33]
 

@@ -428,7 +428,7 @@ __global__ __launch_bounds__(64 * G * R) __attribute__((amdgpu_waves_per_eu(
     __shared__ __align__(1024) uint8_t st0[D::STAGE];
     __shared__ __align__(1024) uint8_t st1[D::STAGE];
     __shared__ __align__(1024) uint8_t st2[D::STAGE];
-    __shared__ uint32_t redo;  // bit g: a row of row group g left the fixed-offset range
+    __shared__ uint32_t redo;  // bit g: a row of recompute group g left the fixed-offset range
 
     const uint32_t kvh = blockIdx.x % kv_heads;
     const uint32_t rest = blockIdx.x / kv_heads;
@@ -450,6 +450,11 @@ __global__ __launch_bounds__(64 * G * R) __attribute__((amdgpu_waves_per_eu(
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t head = wave % G;
     const uint32_t rg = wave / G;
+    // The 32 rows of up to four query heads are recomputed together (below):
+    // with 8 heads, each row group is two recompute groups, as in the
+    // pipelined kernel, whose workgroups hold four.
+    constexpr uint32_t kQuads = G == 8 ? 2 : 1;
+    const uint32_t rgroup = rg * kQuads + head / (G / kQuads);
     const uint32_t c = lane & 31;
     const uint32_t gl = lane >> 5;
     const uint32_t qhead = kvh * G + head;
@@ -688,21 +693,22 @@ __global__ __launch_bounds__(64 * G * R) __attribute__((amdgpu_waves_per_eu(
     // a 32-row group is past that, the group's rows are recomputed with the
     // running max (raised by more than kLazyLog2 at a time, per wave) in a
     // second pass, in which the waves of the other groups stay idle and keep
-    // their first-pass results.  The decision is per row group, never per
+    // their first-pass results.  The decision is per row group (and quad of
+    // heads), never per
     // workgroup, so a row's result does not depend on whether its group
     // shares a workgroup with the item's other group (which a plan of few
     // items avoids): the same rows give the same bits in any batch.
     if (fixed_offset) {
         pass(std::true_type{});
         const bool ok = l_run < kOverflowSum && all_finite(o_acc);  // false for inf and NaN too
-        if (__builtin_amdgcn_ballot_w64(row_ok && !ok) != 0 && lane == 0) atomicOr(&redo, 1u << rg);
+        if (__builtin_amdgcn_ballot_w64(row_ok && !ok) != 0 && lane == 0) atomicOr(&redo, 1u << rgroup);
     } else if (tid == 0) {
-        redo = (1u << R) - 1;
+        redo = (1u << (R * kQuads)) - 1;
     }
     wait_barrier<0>();
     const uint32_t again = uniform_u32(redo);
     if (again != 0) {
-        live = ((again >> rg) & 1u) != 0;
+        live = ((again >> rgroup) & 1u) != 0;
         pass(std::false_type{});
     }
     // Every wave's DMA has landed and its stage reads are done: the stages
@@ -814,8 +820,9 @@ __device__ __forceinline__ PipeItem pipe_item(const uint32_t *desc, const uint32
     return it;
 }
 
-// Persistent: workgroup w serves KV head w % kv_heads and runs the items of
-// slot w / kv_heads (plan[slot] .. plan[slot + 1] - 1 of the descriptors at
+// Persistent: workgroup w serves KV head w % kv_heads (four of its query
+// heads: quad w / kv_heads % quads) and runs the items of
+// slot w / (kv_heads quads) (plan[slot] .. plan[slot + 1] - 1 of the descriptors at
 // plan + num_slots + 1) back to back.  The four LDS stages form one ring
 // across the items: item k's tile t sits in stage (T_k + t) % 4 with
 // T_k+1 = T_k + n_k, and the block table in LDS continues past an item's
@@ -826,8 +833,8 @@ __device__ __forceinline__ PipeItem pipe_item(const uint32_t *desc, const uint32
 // the one stage that holds no prefetched tile.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void prefill_pipe_kernel(
     const uint16_t *__restrict__ k_pool, const uint16_t *__restrict__ v_pool, uint32_t kv_heads,
-    const uint32_t *__restrict__ tables, const uint32_t *__restrict__ plan, uint32_t num_slots,
-    const uint16_t *__restrict__ q, uint16_t *__restrict__ out, uint32_t num_heads, float scale_log2,
+    uint32_t quads, const uint32_t *__restrict__ tables, const uint32_t *__restrict__ plan,
+    uint32_t num_slots, const uint16_t *__restrict__ q, uint16_t *__restrict__ out, uint32_t num_heads, float scale_log2,
     uint32_t fixed_offset, uint32_t pool_bytes) {
     constexpr int HD = 128, G = 4, KS = 8, DT = 4;
     constexpr uint32_t kTile = kBS * HD;
@@ -843,8 +850,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     // barrier, when every wave has read it for item k - 1.
     __shared__ uint32_t redo[2];
 
+    // The quads of a KV head's query heads are kv_heads workgroups apart: with
+    // 8 KV heads on the same XCD, whose L2 then serves both.
     const uint32_t kvh = blockIdx.x % kv_heads;
-    const uint32_t slot = blockIdx.x / kv_heads;
+    const uint32_t quad = blockIdx.x / kv_heads % quads;
+    const uint32_t slot = blockIdx.x / (kv_heads * quads);
     // The slot's first record (its first item's descriptor, that item's
     // tiles 0-2 block ids, the next item's first twelve) sits at an address
     // that depends only on the slot, so the first DMAs, Q loads and table
@@ -856,7 +866,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     if (i >= i_end) return;  // the host plan gives every slot an item
 
     const uint32_t head = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t qhead = kvh * G + head;
+    const uint32_t qhead = (kvh * quads + quad) * G + head;
 
     // Per-lane values.  They are rebuilt after the pipelined loop from a
     // copy of the thread id that the compiler cannot see through, so that
@@ -1322,8 +1332,12 @@ bool prefill_narrow_enabled() {
     return !(v && std::string(v) == "0");
 }
 
+// With 8 query heads to a KV head the pipelined kernel runs steps with a row
+// of more keys than this (both sides measured in launch_gr).
+constexpr uint32_t kPipe8MinKeys = 1024;
+
 // VO_PREFILL_PIPE=0 runs the 8-wavefront DMA kernel instead of the
-// pipelined one at head_dim 128, GQA 4 (A/B).  Read at every launch.
+// pipelined one at head_dim 128, GQA 4 and 8 (A/B).  Read at every launch.
 bool prefill_pipe_enabled() {
     const char *v = std::getenv("VO_PREFILL_PIPE");
     return !(v && std::string(v) == "0");
@@ -1358,13 +1372,22 @@ hipError_t launch_gr(const PoolLayer &pool, const MetaView &meta, const PrefillP
                            meta.table_off, meta.tables, plan.work, q, out, num_heads, scale_log2);
         if (hipError_t err = hipGetLastError(); err != hipSuccess) return err;
     }
-    if constexpr (HD == 128 && G == 4 && R == 2) {
-        // 64-row workgroups at the Llama-3-8B shape: the pipelined kernel.
+    if constexpr (HD == 128 && ((G == 4 && R == 2) || G == 8)) {
+        // 64-row workgroups of four query heads (the Llama-3-8B shape): the
+        // pipelined kernel.  With 8 query heads to a KV head (the 70B layer)
+        // two such workgroups walk its tiles, in place of one of 8 wavefronts
+        // for each 32 rows: half the LDS reads per MFMA and the softmax
+        // beside the MFMAs.  8 x 512 rows at contexts 0-8000: 582 -> 543 us,
+        // 1 x 300 at 5000: 111 -> 101, 3 x 451 at 0-6000: 172 -> 165 (the
+        // same bits).  Its items cost more to start and end: up to 1024 keys the other kernel is
+        // the faster one (6 x 512 rows, no context: 49.8 against 53.0 us).
         if (regs_items < plan.num_items && plan.pipe != nullptr && plan.pipe_slots != 0 &&
-            prefill_pipe_enabled()) {
+            prefill_pipe_enabled() && (G == 4 || plan.max_keys > kPipe8MinKeys)) {
             KernelTimer timer("prefill_pipe", stream);
-            hipLaunchKernelGGL(prefill_pipe_kernel, dim3(plan.pipe_slots * pool.kv_heads), dim3(256), 0,
-                               stream, pool.k, pool.v, pool.kv_heads, meta.tables, plan.pipe,
+            constexpr uint32_t kQuads = G / 4;
+            hipLaunchKernelGGL(prefill_pipe_kernel, dim3(plan.pipe_slots * pool.kv_heads * kQuads),
+                               dim3(256), 0, stream, pool.k, pool.v, pool.kv_heads, kQuads,
+                               meta.tables, plan.pipe,
                                plan.pipe_slots, q, out, num_heads, scale_log2,
                                prefill_fixed_offset() ? 1u : 0u, static_cast<uint32_t>(pool.elems * 2));
             return hipGetLastError();
