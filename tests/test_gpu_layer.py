@@ -134,6 +134,32 @@ def test_streaming_matmul_shapes(vo, gpu_backend, rows, n, k):
         assert torch.equal(b16, got.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("rows", [1, 5, 8, 9])
+@pytest.mark.parametrize("n,k", [(16, 1024), (2032, 3072), (2048, 8192), (2064, 4096)])
+def test_few_output_matmul_shapes(vo, gpu_backend, rows, n, k):
+    """Weights of at most 2048 rows and up to 8 batch rows, where a matrix
+    instruction covers two parts of K: one step of a part and several, one
+    weight tile and the most, and the first sizes past either limit.  Bounds
+    as in test_streaming_matmul_shapes; a row does not depend on its batch."""
+    import torch
+    _say(f"few-output matmul {rows}x{k} . {n}x{k}^T")
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows + n + k)
+    x = torch.randn((rows, k), generator=gen, device="cuda:0").to(torch.bfloat16)
+    w = (0.02 * torch.randn((n, k), generator=gen, device="cuda:0")).to(torch.bfloat16)
+    want = x.double() @ w.double().T
+    bound = 1e-5 * want.abs().max()
+    got = gpu_backend.matmul(x, w, out_dtype=torch.float32)
+    assert (got - want).abs().max() < bound
+    acc = torch.ones_like(got)
+    gpu_backend.matmul(x, w, out=acc, accumulate=True)
+    assert (acc - 1 - want).abs().max() < bound + 2 ** -22 * (1 + want.abs().max())
+    assert torch.equal(gpu_backend.matmul(x, w), got.to(torch.bfloat16))
+    if rows <= 8 and n <= 2048:
+        last = gpu_backend.matmul(x[-1:].contiguous(), w, out_dtype=torch.float32)
+        assert torch.equal(last[0], got[-1])
+
+
 def test_skinny_matmul_rows_independent_of_batch(vo, gpu_backend):
     """The weight-streaming kernel's output for a row does not depend on the
     other rows of the batch: each of 4 rows equals, bitwise, the same row

@@ -397,40 +397,49 @@ __device__ __forceinline__ void store_out4(void *out, uint64_t o, floatx4 t) {
     }
 }
 
-// Backend::matmul for 1..4 rows and a small weight (up to 2^24 values):
-// streaming the weight is the whole cost.  A workgroup owns 16 weight rows
-// (outputs) and splits K over its 8 wavefronts; each wavefront runs
-// v_mfma_f32_16x16x32_bf16 with A = 16 weight rows x 32 k (one 16-byte load
-// per lane) and B = x^T (the batch rows in columns 0..rows-1; columns past
-// the batch repeat its last row and are not stored, so no lane branches), 8
-// steps of loads issued before their MFMAs.  The 8 partial tiles are summed
-// through LDS in wavefront order, so an output depends only on its own row of
-// x, whatever the batch size.  Ordinary loads: a step reads 64 bytes of each
-// weight row, half a cache line, and the next step the other half;
-// non-temporal loads measured 10-15% slower (the line is fetched twice).
-// Here, in the order of one launch and one round of loads, it beats
-// stream_gemm_kernel below (a weight of 3072 x 2048, 4 rows: 5.1 against
-// 5.8 us; 4096 x 4096: 8.7 against 9.4); on larger weights, or with more
-// rows, every workgroup's reads of x from L2 make it the slower one.
+// Backend::matmul for few rows and a small weight (up to 2^24 values):
+// streaming the weight is the whole cost.  A workgroup owns 16 / P weight rows
+// (outputs) and splits K over its 8 wavefronts and, within one, over P parts;
+// each wavefront runs v_mfma_f32_16x16x32_bf16 with A = P blocks of 16 / P
+// weight rows, block p from part p of its columns, and B = x^T laid out alike
+// (the batch rows in columns 0..rows-1 of each block; columns past the batch
+// repeat its last row and are not stored, so no lane branches), so that the P
+// diagonal blocks of D hold the parts' sums and the rest is not looked at.
+// U steps of loads are issued before their MFMAs.  The partial sums are added
+// through LDS in order of wavefront and part, so an output depends only on its
+// own row of x, whatever the batch size.  Ordinary loads: a step reads 64
+// bytes of each weight row, half a cache line, and the next step the other
+// half; non-temporal loads measured 10-15% slower (the line is fetched twice).
+//
+// P = 1 (up to 4 rows), 8 steps of loads in flight: here, in the order of one
+// launch and one round of loads, it beats stream_gemm_kernel below (a weight
+// of 3072 x 2048, 4 rows: 5.1 against 5.8 us; 4096 x 4096: 8.7 against 9.4);
+// on larger weights, or with more rows, every workgroup's reads of x from L2
+// make it the slower one.
+// P = 2 (up to 8 rows): weights of at most 2048 rows, whose 128 tiles of 16
+// leave half the 256 CUs idle: a weight of 2048 x 8192, 4 rows, took 13.4 us
+// with P = 1 and takes 9.1 (3.7 TB/s); 2048 x 2048 4.9 and 4.0.  P = 4 adds
+// nothing (10.2, 4.6), and 2 steps in flight do as well as 4 to 16 (9.2-9.5).
+// From 3072 rows on P = 1 is the better one (5.0 against 5.3).
 constexpr int kSkinnyWaves = 8;
-constexpr int kSkinnyU = 8;     // 32-k steps per load batch
-constexpr int kSkinnyRows = 4;  // largest batch the kernel is used for
 constexpr uint64_t kSkinnyWeight = 1ull << 24;  // largest weight
+constexpr uint32_t kSkinnyHalfN = 2048;         // largest weight rows of P = 2
 
-template <int MODE>
+template <int MODE, int P, int U>
 __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, uint32_t rows, uint32_t n,
     uint32_t k, void *__restrict__ out) {
-    constexpr int U = kSkinnyU;
+    static_assert(P == 1 || P == 2, "blocks of the diagonal");
+    constexpr uint32_t R = 16 / P;  // weight rows of the workgroup, largest batch
     __shared__ floatx4 part[kSkinnyWaves][64];
-    const uint32_t n0 = blockIdx.x * 16;
+    const uint32_t n0 = blockIdx.x * R;
     const uint32_t wave = threadIdx.x >> 6;
     const uint32_t lane = threadIdx.x & 63;
-    const uint32_t kw = k / kSkinnyWaves;  // a multiple of 32 * U
-    const uint32_t r = lane & 15, kg = lane >> 4;
-    const uint16_t *wp = w + static_cast<uint64_t>(n0 + r) * k + wave * kw + 8 * kg;
-    const bool live = r < rows;
-    const uint16_t *xp = x + static_cast<uint64_t>(min(r, rows - 1)) * k + wave * kw + 8 * kg;
+    const uint32_t kw = k / (kSkinnyWaves * P);  // of one part; a multiple of 32 * U
+    const uint32_t r = lane % R, kg = lane >> 4;
+    const uint32_t k0 = (wave * P + (lane & 15) / R) * kw + 8 * kg;
+    const uint16_t *wp = w + static_cast<uint64_t>(n0 + r) * k + k0;
+    const uint16_t *xp = x + static_cast<uint64_t>(min(r, rows - 1)) * k + k0;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
     for (uint32_t kk = 0; kk < kw; kk += 32 * U) {
         u32x4 a[U], b[U];
@@ -447,12 +456,13 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(
     }
     part[wave][lane] = acc;
     __syncthreads();
-    if (wave != 0) return;
+    // Lane l of D holds rows 4 (l / 16) + e, e = 0..3, of column l % 16: block
+    // p's output 4 kg + e of batch row r is in lane 16 kg + r + 40 p (P = 2).
+    if (wave != 0 || (lane & 15) >= R || kg >= 4 / P) return;
     floatx4 t = part[0][lane];
 #pragma unroll
-    for (int v = 1; v < kSkinnyWaves; ++v) t += part[v][lane];
-    // Lane l holds outputs n0 + 4 (l / 16) + e, e = 0..3, of batch row l % 16.
-    if (live) store_out4<MODE>(out, static_cast<uint64_t>(r) * n + n0 + 4 * kg, t);
+    for (int v = 1; v < kSkinnyWaves * P; ++v) t += part[v / P][lane + 40 * (v % P)];
+    if (r < rows) store_out4<MODE>(out, static_cast<uint64_t>(r) * n + n0 + 4 * kg, t);
 }
 
 // Backend::matmul for up to 64 rows: HBM, the weight read once.  MT = tiles
@@ -797,16 +807,25 @@ hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t row
     if (!skinny_gemm_supported(rows, n, k)) return hipErrorInvalidValue;
     KernelTimer timer("matmul_skinny", stream);
     const int mode = !out_f32 ? 0 : (accumulate ? 2 : 1);
-    if (rows <= kSkinnyRows && k % (kSkinnyWaves * 32 * kSkinnyU) == 0 &&
-        static_cast<uint64_t>(n) * k <= kSkinnyWeight) {
-        const dim3 grid(n / 16), block(64 * kSkinnyWaves);
-        if (mode == 0)
-            hipLaunchKernelGGL((skinny_gemm_kernel<0>), grid, block, 0, stream, x, w, rows, n, k, out);
-        else if (mode == 1)
-            hipLaunchKernelGGL((skinny_gemm_kernel<1>), grid, block, 0, stream, x, w, rows, n, k, out);
-        else
-            hipLaunchKernelGGL((skinny_gemm_kernel<2>), grid, block, 0, stream, x, w, rows, n, k, out);
-        return hipGetLastError();
+    if (static_cast<uint64_t>(n) * k <= kSkinnyWeight) {
+        const dim3 block(64 * kSkinnyWaves);
+#define VO_SKINNY(P, U)                                                                          \
+    do {                                                                                         \
+        const dim3 grid(n / 16 * P);                                                             \
+        if (mode == 0)                                                                           \
+            hipLaunchKernelGGL((skinny_gemm_kernel<0, P, U>), grid, block, 0, stream, x, w, rows, \
+                               n, k, out);                                                       \
+        else if (mode == 1)                                                                      \
+            hipLaunchKernelGGL((skinny_gemm_kernel<1, P, U>), grid, block, 0, stream, x, w, rows, \
+                               n, k, out);                                                       \
+        else                                                                                     \
+            hipLaunchKernelGGL((skinny_gemm_kernel<2, P, U>), grid, block, 0, stream, x, w, rows, \
+                               n, k, out);                                                       \
+        return hipGetLastError();                                                                \
+    } while (0)
+        if (rows <= 8 && n <= kSkinnyHalfN && k % (kSkinnyWaves * 2 * 32 * 2) == 0) VO_SKINNY(2, 2);
+        if (rows <= 4 && k % (kSkinnyWaves * 32 * 8) == 0) VO_SKINNY(1, 8);
+#undef VO_SKINNY
     }
     switch ((rows + 15) / 16) {
         case 1: launch_stream_rows<1>(x, w, rows, n, k, out, mode, stream); break;
