@@ -699,6 +699,15 @@ int32_t vo_matmul(vo_gemm *gemm, const void *x, uint64_t rows, uint64_t x_cols, 
                   uint64_t out_features, uint64_t in_features, void *out, int32_t out_dtype,
                   int32_t accumulate, void *stream);
 
+/* vo_matmul by a fused [gate; up] weight [2 * ffn, in_features], then
+ * vo_silu_mul of the two halves: out [rows, ffn] bf16.  gate_up is room for
+ * the product, [rows, 2 * ffn] bf16; decode-sized batches (up to 64 rows of a
+ * weight the library's own kernels take) run as one launch and leave it
+ * alone, rounding the two halves to bf16 in between all the same. */
+int32_t vo_matmul_silu_mul(vo_gemm *gemm, const void *x, uint64_t rows, uint64_t x_cols,
+                           const void *weight, uint64_t ffn, uint64_t in_features, void *gate_up,
+                           void *out, void *stream);
+
 /* ------------------------------------------------------------------ */
 /* Opt-in kernel timing (the reference's opt-in per-op timing,         */
 /* arena.rs:82-87 OpStat, :129-136 enable_profiling)                   */

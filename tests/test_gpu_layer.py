@@ -18,6 +18,7 @@ tolerance written in each test; greedy ids agree wherever the oracle's top-1
 / top-2 gap exceeds the logit tolerance (the gap-aware comparison of the
 reference's HF check, tests/hf_match.rs).
 """
+import ctypes
 import math
 
 import numpy as np
@@ -132,6 +133,40 @@ def test_streaming_matmul_shapes(vo, gpu_backend, rows, n, k):
     b16 = gpu_backend.matmul(x, w)
     if rows <= 16 or (rows <= 64 and k <= 2 * n):  # the same sums, rounded once
         assert torch.equal(b16, got.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("rows", [1, 16, 17, 48, 64, 65])
+@pytest.mark.parametrize("ffn,k", [(16, 512), (24, 512), (2064, 1024), (2576, 1536), (4112, 512),
+                                   (12304, 512), (32784, 512)])
+def test_matmul_silu_mul_shapes(vo, gpu_backend, rows, ffn, k):
+    """SwiGLU in the gate/up product: each workgroup shape with a remainder of
+    its tile pairs, and the forms that run as the two steps, bitwise (24
+    outputs, 65 rows, 16 outputs past 16 rows: the library's product).  Against
+    f64: g, u and the output are each rounded to bf16 (8 significant bits: at
+    most 2^-8 of the value), which silu(g) * u takes up at most 1 + |g| times
+    from g, once from u and once itself, to first order (1.02 covers the
+    rest), beside the 1e-5 of the f32 sums (silu' < 1.1)."""
+    import torch
+    _say(f"matmul_silu_mul {rows}x{k} . 2x{ffn}x{k}^T")
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows + ffn + k)
+    x = torch.randn((rows, k), generator=gen, device="cuda:0").to(torch.bfloat16)
+    w = (0.05 * torch.randn((2 * ffn, k), generator=gen, device="cuda:0")).to(torch.bfloat16)
+    gu = torch.empty((rows, 2 * ffn), dtype=torch.bfloat16, device="cuda:0")
+    out = torch.full((rows, ffn), 7.0, dtype=torch.bfloat16, device="cuda:0")
+    P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    vo._check(vo.lib.vo_matmul_silu_mul(gpu_backend.gemm().handle, P(x), rows, k, P(w), ffn, k, P(gu),
+                                        P(out), vo._stream_ptr(None)))
+    if rows > 64 or ffn % 16 or (rows > 16 and k > 4 * ffn):
+        two = gpu_backend.matmul(x, w)
+        assert torch.equal(out, gpu_backend.silu_mul(two[:, :ffn], two[:, ffn:]))
+        return
+    exact = x.double() @ w.double().T
+    g, u = exact[:, :ffn], exact[:, ffn:]
+    want = g * torch.sigmoid(g) * u
+    sums = 1e-5 * exact.abs().max()
+    bound = (3 + g.abs()) * 2 ** -8 * 1.02 * want.abs() + sums * (1.1 * u.abs() + g.abs()) + 1e-30
+    assert ((out.double() - want).abs() <= bound).all()
 
 
 @pytest.mark.parametrize("rows", [1, 5, 8, 9])

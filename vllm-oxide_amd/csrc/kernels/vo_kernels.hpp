@@ -144,6 +144,10 @@ bool skinny_gemm_supported(uint64_t rows, uint64_t n, uint64_t k);
 hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
                               uint32_t k, void *out, bool out_f32, bool accumulate,
                               hipStream_t stream);
+// The same for a weight [gate; up] of 2 * ffn rows (ffn % 16 == 0) with SwiGLU:
+// out [rows, ffn] = silu(x . gate^T) * (x . up^T).
+hipError_t launch_swiglu_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t ffn,
+                              uint32_t k, uint16_t *out, hipStream_t stream);
 hipError_t launch_matmul_generic(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
                                  uint32_t k, void *out, bool out_f32, bool accumulate,
                                  hipStream_t stream);

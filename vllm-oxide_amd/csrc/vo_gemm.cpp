@@ -226,6 +226,12 @@ vo_status make_plan(vo_gemm *g, const LtApi &api, uint64_t rows, uint64_t n, uin
     return VO_OK;
 }
 
+// Decode-sized batches: the weight-streaming kernel (VO_SKINNY_GEMM=0: off).
+bool skinny_on() {
+    static const bool on = env_int("VO_SKINNY_GEMM", 1) != 0;
+    return on;
+}
+
 }  // namespace
 
 extern "C" int32_t vo_gemm_create(int32_t device, uint64_t workspace_bytes, vo_gemm **out) {
@@ -306,9 +312,7 @@ extern "C" int32_t vo_matmul(vo_gemm *g, const void *x, uint64_t rows, uint64_t 
                                      static_cast<uint32_t>(in_features), out,
                                      out_dtype == VO_DTYPE_F32, accumulate != 0,
                                      static_cast<hipStream_t>(stream)));
-    // Decode-sized batches: the weight-streaming kernel (VO_SKINNY_GEMM=0: off).
-    static const bool skinny_on = env_int("VO_SKINNY_GEMM", 1) != 0;
-    if (skinny_on && kernels::skinny_gemm_supported(rows, out_features, in_features))
+    if (skinny_on() && kernels::skinny_gemm_supported(rows, out_features, in_features))
         return device_status(op, kernels::launch_skinny_gemm(
                                      static_cast<const uint16_t *>(x),
                                      static_cast<const uint16_t *>(weight),
@@ -342,4 +346,33 @@ extern "C" int32_t vo_matmul(vo_gemm *g, const void *x, uint64_t rows, uint64_t 
     if (st != HIPBLAS_STATUS_SUCCESS) return lt_fail(op, "hipblasLtMatmul", st);
     clear_error();
     return VO_OK;
+}
+
+extern "C" int32_t vo_matmul_silu_mul(vo_gemm *g, const void *x, uint64_t rows, uint64_t x_cols,
+                                      const void *weight, uint64_t ffn, uint64_t in_features,
+                                      void *gate_up, void *out, void *stream) {
+    const char *op = "matmul_silu_mul";
+    if (!g) return fail_argument(op, "null gemm");
+    if (ffn > 0x3fffffffull) return fail_capacity("matmul_silu_mul columns", ffn, 0x3fffffffull);
+    // The decode-sized batches of whole tiles: one launch, nothing in gate_up.
+    // Every other form, and every argument the two steps refuse, goes to them.
+    const uint64_t ob = rows * ffn * 2;
+    if (skinny_on() && x && weight && out && in_features == x_cols && ffn % 16 == 0 &&
+        aligned16(x) && aligned16(weight) && aligned16(out) &&
+        kernels::skinny_gemm_supported(rows, 2 * ffn, in_features) &&
+        !overlaps(out, ob, x, rows * x_cols * 2) &&
+        !overlaps(out, ob, weight, 2 * ffn * in_features * 2)) {
+        DeviceGuard guard(g->device);
+        return device_status(op, kernels::launch_swiglu_gemm(
+                                     static_cast<const uint16_t *>(x),
+                                     static_cast<const uint16_t *>(weight),
+                                     static_cast<uint32_t>(rows), static_cast<uint32_t>(ffn),
+                                     static_cast<uint32_t>(in_features),
+                                     static_cast<uint16_t *>(out), static_cast<hipStream_t>(stream)));
+    }
+    if (int32_t rc = vo_matmul(g, x, rows, x_cols, weight, 2 * ffn, in_features, gate_up,
+                               VO_DTYPE_BF16, 0, stream))
+        return rc;
+    return vo_silu_mul(gate_up, 2 * ffn, static_cast<const uint16_t *>(gate_up) + ffn, 2 * ffn,
+                       rows, ffn, out, ffn, stream);
 }

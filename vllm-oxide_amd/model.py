@@ -220,9 +220,7 @@ class Llama:
             _check(attention(q, T, qd, pool.handle, li, mh, attn, s))
             _check(lib.vo_matmul(g, attn, T, qd, _ptr(L["wo"]), H, qd, res, f32, 1, s))
             _check(lib.vo_rmsnorm(res, T, H, _ptr(L["mlp_norm"]), H, eps, nrm, s))
-            _check(lib.vo_matmul(g, nrm, T, H, _ptr(L["wgu"]), 2 * F, H, gu, bf, 0, s))
-            gu_up = _vp(B.gu.data_ptr() + F * 2)
-            _check(lib.vo_silu_mul(gu, 2 * F, gu_up, 2 * F, T, F, act, F, s))
+            _check(lib.vo_matmul_silu_mul(g, nrm, T, H, _ptr(L["wgu"]), F, H, gu, act, s))
             _check(lib.vo_matmul(g, act, T, F, _ptr(L["wd"]), H, F, res, f32, 1, s))
         _check(lib.vo_rmsnorm_last_rows(res, T, H, _ptr(self.final_norm), H, eps, mh,
                                         _ptr(B.last), s))
