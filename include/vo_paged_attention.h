@@ -708,6 +708,16 @@ int32_t vo_matmul_silu_mul(vo_gemm *gemm, const void *x, uint64_t rows, uint64_t
                            const void *weight, uint64_t ffn, uint64_t in_features, void *gate_up,
                            void *out, void *stream);
 
+/* vo_rmsnorm of x [rows, cols] f32 by norm [cols], then vo_matmul into out
+ * [rows, out_features] bf16, or with silu_mul = 1 vo_matmul_silu_mul (weight
+ * [gate; up] of out_features rows, out [rows, out_features / 2]).  normed is
+ * room for [rows, cols] bf16, gate_up for [rows, out_features] bf16 (silu_mul
+ * = 1 only); the few rows of a decode step run as one launch, rounded in
+ * between as the steps are, and leave both alone. */
+int32_t vo_rmsnorm_matmul(vo_gemm *gemm, const float *x, uint64_t rows, uint64_t cols,
+                          const void *norm, float eps, const void *weight, uint64_t out_features,
+                          int32_t silu_mul, void *normed, void *gate_up, void *out, void *stream);
+
 /* ------------------------------------------------------------------ */
 /* Opt-in kernel timing (the reference's opt-in per-op timing,         */
 /* arena.rs:82-87 OpStat, :129-136 enable_profiling)                   */

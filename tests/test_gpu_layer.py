@@ -169,6 +169,51 @@ def test_matmul_silu_mul_shapes(vo, gpu_backend, rows, ffn, k):
     assert ((out.double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("rows,k", [(1, 512), (3, 1536), (4, 1024), (5, 1024), (4, 2048), (8, 2048),
+                                    (9, 2048), (1, 4096)])
+@pytest.mark.parametrize("n", [32, 48, 2080, 8224])
+@pytest.mark.parametrize("swiglu", [0, 1])
+def test_rmsnorm_matmul_shapes(vo, gpu_backend, rows, k, n, swiglu):
+    """RMSNorm inside the product, each workgroup shape with a remainder of its
+    tiles, more rows than wavefronts, and sizes that run as the steps, against
+    the steps in f64.  The normed row is rounded to bf16 (2^-8; at a tie of the
+    f32 value's last bits either way), as is each output: with x~ the normed
+    row, an output differs by at most 2^-8 sum |x~ w| + 2^-8 |o|; SwiGLU takes
+    g's part up 1.1 |u| times and u's |silu(g)| <= |g| times, then rounds."""
+    import torch
+    _say(f"rmsnorm_matmul {rows}x{k} . {n}x{k}^T swiglu {swiglu}")
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows + n + k)
+    x = 3.0 * torch.randn((rows, k), generator=gen, device="cuda:0")
+    norm = (1 + 0.2 * torch.randn((k,), generator=gen, device="cuda:0")).to(torch.bfloat16)
+    w = (0.05 * torch.randn((n, k), generator=gen, device="cuda:0")).to(torch.bfloat16)
+    outputs = n // 2 if swiglu else n
+    out = torch.full((rows, outputs), 7.0, dtype=torch.bfloat16, device="cuda:0")
+    normed = torch.empty((rows, k), dtype=torch.bfloat16, device="cuda:0")
+    gu = torch.empty((rows, n), dtype=torch.bfloat16, device="cuda:0")
+    P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+
+    def run(xs, o):
+        vo._check(vo.lib.vo_rmsnorm_matmul(gpu_backend.gemm().handle, P(xs), xs.shape[0], k, P(norm),
+                                           1e-5, P(w), n, swiglu, P(normed), P(gu), P(o),
+                                           vo._stream_ptr(None)))
+    run(x, out)
+    xd = x.double()
+    xn = xd * torch.rsqrt((xd * xd).mean(1, keepdim=True) + 1e-5) * norm.double()
+    o = xn @ w.double().T
+    # 1.01: second-order terms, and the f32 sums (1e-5 of a sum of magnitudes).
+    err = 1.01 * 2 ** -8 * (xn.abs() @ w.double().abs().T + o.abs())
+    if swiglu:
+        g, u, eg, eu = o[:, :outputs], o[:, outputs:], err[:, :outputs], err[:, outputs:]
+        o = g * torch.sigmoid(g) * u
+        err = 1.1 * eg * (u.abs() + eu) + g.abs() * eu + 2 ** -8 * 1.1 * o.abs()
+    assert ((out.double() - o).abs() <= err + 1e-30).all()
+    if k <= 2048 and rows <= (4 if n >= 8192 else 8):  # whatever the batch
+        one = torch.empty((1, outputs), dtype=torch.bfloat16, device="cuda:0")
+        run(x[-1:].contiguous(), one)
+        assert torch.equal(one[0], out[-1])
+
+
 @pytest.mark.parametrize("rows", [1, 5, 8, 9])
 @pytest.mark.parametrize("n,k", [(16, 1024), (2032, 3072), (2048, 8192), (2064, 4096)])
 def test_few_output_matmul_shapes(vo, gpu_backend, rows, n, k):

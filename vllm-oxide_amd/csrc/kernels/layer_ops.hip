@@ -660,6 +660,146 @@ __global__ __launch_bounds__(64 * NW * KG) void stream_gemm_kernel(
     }
 }
 
+// RMSNorm, then stream_gemm_kernel's product (MODE 0, or 3 with SwiGLU) for the
+// few rows of a decode step, whose RMSNorm alone is a launch of 3 us and a gap.
+// Every workgroup normalises the rows again, one to a wavefront, while its
+// first weight chunk is on its way: 8 loads of 16 bytes per lane and row, out
+// of L2 since all workgroups read the same, a reduction within the wavefront,
+// and the row in bf16 to LDS, where it stays: no DMA and no barrier in the
+// loop over K.  The 16-byte units of a row are swizzled as above.
+//
+// Rows 1 / 4 / 8 / 16, launched back to back, against RMSNorm and the product:
+// 3072 x 2048: 5.7 / 5.9 / 7.1 / 8.7 us, two launches 7.2 / 7.8 / 8.5 / 8.7;
+// 4096 x 2048 with SwiGLU: 9.6 / 9.4 / 10.7 / 10.9, 10.9 / 10.8 / 10.8 / 10.9;
+// 16384 x 2048 with SwiGLU: 16.6 / 16.8 / 17.2 / 17.0, 17.3 / 17.3 / 16.8 / 17.1
+// (a second group of wavefronts per workgroup there: no faster).
+constexpr uint32_t kNormGemmK = 2048;  // largest k
+constexpr uint32_t kNormGemmRows = 8;  // largest batch
+
+template <int MODE, int NW, int KG>
+__global__ __launch_bounds__(64 * NW * KG) void norm_gemm_kernel(
+    const float *__restrict__ x, const uint16_t *__restrict__ norm, float eps,
+    const uint16_t *__restrict__ w, uint32_t rows, uint32_t n, uint32_t k,
+    uint16_t *__restrict__ out) {
+    constexpr int W = NW * KG;
+    constexpr int U = 8;
+    constexpr uint32_t KC = 32 * U;
+    constexpr int KJ = kNormGemmK / 512;
+    constexpr bool GLU = MODE == 3;
+    static_assert(!GLU || NW % 2 == 0, "gate and up tiles");
+    __shared__ __align__(1024) uint8_t xs[2 * kNormGemmRows * kNormGemmK];
+    __shared__ floatx4 part[W][64];
+
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t nw = wave % NW, grp = wave / NW;
+    const uint32_t r = lane & 15, kg = lane >> 4;
+    const uint32_t half = GLU ? n / 2 : n;  // outputs
+    const uint32_t n0 = (GLU ? blockIdx.x * (NW / 2) + nw / 2 : blockIdx.x * NW + nw) * 16;
+    const uint32_t nr = min(n0, half - 16) + (GLU ? nw % 2 * half : 0);
+    const uint32_t kslice = k / KG, k0 = grp * kslice, nch = kslice / KC;
+    const uint32_t upr = k / 8;  // 16-byte units of a row
+    const uint32_t rot = blockIdx.x % nch;
+    auto chunk_at = [&](uint32_t c) {  // c < nch
+        c += rot;
+        return c >= nch ? c - nch : c;
+    };
+    const uint16_t *wp = w + static_cast<uint64_t>(nr + r) * k + k0 + 8 * kg;
+    auto load_w = [&](u32x4 (&a)[U], uint32_t c) __attribute__((always_inline)) {
+        const uint16_t *p = wp + chunk_at(c) * KC;
+#pragma unroll
+        for (int u = 0; u < U; ++u) a[u] = *reinterpret_cast<const u32x4 *>(p + 32 * u);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // A lane's columns of a row: 8 from 512 j + 8 lane on (k % 512 == 0; past k
+    // the row's last 8, not used).
+    floatx4 v[2 * KJ];
+    u32x4 g[KJ];
+    auto load_row = [&](uint32_t row) __attribute__((always_inline)) {
+        const float *p = x + static_cast<uint64_t>(row) * k;
+#pragma unroll
+        for (int j = 0; j < KJ; ++j) {
+            const uint32_t c = min(512 * j + 8 * lane, k - 8);
+            v[2 * j] = *reinterpret_cast<const floatx4 *>(p + c);
+            v[2 * j + 1] = *reinterpret_cast<const floatx4 *>(p + c + 4);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    load_row(min(wave, rows - 1));
+#pragma unroll
+    for (int j = 0; j < KJ; ++j)
+        g[j] = *reinterpret_cast<const u32x4 *>(norm + min(512 * j + 8 * lane, k - 8));
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 a0[U], a1[U];
+    load_w(a0, 0);
+    for (uint32_t row = wave; row < rows; row += W) {
+        if (row != wave) load_row(row);
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < KJ; ++j)
+            if (512 * j < k) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    ss += v[2 * j][e] * v[2 * j][e] + v[2 * j + 1][e] * v[2 * j + 1][e];
+            }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+        const float inv_rms = 1.0f / sqrtf(ss / static_cast<float>(k) + eps);
+#pragma unroll
+        for (int j = 0; j < KJ; ++j)
+            if (512 * j < k) {
+                float wf[8], o[8];
+                unpack8(g[j], wf);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    o[e] = wf[e] * (v[2 * j][e] * inv_rms);
+                    o[4 + e] = wf[4 + e] * (v[2 * j + 1][e] * inv_rms);
+                }
+                *reinterpret_cast<u32x4 *>(xs + (row * upr + ((64 * j + lane) ^ (row & 15))) * 16) =
+                    pack8(o);
+            }
+    }
+    __syncthreads();
+
+    // Columns past the batch repeat its last row and are not stored.
+    const uint32_t xrow = min(r, rows - 1);
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    auto step = [&](u32x4 (&a)[U], u32x4 (&an)[U], uint32_t c) __attribute__((always_inline)) {
+        load_w(an, min(c + 1, nch - 1));
+        const uint32_t u0 = (k0 + chunk_at(c) * KC) / 8 + kg;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bf16x8 b = *reinterpret_cast<const bf16x8 *>(
+                xs + (xrow * upr + ((u0 + 4 * u) ^ (xrow & 15))) * 16);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[u]), b, acc,
+                                                          0, 0, 0);
+        }
+    };
+    for (uint32_t c = 0;;) {
+        step(a0, a1, c);
+        if (++c >= nch) break;
+        step(a1, a0, c);
+        if (++c >= nch) break;
+    }
+
+    // Lane l holds outputs n0 + 4 (l / 16) + e, e = 0..3, of batch row l % 16.
+    part[wave][lane] = acc;
+    __syncthreads();
+    constexpr uint32_t NT = GLU ? NW / 2 : NW;
+    if (wave >= NT) return;
+    auto total = [&](uint32_t t) __attribute__((always_inline)) {
+        floatx4 sum = part[t][lane];
+#pragma unroll
+        for (int q = 1; q < KG; ++q) sum += part[q * NW + t][lane];
+        return sum;
+    };
+    const uint32_t nt = (blockIdx.x * NT + wave) * 16;
+    if (r >= rows || nt >= half) return;
+    const uint64_t o = static_cast<uint64_t>(r) * half + nt + 4 * kg;
+    if constexpr (GLU) store_out4<0>(out, o, swiglu4(total(2 * wave), total(2 * wave + 1)));
+    else store_out4<0>(out, o, total(wave));
+}
+
 template <int MT, int NW, int KG, int KC>
 void launch_stream(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n, uint32_t k,
                    void *out, int mode, hipStream_t stream) {
@@ -882,6 +1022,34 @@ hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t row
 #undef VO_SKINNY
     }
     return launch_stream_any(x, w, rows, n, k, out, mode, stream);
+}
+
+// Up to 8 rows of 2048 values, 4 for a weight of 8192 rows and more, where
+// the product's own time hides less of them (figures at norm_gemm_kernel);
+// longer rows lose: 6144 x 4096, 1 and 4 rows, 19.3 and 20.2 us against 15.4 and
+// 15.8 as two launches, 28672 x 4096 with SwiGLU 46.0 and 45.2 against 46.2
+// and 46.3.
+bool norm_gemm_supported(uint64_t rows, uint64_t n, uint64_t k, bool swiglu) {
+    const uint32_t kg = n >= 8192 ? 1 : swiglu ? 4 : 8;
+    return rows >= 1 && rows <= (n >= 8192 ? 4 : kNormGemmRows) && k >= 512 && k <= kNormGemmK &&
+           k % 512 == 0 && k % (256 * kg) == 0 && n >= 16 && n <= 0x7fffffffull &&
+           n % (swiglu ? 32 : 16) == 0;
+}
+
+hipError_t launch_norm_gemm(const float *x, const uint16_t *norm, float eps, const uint16_t *w,
+                            uint32_t rows, uint32_t n, uint32_t k, bool swiglu, uint16_t *out,
+                            hipStream_t stream) {
+    if (!norm_gemm_supported(rows, n, k, swiglu)) return hipErrorInvalidValue;
+    KernelTimer timer("matmul_norm", stream);
+#define VO_NORM(MODE, NW, KG)                                                                \
+    hipLaunchKernelGGL((norm_gemm_kernel<MODE, NW, KG>), dim3((n + 16 * NW - 1) / (16 * NW)), \
+                       dim3(64 * NW * KG), 0, stream, x, norm, eps, w, rows, n, k, out)
+    if (swiglu && n >= 8192) VO_NORM(3, 4, 1);
+    else if (swiglu) VO_NORM(3, 2, 4);
+    else if (n >= 8192) VO_NORM(0, 4, 1);
+    else VO_NORM(0, 1, 8);
+#undef VO_NORM
+    return hipGetLastError();
 }
 
 hipError_t launch_swiglu_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t ffn,

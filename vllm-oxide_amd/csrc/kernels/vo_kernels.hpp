@@ -148,6 +148,12 @@ hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t row
 // out [rows, ffn] = silu(x . gate^T) * (x . up^T).
 hipError_t launch_swiglu_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t ffn,
                               uint32_t k, uint16_t *out, hipStream_t stream);
+// RMSNorm of x [rows, k] f32 by norm, then the product with w [n, k], out bf16
+// [rows, n], or with SwiGLU [rows, n / 2]: one launch for few rows.
+bool norm_gemm_supported(uint64_t rows, uint64_t n, uint64_t k, bool swiglu);
+hipError_t launch_norm_gemm(const float *x, const uint16_t *norm, float eps, const uint16_t *w,
+                            uint32_t rows, uint32_t n, uint32_t k, bool swiglu, uint16_t *out,
+                            hipStream_t stream);
 hipError_t launch_matmul_generic(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
                                  uint32_t k, void *out, bool out_f32, bool accumulate,
                                  hipStream_t stream);

@@ -376,3 +376,36 @@ extern "C" int32_t vo_matmul_silu_mul(vo_gemm *g, const void *x, uint64_t rows, 
     return vo_silu_mul(gate_up, 2 * ffn, static_cast<const uint16_t *>(gate_up) + ffn, 2 * ffn,
                        rows, ffn, out, ffn, stream);
 }
+
+extern "C" int32_t vo_rmsnorm_matmul(vo_gemm *g, const float *x, uint64_t rows, uint64_t cols,
+                                     const void *norm, float eps, const void *weight,
+                                     uint64_t out_features, int32_t silu_mul, void *normed,
+                                     void *gate_up, void *out, void *stream) {
+    const char *op = "rmsnorm_matmul";
+    if (!g) return fail_argument(op, "null gemm");
+    if (silu_mul != 0 && silu_mul != 1) return fail_argument(op, "silu_mul must be 0 or 1");
+    if (silu_mul && out_features % 2)
+        return fail_shape(op, "an odd number of gate and up rows, " + std::to_string(out_features));
+    // The decode-sized batches of whole tiles: one launch, nothing in normed or
+    // gate_up.  Every other form, and every argument the steps refuse, goes to
+    // them.
+    const uint64_t outputs = silu_mul ? out_features / 2 : out_features;
+    if (skinny_on() && x && norm && weight && out &&
+        kernels::norm_gemm_supported(rows, out_features, cols, silu_mul != 0) && aligned16(x) &&
+        aligned16(norm) && aligned16(weight) && aligned16(out) &&
+        !overlaps(out, rows * outputs * 2, x, rows * cols * 4) &&
+        !overlaps(out, rows * outputs * 2, norm, cols * 2) &&
+        !overlaps(out, rows * outputs * 2, weight, out_features * cols * 2)) {
+        DeviceGuard guard(g->device);
+        return device_status(op, kernels::launch_norm_gemm(
+                                     x, static_cast<const uint16_t *>(norm), eps,
+                                     static_cast<const uint16_t *>(weight),
+                                     static_cast<uint32_t>(rows), static_cast<uint32_t>(out_features),
+                                     static_cast<uint32_t>(cols), silu_mul != 0,
+                                     static_cast<uint16_t *>(out), static_cast<hipStream_t>(stream)));
+    }
+    if (int32_t rc = vo_rmsnorm(x, rows, cols, norm, cols, eps, normed, stream)) return rc;
+    if (silu_mul)
+        return vo_matmul_silu_mul(g, normed, rows, cols, weight, outputs, cols, gate_up, out, stream);
+    return vo_matmul(g, normed, rows, cols, weight, out_features, cols, out, VO_DTYPE_BF16, 0, stream);
+}

@@ -36,7 +36,7 @@ from typing import List, Optional, Sequence
 
 import numpy as np
 
-from . import (VO_DTYPE_BF16, VO_DTYPE_F32, CapacityError, DecodeMeta, HipBackend, KvLayout,
+from . import (VO_DTYPE_F32, CapacityError, DecodeMeta, HipBackend, KvLayout,
                KvPool, PrefillMeta, RopeTable, ShapeError, _check, _engine_error, _stream_ptr,
                _vp, lib, VO_ERR_CAPACITY, VO_ERR_SHAPE)
 
@@ -205,13 +205,13 @@ class Llama:
                                   _ptr(B.attn))
         gu, act = _ptr(B.gu), _ptr(B.act)
         g = B.gemm
-        bf, f32 = VO_DTYPE_BF16, VO_DTYPE_F32
+        f32 = VO_DTYPE_F32
         fused = pool.layout.block_size == 16 and hd in (64, 128)
         attention = lib.vo_prefill_attention if prefill else lib.vo_decode_attention
         _check(lib.vo_embed(_ptr(self.embed), V, H, mh, T, res, s))
         for li, L in enumerate(self.layers):
-            _check(lib.vo_rmsnorm(res, T, H, _ptr(L["attn_norm"]), H, eps, nrm, s))
-            _check(lib.vo_matmul(g, nrm, T, H, _ptr(L["wqkv"]), qd + 2 * kvd, H, qkv, bf, 0, s))
+            _check(lib.vo_rmsnorm_matmul(g, res, T, H, _ptr(L["attn_norm"]), eps, _ptr(L["wqkv"]),
+                                         qd + 2 * kvd, 0, nrm, None, qkv, s))
             if fused:
                 _check(lib.vo_qkv_rope_write_kv(pool.handle, li, self.rope.handle, qkv, T, qd,
                                                 kvd, mh, q, s))
@@ -219,8 +219,8 @@ class Llama:
                 self._rope_write_unfused(pool, li, T, m, stream, B)
             _check(attention(q, T, qd, pool.handle, li, mh, attn, s))
             _check(lib.vo_matmul(g, attn, T, qd, _ptr(L["wo"]), H, qd, res, f32, 1, s))
-            _check(lib.vo_rmsnorm(res, T, H, _ptr(L["mlp_norm"]), H, eps, nrm, s))
-            _check(lib.vo_matmul_silu_mul(g, nrm, T, H, _ptr(L["wgu"]), F, H, gu, act, s))
+            _check(lib.vo_rmsnorm_matmul(g, res, T, H, _ptr(L["mlp_norm"]), eps, _ptr(L["wgu"]),
+                                         2 * F, 1, nrm, gu, act, s))
             _check(lib.vo_matmul(g, act, T, F, _ptr(L["wd"]), H, F, res, f32, 1, s))
         _check(lib.vo_rmsnorm_last_rows(res, T, H, _ptr(self.final_norm), H, eps, mh,
                                         _ptr(B.last), s))
