@@ -718,6 +718,16 @@ int32_t vo_rmsnorm_matmul(vo_gemm *gemm, const float *x, uint64_t rows, uint64_t
                           const void *norm, float eps, const void *weight, uint64_t out_features,
                           int32_t silu_mul, void *normed, void *gate_up, void *out, void *stream);
 
+/* vo_rmsnorm_matmul of x by a layer's fused [wq; wk; wv] weight (q_cols + 2 *
+ * kv_cols rows) into qkv, then vo_qkv_rope_write_kv of it.  normed is room for
+ * [rows, cols] bf16, qkv for the product; the few rows of a decode step run as
+ * one launch, rounded in between as the steps are, and leave both alone. */
+int32_t vo_rmsnorm_qkv_rope_write_kv(vo_gemm *gemm, const float *x, uint64_t rows, uint64_t cols,
+                                     const void *norm, float eps, const void *weight,
+                                     vo_kv_pool *pool, uint64_t layer, const vo_rope_table *table,
+                                     uint64_t q_cols, uint64_t kv_cols, const vo_step_meta *meta,
+                                     void *normed, void *qkv, void *q_out, void *stream);
+
 /* ------------------------------------------------------------------ */
 /* Opt-in kernel timing (the reference's opt-in per-op timing,         */
 /* arena.rs:82-87 OpStat, :129-136 enable_profiling)                   */

@@ -19,6 +19,7 @@ tolerance written in each test; greedy ids agree wherever the oracle's top-1
 reference's HF check, tests/hf_match.rs).
 """
 import ctypes
+import dataclasses
 import math
 
 import numpy as np
@@ -212,6 +213,67 @@ def test_rmsnorm_matmul_shapes(vo, gpu_backend, rows, k, n, swiglu):
         one = torch.empty((1, outputs), dtype=torch.bfloat16, device="cuda:0")
         run(x[-1:].contiguous(), one)
         assert torch.equal(one[0], out[-1])
+
+
+@pytest.mark.parametrize("hd,heads,kvh,k", [(64, 4, 2, 2048), (128, 8, 2, 2048), (64, 32, 8, 2048),
+                                            (128, 56, 8, 512), (64, 4, 2, 1024)])
+@pytest.mark.parametrize("rows", [1, 3, 4, 8, 9])
+def test_rmsnorm_qkv_rope_write_kv_matches_steps(vo, gpu_backend, hd, heads, kvh, k, rows):
+    """RoPE and the cache write inside the QKV product, both workgroup shapes
+    and sizes that run as the steps, against the two calls: q and the cached
+    rows, a row whose slot a later row takes again among them.  Bitwise below
+    8192 outputs.  From there a workgroup starts its walk over K at a chunk
+    that depends on its index, and an output sits in another workgroup than in
+    the plain product: its f32 sum takes another order and may round to the
+    next bf16, 2^-7 of it away.  A pair (a, b) of norm p is then rotated from
+    values up to 2^-7 |a|, 2^-7 |b| off, so by up to 2^-7 p, and rounded again
+    (2^-7 of the result, at most p): 2^-6 p, V 2^-7 |v|."""
+    import torch
+    _say(f"rmsnorm_qkv_rope_write_kv {rows}x{k} hd={hd} heads={heads}/{kvh}")
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows + hd + k)
+    qd, kvd = heads * hd, kvh * hd
+    n = qd + 2 * kvd
+    x = 3.0 * torch.randn((rows, k), generator=gen, device="cuda:0")
+    norm = (1 + 0.2 * torch.randn((k,), generator=gen, device="cuda:0")).to(torch.bfloat16)
+    w = (0.05 * torch.randn((n, k), generator=gen, device="cuda:0")).to(torch.bfloat16)
+    table = vo.RopeTable(hd, 500000.0, 600)
+    pool = gpu_backend.alloc_kv_pool(vo.KvLayout(2, 80, 16, kvh, hd))
+    meta = vo.DecodeMeta.new([vo.DecodeSeq(37 * i + 3, list(range(40 + i - (37 * i + 3) // 16, 41 + i)))
+                              for i in range(rows)], 16)
+    if rows > 2:
+        slots = list(meta.slot_mapping)
+        slots[1] = slots[2]
+        meta = dataclasses.replace(meta, slot_mapping=slots)
+    m = gpu_backend.step_meta(pool)
+    m.upload(meta)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    bf = lambda *shape: torch.full(shape, 7.0, dtype=torch.bfloat16, device="cuda:0")  # noqa: E731
+    normed, qkv, q0, q1 = bf(rows, k), bf(rows, n), bf(rows, qd), bf(rows, qd)
+    g, s = gpu_backend.gemm().handle, vo._stream_ptr(None)
+    vo._check(vo.lib.vo_rmsnorm_matmul(g, P(x), rows, k, P(norm), 1e-5, P(w), n, 0, P(normed), None,
+                                       P(qkv), s))
+    vo._check(vo.lib.vo_qkv_rope_write_kv(pool.handle, 0, table.handle, P(qkv), rows, qd, kvd, m.handle,
+                                          P(q0), s))
+    vo._check(vo.lib.vo_rmsnorm_qkv_rope_write_kv(g, P(x), rows, k, P(norm), 1e-5, P(w), pool.handle, 1,
+                                                  table.handle, qd, kvd, m.handle, P(normed), P(qkv),
+                                                  P(q1), s))
+    torch.cuda.synchronize()
+
+    def same(a, b, rotated):
+        if n < 8192:
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+            return
+        a, b = a.double().reshape(-1, 2, hd // 2), b.double().reshape(-1, 2, hd // 2)
+        bound = 2 ** -6 * a.norm(dim=1, keepdim=True) if rotated else 2 ** -7 * a.abs()
+        assert ((a - b).abs() <= 1.01 * bound).all()
+
+    same(q0, q1, True)
+    everything = vo.DecodeMeta.new([vo.DecodeSeq(80 * 16 - 1, list(range(80)))], 16)
+    for a, b, rotated in zip(gpu_backend.read_kv(pool, 0, everything, 0, 80 * 16),
+                             gpu_backend.read_kv(pool, 1, everything, 0, 80 * 16), (True, False)):
+        same(a, b, rotated)
+        assert bool((a != 0).any())
 
 
 @pytest.mark.parametrize("rows", [1, 5, 8, 9])

@@ -185,6 +185,9 @@ SIGNATURES = {
     "vo_matmul_silu_mul": (ctypes.c_int32, [_vp, _vp, _u64, _u64, _vp, _u64, _u64, _vp, _vp, _vp]),
     "vo_rmsnorm_matmul": (ctypes.c_int32, [_vp, _vp, _u64, _u64, _vp, ctypes.c_float, _vp, _u64,
                                            ctypes.c_int32, _vp, _vp, _vp, _vp]),
+    "vo_rmsnorm_qkv_rope_write_kv": (ctypes.c_int32, [_vp, _vp, _u64, _u64, _vp, ctypes.c_float, _vp,
+                                                      _vp, _u64, _vp, _u64, _u64, _vp, _vp, _vp,
+                                                      _vp, _vp]),
     "vo_workspace_create": (ctypes.c_int32, [ctypes.c_int32, _u64, ctypes.POINTER(_vp)]),
     "vo_workspace_destroy": (None, [_vp]),
     "vo_workspace_elems": (_u64, [_vp]),

@@ -43,23 +43,6 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
            (static_cast<uint32_t>(f32_to_bf16_bits(b)) << 16);
 }
 
-// x1' (first half) and x2' (second half) of rope.rs:95-96.  HIP compiles
-// with contraction on, which would fuse a product into the following add
-// (an FMA rounds once where the reference rounds twice); the pragma keeps
-// each product and sum rounded on its own.
-__device__ __forceinline__ float rot_first(float a, float b, float c, float s) {
-#pragma clang fp contract(off)
-    const float ac = a * c;
-    const float bs = b * s;
-    return ac - bs;
-}
-__device__ __forceinline__ float rot_second(float a, float b, float c, float s) {
-#pragma clang fp contract(off)
-    const float bc = b * c;
-    const float as = a * s;
-    return bc + as;
-}
-
 // 8 pairs: x1 = a (8 bf16), x2 = b (8 bf16) -> rotated in place.
 __device__ __forceinline__ void rotate8(u32x4 &a, u32x4 &b, const float *c, const float *s) {
 #pragma unroll

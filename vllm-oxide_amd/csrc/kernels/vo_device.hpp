@@ -40,6 +40,23 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
     return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 
+// x1' (first half) and x2' (second half) of rope.rs:95-96.  HIP compiles
+// with contraction on, which would fuse a product into the following add
+// (an FMA rounds once where the reference rounds twice); the pragma keeps
+// each product and sum rounded on its own.
+__device__ __forceinline__ float rot_first(float a, float b, float c, float s) {
+#pragma clang fp contract(off)
+    const float ac = a * c;
+    const float bs = b * s;
+    return ac - bs;
+}
+__device__ __forceinline__ float rot_second(float a, float b, float c, float s) {
+#pragma clang fp contract(off)
+    const float bc = b * c;
+    const float as = a * s;
+    return bc + as;
+}
+
 struct PoolDims {
     uint32_t kv_heads;
     uint32_t head_dim;

@@ -154,6 +154,18 @@ bool norm_gemm_supported(uint64_t rows, uint64_t n, uint64_t k, bool swiglu);
 hipError_t launch_norm_gemm(const float *x, const uint16_t *norm, float eps, const uint16_t *w,
                             uint32_t rows, uint32_t n, uint32_t k, bool swiglu, uint16_t *out,
                             hipStream_t stream);
+// Where the QKV product of a layer goes: the first q_cols outputs of a row,
+// rotated, to q_out [rows, q_cols], the next kv_heads * head_dim, rotated, and
+// the last as many to the row's slot of the pool (slot kSkipSlot: nowhere).
+struct QkvRope {
+    uint16_t *k_pool, *v_pool, *q_out;
+    uint32_t kv_heads, head_dim, q_cols;  // head_dim 64 or 128, blocks of 16 tokens
+    const uint32_t *positions, *slots;
+    const float *cos_tab, *sin_tab;  // [position][head_dim / 2]
+};
+// launch_norm_gemm of a layer's [wq; wk; wv], with RoPE and the cache write.
+hipError_t launch_norm_qkv_rope(const float *x, const uint16_t *norm, float eps, const uint16_t *w,
+                                uint32_t rows, uint32_t k, const QkvRope &to, hipStream_t stream);
 hipError_t launch_matmul_generic(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
                                  uint32_t k, void *out, bool out_f32, bool accumulate,
                                  hipStream_t stream);

@@ -1010,8 +1010,6 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
         err = hipMalloc(reinterpret_cast<void **>(&m->d_arrivals),
                         max_rows * m->kv_heads * sizeof(uint32_t));
     if (err == hipSuccess)
-        err = hipMemset(m->d_arrivals, 0, max_rows * m->kv_heads * sizeof(uint32_t));
-    if (err == hipSuccess)
         err = hipMalloc(reinterpret_cast<void **>(&m->d_tokens), max_rows * sizeof(uint32_t));
     if (err == hipSuccess) err = m->tokens_stage.create(max_rows * sizeof(uint32_t));
     if (err == hipSuccess)
@@ -1021,6 +1019,10 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
     if (err == hipSuccess) err = m->aux_stage.create(max_rows * sizeof(uint32_t));
     // Default priority, like every stream here.
     if (err == hipSuccess) err = hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking);
+    // On a stream of its own, as the null stream's work may be under capture.
+    if (err == hipSuccess)
+        err = hipMemsetAsync(m->d_arrivals, 0, max_rows * m->kv_heads * sizeof(uint32_t), m->side);
+    if (err == hipSuccess) err = hipStreamSynchronize(m->side);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&m->fork, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&m->join, hipEventDisableTiming);
     if (err != hipSuccess) {
@@ -1716,6 +1718,50 @@ extern "C" int32_t vo_qkv_rope_write_kv(vo_kv_pool *pool, uint64_t layer, const 
         static_cast<uint32_t>(ld), m->write_plan, m->view.positions, t->d_cos, t->d_sin,
         static_cast<hipStream_t>(stream));
     return device_status(op, err);
+}
+
+extern "C" int32_t vo_rmsnorm_qkv_rope_write_kv(vo_gemm *g, const float *x, uint64_t rows,
+                                                uint64_t cols, const void *norm, float eps,
+                                                const void *weight, vo_kv_pool *pool,
+                                                uint64_t layer, const vo_rope_table *t,
+                                                uint64_t q_cols, uint64_t kv_cols,
+                                                const vo_step_meta *m, void *normed, void *qkv,
+                                                void *q_out, void *stream) {
+    const char *op = "rmsnorm_qkv_rope_write_kv";
+    if (!g || !pool || !t || !m) return fail_argument(op, "null gemm, pool, table or meta");
+    const vo_kv_layout &L = pool->layout;
+    if (q_cols > kU32Limit || kv_cols > kU32Limit || q_cols + 2 * kv_cols > kU32Limit)
+        return fail_capacity("qkv columns (u32)", std::max(q_cols, kv_cols), kU32Limit);
+    // The few rows of a decode step: one launch, nothing in normed or qkv.
+    // Every other form, and every argument the steps refuse, goes to them.
+    const uint64_t n = q_cols + 2 * kv_cols;
+    if (skinny_on() && x && norm && weight && qkv && q_out &&
+        kernels::norm_gemm_supported(rows, n, cols, false) &&
+        kernels::cache_write_supported(static_cast<uint32_t>(L.head_dim),
+                                       static_cast<uint32_t>(L.block_size)) &&
+        q_cols != 0 && q_cols % (L.kv_heads * L.head_dim) == 0 && aligned16(x) &&
+        aligned16(norm) && aligned16(weight) && aligned16(qkv) && aligned16(q_out) &&
+        !overlaps(q_out, rows * q_cols * 2, x, rows * cols * 4) &&
+        !overlaps(q_out, rows * q_cols * 2, norm, cols * 2) &&
+        !overlaps(q_out, rows * q_cols * 2, weight, n * cols * 2) &&
+        !overlaps(q_out, rows * q_cols * 2, qkv, rows * n * 2) &&
+        check_rope("rope", t, rows, q_cols, L.head_dim, m) == VO_OK &&
+        check_write(pool, layer, rows, kv_cols, m) == VO_OK) {
+        DeviceGuard guard(pool->device);
+        const kernels::PoolLayer at = pool->layer(layer);
+        const kernels::QkvRope to{at.k, at.v, static_cast<uint16_t *>(q_out), at.kv_heads,
+                                  at.head_dim, static_cast<uint32_t>(q_cols), m->view.positions,
+                                  m->d_write_slots, t->d_cos, t->d_sin};
+        return device_status(op, kernels::launch_norm_qkv_rope(
+                                     x, static_cast<const uint16_t *>(norm), eps,
+                                     static_cast<const uint16_t *>(weight),
+                                     static_cast<uint32_t>(rows), static_cast<uint32_t>(cols), to,
+                                     static_cast<hipStream_t>(stream)));
+    }
+    if (int32_t rc = vo_rmsnorm_matmul(g, x, rows, cols, norm, eps, weight, n, 0, normed, nullptr,
+                                       qkv, stream))
+        return rc;
+    return vo_qkv_rope_write_kv(pool, layer, t, qkv, rows, q_cols, kv_cols, m, q_out, stream);
 }
 
 extern "C" int32_t vo_prefill_attention(const void *queries, uint64_t rows, uint64_t cols,

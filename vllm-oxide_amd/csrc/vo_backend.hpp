@@ -293,6 +293,10 @@ namespace vo {
 vo_status aux_upload(vo_step_meta *m, std::vector<uint32_t> &held, bool &valid, uint32_t *dev,
                      const uint32_t *values, uint64_t n, hipStream_t stream, const char *op);
 
+// Whether decode-sized products run on the weight-streaming kernels
+// (VO_SKINNY_GEMM=0: off).
+bool skinny_on();
+
 }  // namespace vo
 
 struct vo_rope_table {

@@ -226,13 +226,16 @@ vo_status make_plan(vo_gemm *g, const LtApi &api, uint64_t rows, uint64_t n, uin
     return VO_OK;
 }
 
-// Decode-sized batches: the weight-streaming kernel (VO_SKINNY_GEMM=0: off).
+}  // namespace
+
+namespace vo {
+
 bool skinny_on() {
     static const bool on = env_int("VO_SKINNY_GEMM", 1) != 0;
     return on;
 }
 
-}  // namespace
+}  // namespace vo
 
 extern "C" int32_t vo_gemm_create(int32_t device, uint64_t workspace_bytes, vo_gemm **out) {
     const char *op = "matmul";

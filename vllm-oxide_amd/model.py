@@ -210,12 +210,13 @@ class Llama:
         attention = lib.vo_prefill_attention if prefill else lib.vo_decode_attention
         _check(lib.vo_embed(_ptr(self.embed), V, H, mh, T, res, s))
         for li, L in enumerate(self.layers):
-            _check(lib.vo_rmsnorm_matmul(g, res, T, H, _ptr(L["attn_norm"]), eps, _ptr(L["wqkv"]),
-                                         qd + 2 * kvd, 0, nrm, None, qkv, s))
             if fused:
-                _check(lib.vo_qkv_rope_write_kv(pool.handle, li, self.rope.handle, qkv, T, qd,
-                                                kvd, mh, q, s))
+                _check(lib.vo_rmsnorm_qkv_rope_write_kv(
+                    g, res, T, H, _ptr(L["attn_norm"]), eps, _ptr(L["wqkv"]), pool.handle, li,
+                    self.rope.handle, qd, kvd, mh, nrm, qkv, q, s))
             else:
+                _check(lib.vo_rmsnorm_matmul(g, res, T, H, _ptr(L["attn_norm"]), eps,
+                                             _ptr(L["wqkv"]), qd + 2 * kvd, 0, nrm, None, qkv, s))
                 self._rope_write_unfused(pool, li, T, m, stream, B)
             _check(attention(q, T, qd, pool.handle, li, mh, attn, s))
             _check(lib.vo_matmul(g, attn, T, qd, _ptr(L["wo"]), H, qd, res, f32, 1, s))
