@@ -41,13 +41,15 @@
 // and 13.8 as 220 fine ones, of a 53 MB read; one row of 8000 keys 27 and
 // 13.8 us a call.
 //
-// The merge.  In a plan without packs the last workgroup of a row (and KV
-// head) to finish merges the row's partials: they are written and read with
+// The merge.  The last workgroup of a row (and KV head) to finish merges the
+// row's partials: they are written and read with
 // agent-scope accesses and counted with a relaxed atomic, and no reduce
 // launch follows (3 us of GPU time, and 2.5 us of the host's in a small
-// call: 13.8 -> 11.1 us for one row of 8000 keys of 64 dims).  (A release and an acquire fence
+// call: 13.8 -> 11.1 us for one row of 8000 keys of 64 dims; with shared packs,
+// whose workgroups count for each of their rows, 64 rows behind a 4096-key
+// prefix and one of 32768 keys 73.5 -> 72.7 us).  (A release and an acquire fence
 // per workgroup instead are an L2 writeback and invalidate each time, which
-// measured 5-9x slower than the separate launch.)  Plans with packs and
+// measured 5-9x slower than the separate launch.)  Packs of one tile and
 // fixed launches keep the reduce kernel.
 // Workgroups are numbered KV head fastest, so the KV heads of one block are
 // read at about the same time.
@@ -317,6 +319,29 @@ __device__ __forceinline__ void fold_state(float &mf, float &lf, floatx4 (&accf)
         for (int j = 0; j < 4; ++j) accf[dt][j] = __builtin_fmaf(accf[dt][j], ef, acc[dt][j] * e);
 }
 
+// Split-K partials of a row are merged by the reduce kernel, or by the
+// last workgroup of the row's items to finish (`arrivals`; see decode_splitk_kernel).
+// In the second form they cross workgroups inside a launch, so they are
+// written and read with agent-scope (device-coherent) accesses.
+__device__ __forceinline__ void put_f32(float *p, float v, bool agent) {
+    if (agent)
+        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else
+        *p = v;
+}
+
+__device__ __forceinline__ void put_f32x4(float *p, floatx4 v, bool agent) {
+    if (agent) {
+        typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
+        const u64x2 w = __builtin_bit_cast(u64x2, v);
+        uint64_t *d = reinterpret_cast<uint64_t *>(p);
+        __hip_atomic_store(d, static_cast<uint64_t>(w[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(d + 1, static_cast<uint64_t>(w[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+        *reinterpret_cast<floatx4 *>(p) = v;
+    }
+}
+
 // One state's run in progress (m, l, acc) and the merge of the runs before
 // it.  `flush` ends a run; `finish` leaves the state in (m, l, acc).  With a
 // wavefront's LDS given to flush and finish (room for DT * 64 floatx4), the
@@ -434,7 +459,7 @@ __device__ __forceinline__ void shared_split(
     uint16_t *__restrict__ out, float *__restrict__ part_acc, float *__restrict__ part_ml,
     uint32_t num_heads, uint32_t group, float scale_log2, const uint32_t *__restrict__ mates,
     uint32_t pack, uint8_t *__restrict__ st0, uint8_t *__restrict__ st1,
-    uint8_t *__restrict__ st2, uint8_t *__restrict__ st3) {
+    uint8_t *__restrict__ st2, uint8_t *__restrict__ st3, bool agent) {
 #pragma clang fp contract(off)  // the merge below rounds as the register path's does
     constexpr int KK = HD / 32;
     constexpr int DT = HD / 16;
@@ -649,10 +674,10 @@ __device__ __forceinline__ void shared_split(
         const uint64_t part = static_cast<uint64_t>(cinfo[0] + split) * num_heads + qhead;
         float *ap = part_acc + part * HD + 4 * g;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<floatx4 *>(ap + 16 * dt) = num[dt];
+        for (int dt = 0; dt < DT; ++dt) put_f32x4(ap + 16 * dt, num[dt], agent);
         if (g == 0) {
-            part_ml[2 * part] = mx;
-            part_ml[2 * part + 1] = den;
+            put_f32(part_ml + 2 * part, mx, agent);
+            put_f32(part_ml + 2 * part + 1, den, agent);
         }
     }
 }
@@ -678,7 +703,7 @@ __device__ __forceinline__ void shared_split_pairs(
     uint16_t *__restrict__ out, float *__restrict__ part_acc, float *__restrict__ part_ml,
     uint32_t num_heads, uint32_t group, float scale_log2, const uint32_t *__restrict__ mates,
     uint32_t pack, uint8_t *__restrict__ st0, uint8_t *__restrict__ st1,
-    uint8_t *__restrict__ st2, uint8_t *__restrict__ st3) {
+    uint8_t *__restrict__ st2, uint8_t *__restrict__ st3, bool agent) {
 #pragma clang fp contract(off)  // the merge below rounds as the register path's does
     constexpr int KK = HD / 32;
     constexpr int DT = HD / 16;
@@ -929,34 +954,11 @@ __device__ __forceinline__ void shared_split_pairs(
         const uint64_t part = static_cast<uint64_t>(cinfo[0] + split) * num_heads + qhead;
         float *ap = part_acc + part * HD + 4 * g;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<floatx4 *>(ap + 16 * dt) = num[dt];
+        for (int dt = 0; dt < DT; ++dt) put_f32x4(ap + 16 * dt, num[dt], agent);
         if (g == 0) {
-            part_ml[2 * part] = mx;
-            part_ml[2 * part + 1] = den;
+            put_f32(part_ml + 2 * part, mx, agent);
+            put_f32(part_ml + 2 * part + 1, den, agent);
         }
-    }
-}
-
-// Split-K partials of a row are merged by the reduce kernel, or by the
-// last workgroup of the row's items to finish (`arrivals`; see decode_splitk_kernel).
-// In the second form they cross workgroups inside a launch, so they are
-// written and read with agent-scope (device-coherent) accesses.
-__device__ __forceinline__ void put_f32(float *p, float v, bool agent) {
-    if (agent)
-        __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    else
-        *p = v;
-}
-
-__device__ __forceinline__ void put_f32x4(float *p, floatx4 v, bool agent) {
-    if (agent) {
-        typedef uint64_t u64x2 __attribute__((ext_vector_type(2)));
-        const u64x2 w = __builtin_bit_cast(u64x2, v);
-        uint64_t *d = reinterpret_cast<uint64_t *>(p);
-        __hip_atomic_store(d, static_cast<uint64_t>(w[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(d + 1, static_cast<uint64_t>(w[1]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else {
-        *reinterpret_cast<floatx4 *>(p) = v;
     }
 }
 
@@ -1090,8 +1092,8 @@ __device__ __forceinline__ void merge_row(const float *part_acc, const float *pa
     *reinterpret_cast<u32x2 *>(out + d) = packed;
 }
 
-// The kernels of a launch: one without packs (single rows, fine items, the
-// in-launch merge) and one for each form of shared packs beside single rows,
+// The kernels of a launch: one without packs (single rows, fine items)
+// and one for each form of shared packs beside single rows,
 // so that neither carries the other's code, which would not fit half the
 // instruction cache (22 and 33 KB at head_dim 128; all in one 50 KB, and the
 // 64-row decode step 0.9% longer).
@@ -1127,7 +1129,7 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     __shared__ __align__(1024) uint8_t sh2[kStageBytes];
     __shared__ __align__(1024) uint8_t sh3[kStageBytes];
     __shared__ float s_ml[kStages ? 2 * W * 16 : 1];
-    __shared__ uint32_t s_last;
+    __shared__ uint32_t s_last[PACKS == kNoPacks ? 1 : 64];  // who merges (arrivals)
     static_assert(!kStages || 16 * kAccStride<HD> * 4 <= kStageBytes, "merge fits a stage");
 
     const uint32_t item = blockIdx.x / kv_heads;
@@ -1150,17 +1152,62 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
             out[out_base + static_cast<uint64_t>(kvh) * group * HD + idx] = 0;
         return;
     }
+    // Each partial was written with agent-scope stores: waits until this
+    // wavefront's are done, and for the workgroup's other wavefronts.
+    auto stored = []() __attribute__((always_inline)) {
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0)
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __syncthreads();
+    };
+    // Counts one of row r's `expected` items for this KV head.  True for the
+    // last, which leaves the counter at zero for the next launch.
+    auto count_item = [&](uint32_t r, uint32_t expected) {
+        uint32_t *const count = arrivals + static_cast<uint64_t>(r) * kv_heads + kvh;
+        const uint32_t before =
+            __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const bool last = before + 1 == expected;
+        if (last) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return last;
+    };
+    // This workgroup's merge of row r for its KV head's query heads.
+    auto merge = [&](uint32_t r, uint32_t first, uint32_t nsplit, bool fine_row) {
+        constexpr uint32_t NQ = HD / 4;
+        for (uint32_t i = threadIdx.x; i < group * NQ; i += 64 * W) {
+            const uint32_t qh = kvh * group + i / NQ;
+            merge_row<HD, true>(part_acc, part_ml, first, nsplit, fine_row, nk, split_keys, num_heads,
+                                qh, 4 * (i % NQ), out + (static_cast<uint64_t>(r) * num_heads + qh) * HD);
+        }
+    };
+    // The end of a shared pack, when the rows' last workgroups merge: one lane
+    // counts the item for each of the pack's rows (at most 64).
+    auto arrive_pack = [&]() {
+        stored();
+        if (threadIdx.x < pack) {
+            const uint32_t r = threadIdx.x == 0 ? row : mates[(pack - 1) * item + threadIdx.x - 1];
+            const uint32_t nsplit = r == kNoMate ? 1u : row_info[2 * static_cast<uint64_t>(r) + 1];
+            s_last[threadIdx.x] = nsplit > 1 && count_item(r, nsplit) ? r : kNoMate;
+        }
+        __syncthreads();
+        for (uint32_t j = 0; j < pack; ++j) {
+            const uint32_t r = uniform_u32(s_last[j]);
+            if (r == kNoMate) continue;
+            const u32x2 info = *reinterpret_cast<const u32x2 *>(row_info + 2 * static_cast<uint64_t>(r));
+            merge(r, info[0], info[1], false);
+        }
+    };
     if constexpr (kStages && PACKS != kNoPacks) {
         if (item < num_shared) {
             if constexpr (PACKS == kPairPacks)
                 shared_split_pairs<HD, W>(k_pool, v_pool, kv_heads, kvh, item, rec, tables,
                                           row_info, split_keys, q, out, part_acc, part_ml,
                                           num_heads, group, scale_log2, mates, pack, sh0, sh1,
-                                          sh2, sh3);
+                                          sh2, sh3, arrivals != nullptr);
             else
                 shared_split<HD, W>(k_pool, v_pool, kv_heads, kvh, item, rec, tables, row_info,
                                     split_keys, q, out, part_acc, part_ml, num_heads, group,
-                                    scale_log2, mates, pack, sh0, sh1, sh2, sh3);
+                                    scale_log2, mates, pack, sh0, sh1, sh2, sh3, arrivals != nullptr);
+            if (arrivals) arrive_pack();
             return;
         }
     }
@@ -1227,33 +1274,16 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     if (head_ok) cinfo = *reinterpret_cast<const u32x2 *>(row_info + 2 * static_cast<uint64_t>(crow));
 
     // The end of an item with a partial, when the row's last workgroup merges
-    // (a plan without packs: every column is this row's).  Each partial was
-    // written with agent-scope stores; once this wavefront's are done and the
-    // workgroup has met, one lane counts the item, and the workgroup that
-    // counts the row's last one for this KV head reads the partials back with
-    // agent-scope loads and leaves the counter at zero for the next launch.
+    // (every column is this row's): the workgroup that counts the row's last
+    // item for this KV head reads the partials back with agent-scope loads.
     // (No release or acquire fence: see the top of this file.)
     auto arrive = [&](uint32_t first, uint32_t nsplit, bool fine_row) {
-        __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));  // vmcnt(0): the stores are done
+        stored();
+        if (threadIdx.x == 0)
+            s_last[0] = count_item(row, fine_row ? W * (nk / split_keys) + split_states(nk % split_keys)
+                                                 : nsplit);
         __syncthreads();
-        if (threadIdx.x == 0) {
-            const uint32_t expected = fine_row ? W * (nk / split_keys) + split_states(nk % split_keys)
-                                               : nsplit;
-            uint32_t *const count = arrivals + static_cast<uint64_t>(row) * kv_heads + kvh;
-            const uint32_t before =
-                __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const bool last = before + 1 == expected;
-            if (last) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            s_last = last ? 1u : 0u;
-        }
-        __syncthreads();
-        if (s_last == 0) return;
-        constexpr uint32_t NQ = HD / 4;
-        for (uint32_t i = threadIdx.x; i < group * NQ; i += 64 * W) {
-            const uint32_t qh = kvh * group + i / NQ;
-            merge_row<HD, true>(part_acc, part_ml, first, nsplit, fine_row, nk, split_keys, num_heads,
-                                qh, 4 * (i % NQ), out + out_base + static_cast<uint64_t>(qh) * HD);
-        }
+        if (s_last[0] != 0) merge(row, first, nsplit, fine_row);
     };
 
     // Block ids of chunk cc: wave-uniform, so scalar loads from the table
@@ -1486,14 +1516,14 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
                     f32_to_bf16_bits(num / den);
             } else {
                 const uint64_t part = static_cast<uint64_t>(s_col[1][col] + split) * num_heads + qh;
-                put_f32(part_acc + part * HD + d, num, kFine && arrivals != nullptr);
+                put_f32(part_acc + part * HD + d, num, kStages && arrivals != nullptr);
                 if (d == 0) {
-                    put_f32(part_ml + 2 * part, mx, kFine && arrivals != nullptr);
-                    put_f32(part_ml + 2 * part + 1, den, kFine && arrivals != nullptr);
+                    put_f32(part_ml + 2 * part, mx, kStages && arrivals != nullptr);
+                    put_f32(part_ml + 2 * part + 1, den, kStages && arrivals != nullptr);
                 }
             }
         }
-        if constexpr (kFine)
+        if constexpr (kStages)
             if (arrivals && s_col[2][0] > 1) arrive(s_col[1][0], s_col[2][0], false);
     }
 }
@@ -1501,7 +1531,7 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
 // Merges the split-K partials of the rows listed in reduce_rows (those with
 // more than one split, and those of fine items; rows with one whole split
 // were written by the split kernel), where the row's last workgroup does not:
-// plans with packs and fixed launches.  A wavefront is a workgroup and takes
+// plans with one-tile packs and fixed launches.  A wavefront is a workgroup and takes
 // 64 / (HD / 4) query heads of one row, a thread four dims (with four such to
 // a workgroup 65 rows of 64 heads took 5.8 us instead of 5.5).
 template <int HD>
@@ -1539,7 +1569,7 @@ hipError_t launch_split_kind(const PoolLayer &pool, const MetaView &meta, const 
         return hipErrorInvalidValue;
     const uint32_t item_pack = shared ? 1u : pack;
     static_assert(PACKS == kNoPacks || W == kSharedWaves, "packs need the stages");
-    if (plan.arrivals && (pack != 1 || W != kSharedWaves)) return hipErrorInvalidValue;
+    if (plan.arrivals && (item_pack != 1 || pack > 64 || W != kSharedWaves)) return hipErrorInvalidValue;
     if (item_pack * group > 16 || (pack > 1 && plan.mates == nullptr)) return hipErrorInvalidValue;
     // With 4 wavefronts (not streaming) the merge lives in the shared-pack
     // stages (at most 16 columns of HD floats per wavefront, 8 KiB at

@@ -221,8 +221,9 @@ struct DecodePlan {
     bool shared_pairs;
     // With arrivals, [rows][kv_heads] counters that are zero between
     // launches, the workgroup that finishes a row's last item for a KV head
-    // merges its partials and no reduce kernel runs; only for plans without
-    // packs, on 2 or more wavefronts.  Null: the reduce kernel.
+    // merges its partials and no reduce kernel runs; only for plans whose
+    // packs, if any, are shared ones, on four wavefronts.  Null: the reduce
+    // kernel.
     uint32_t *arrivals;
 };
 

@@ -542,7 +542,7 @@ uint64_t decode_fine_limit(uint64_t num_cus) {
     return env >= 0 ? static_cast<uint64_t>(env) : num_cus * 5 / 8;
 }
 
-// Whether the decode launch merges the partials itself (plans without packs;
+// Whether the decode launch merges the partials itself (plans without one-tile packs;
 // VO_DECODE_ARRIVE=0: the reduce kernel does, a tuning knob).
 bool decode_arrive() { return env_int("VO_DECODE_ARRIVE", 1) != 0; }
 
@@ -703,7 +703,7 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
     m->plan.part_acc = m->d_part_acc;
     m->plan.part_ml = m->d_part_ml;
     m->plan.arrivals = nullptr;
-    if (!pk.fixed() && P == 1 && waves == 4 && decode_arrive()) m->plan.arrivals = m->d_arrivals;
+    if (!pk.fixed() && (P == 1 || m->plan.num_shared != 0) && waves == 4 && decode_arrive()) m->plan.arrivals = m->d_arrivals;
     m->h_counts[0] = static_cast<uint32_t>(num_work);
     m->h_counts[1] = static_cast<uint32_t>(nred);
     m->plan.counts = m->d_counts;
