@@ -57,7 +57,12 @@ __global__ void reshape_and_cache_kernel(uint16_t *__restrict__ k_pool,
 }
 
 // One wavefront per (run of rows with consecutive slots in one block, KV
-// head); four per workgroup.  Needs block size 16 and head_dim 64 or 128.
+// head), a workgroup of its own.  Needs block size 16 and head_dim 64 or 128.
+// Bound: one wavefront's chain (record, loads, stores), so the loads go out
+// together and the wavefronts spread over the CUs.  With a branch around each
+// row's loads and four wavefronts to a workgroup, write_kv and prefill
+// attention of 8 x 512 rows (8 KV heads of 128) took 276.1 us, now 269.7; a
+// mixed step of 256 + 1024 rows 308.9, now 305.1.
 //   K: lane = (row, 16-byte unit); each store puts 8 dims of one key into the
 //      key-major tile, and the 4 units of one (key, 32-dim chunk) are one
 //      64-byte run.
@@ -68,7 +73,7 @@ __global__ void reshape_and_cache_kernel(uint16_t *__restrict__ k_pool,
 //      4 KiB dim-major tile contiguously; shorter runs (chunk ends, decode
 //      rows) write 2-byte elements.
 template <int HD>
-__global__ __launch_bounds__(256) void cache_write_kernel(
+__global__ __launch_bounds__(64) void cache_write_kernel(
     uint16_t *__restrict__ k_pool, uint16_t *__restrict__ v_pool, uint32_t kv_heads,
     const uint16_t *__restrict__ keys, const uint16_t *__restrict__ values,
     const uint32_t *__restrict__ segments, uint32_t num_items) {
@@ -76,9 +81,9 @@ __global__ __launch_bounds__(256) void cache_write_kernel(
     constexpr int DPL = HD / 64;            // V dims per lane
     constexpr uint32_t UPR = HD / 8;        // 16-byte K units per row
     constexpr uint32_t RPI = 64 / UPR;      // K rows per load instruction
-    const uint32_t item = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (item >= num_items) return;  // whole wavefront
-    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t item = blockIdx.x;
+    if (item >= num_items) return;
+    const uint32_t lane = threadIdx.x;
     const uint32_t seg = item / kv_heads;
     const uint32_t kvh = item % kv_heads;
     const uint32_t row0 = segments[3 * seg];
@@ -89,7 +94,8 @@ __global__ __launch_bounds__(256) void cache_write_kernel(
     const uint64_t width = static_cast<uint64_t>(kv_heads) * HD;
     const uint64_t tile = (static_cast<uint64_t>(slot0 / BS) * kv_heads + kvh) * (BS * HD);
 
-    // Every load of the run is issued before the first store.
+    // Every load of the run is issued before the first store; rows past the
+    // run load its last row (not stored), so no branch parts the loads.
     const uint32_t u = lane % UPR;
     const uint32_t d = 8 * u;
     const uint32_t i0 = lane / UPR;
@@ -97,22 +103,21 @@ __global__ __launch_bounds__(256) void cache_write_kernel(
     u32x4 kreg[KI];
 #pragma unroll
     for (uint32_t j = 0; j < KI; ++j) {
-        const uint32_t i = i0 + RPI * j;
-        if (i < n) kreg[j] = *reinterpret_cast<const u32x4 *>(keys + (row0 + i) * width + kvh * HD + d);
+        const uint32_t i = min(i0 + RPI * j, n - 1);
+        kreg[j] = *reinterpret_cast<const u32x4 *>(keys + (row0 + i) * width + kvh * HD + d);
     }
 
     uint16_t vv[DPL][BS];
     const uint16_t *vsrc = values + static_cast<uint64_t>(row0) * width + kvh * HD + DPL * lane;
 #pragma unroll
     for (uint32_t i = 0; i < BS; ++i) {
-        if (i < n) {
-            if constexpr (DPL == 2) {
-                const uint32_t w = *reinterpret_cast<const uint32_t *>(vsrc + i * width);
-                vv[0][i] = static_cast<uint16_t>(w & 0xffffu);
-                vv[1][i] = static_cast<uint16_t>(w >> 16);
-            } else {
-                vv[0][i] = vsrc[i * width];
-            }
+        const uint64_t at = min(i, n - 1) * width;
+        if constexpr (DPL == 2) {
+            const uint32_t w = *reinterpret_cast<const uint32_t *>(vsrc + at);
+            vv[0][i] = static_cast<uint16_t>(w & 0xffffu);
+            vv[1][i] = static_cast<uint16_t>(w >> 16);
+        } else {
+            vv[0][i] = vsrc[at];
         }
     }
 #pragma unroll
@@ -221,15 +226,15 @@ hipError_t launch_cache_write(const PoolLayer &pool, const uint16_t *keys, const
     if (plan.num_segments == 0) return hipSuccess;
     if (!cache_write_supported(pool.head_dim, pool.block_size)) return hipErrorInvalidValue;
     const uint64_t items = static_cast<uint64_t>(plan.num_segments) * pool.kv_heads;
-    const uint64_t grid = (items + 3) / 4;
+    const uint64_t grid = items;
     if (grid > 0x7fffffffull) return hipErrorInvalidValue;
     KernelTimer timer("reshape_and_cache", stream);
     if (pool.head_dim == 128)
-        hipLaunchKernelGGL((cache_write_kernel<128>), dim3(static_cast<uint32_t>(grid)), dim3(256), 0,
+        hipLaunchKernelGGL((cache_write_kernel<128>), dim3(static_cast<uint32_t>(grid)), dim3(64), 0,
                            stream, pool.k, pool.v, pool.kv_heads, keys, values, plan.segments,
                            static_cast<uint32_t>(items));
     else
-        hipLaunchKernelGGL((cache_write_kernel<64>), dim3(static_cast<uint32_t>(grid)), dim3(256), 0,
+        hipLaunchKernelGGL((cache_write_kernel<64>), dim3(static_cast<uint32_t>(grid)), dim3(64), 0,
                            stream, pool.k, pool.v, pool.kv_heads, keys, values, plan.segments,
                            static_cast<uint32_t>(items));
     return hipGetLastError();
