@@ -243,11 +243,13 @@ __device__ __forceinline__ void mask_tail_v(bf16x8 (&va)[HD / 16], int nv) {
         va[dt] = __builtin_bit_cast(bf16x8, __builtin_bit_cast(u32x4, va[dt]) & mask);
 }
 
-template <int HD, bool FIRST = false>
+// `first` (wave-uniform): the chunk begins a run, whose sums start at zero and
+// not at what acc holds.
+template <int HD>
 __device__ __forceinline__ void chunk_update(const floatx4 &s0, const floatx4 &s1,
                                              const bf16x8 (&va)[HD / 16], bool tail, int nv,
                                              float scale_log2, float &m_run, float &l_run,
-                                             floatx4 (&acc)[HD / 16]) {
+                                             floatx4 (&acc)[HD / 16], bool first) {
 #pragma clang fp contract(off)
     float sc[8];
 #pragma unroll
@@ -282,24 +284,26 @@ __device__ __forceinline__ void chunk_update(const floatx4 &s0, const floatx4 &s
     }
     l_run = l_run * alpha + ps;
     m_run = m_new;
+    if (first) {
 #pragma unroll
-    for (int dt = 0; dt < HD / 16; ++dt) {
-        if constexpr (FIRST)
+        for (int dt = 0; dt < HD / 16; ++dt)
             acc[dt] = mfma16x16x32(va[dt], pb_lo, floatx4{0.f, 0.f, 0.f, 0.f});
-        else
-            acc[dt] = mfma16x16x32(va[dt], pb_lo, acc[dt] * alpha);
-        acc[dt] = mfma16x16x32(va[dt], pb_hi, acc[dt]);
+    } else {
+#pragma unroll
+        for (int dt = 0; dt < HD / 16; ++dt) acc[dt] = mfma16x16x32(va[dt], pb_lo, acc[dt] * alpha);
     }
+#pragma unroll
+    for (int dt = 0; dt < HD / 16; ++dt) acc[dt] = mfma16x16x32(va[dt], pb_hi, acc[dt]);
 }
 
 template <int HD>
 __device__ __forceinline__ void compute_chunk(Chunk<HD> &r, const bf16x8 (&qv)[HD / 32], bool tail,
                                               int nv, float scale_log2, float &m_run, float &l_run,
-                                              floatx4 (&acc)[HD / 16]) {
+                                              floatx4 (&acc)[HD / 16], bool first) {
     floatx4 s0, s1;
     chunk_qk<HD>(r.ka, r.kb, qv, s0, s1);
     if (tail) mask_tail_v<HD>(r.va, nv);
-    chunk_update<HD>(s0, s1, r.va, tail, nv, scale_log2, m_run, l_run, acc);
+    chunk_update<HD>(s0, s1, r.va, tail, nv, scale_log2, m_run, l_run, acc, first);
 }
 
 // (mf, lf, accf) := (mf, lf, accf) merged with the run (m, l, acc) after it.
@@ -343,17 +347,21 @@ __device__ __forceinline__ void put_f32x4(float *p, floatx4 v, bool agent) {
 }
 
 // One state's run in progress (m, l, acc) and the merge of the runs before
-// it.  `flush` ends a run; `finish` leaves the state in (m, l, acc).  With a
-// wavefront's LDS given to flush and finish (room for DT * 64 floatx4), the
-// merged accumulators live there between runs, not in registers: 32
-// registers at head_dim 128, which the two chunks in flight need.
+// it.  `flush` ends a run, whose successor's first chunk replaces acc; `finish`
+// leaves the state in (m, l, acc).  With a wavefront's LDS given to flush and
+// finish (room for DT * 64 floatx4), the merged accumulators live there
+// between runs, not in registers: 32 registers at head_dim 128, which the two
+// chunks in flight need.  They come back in one round of loads, and acc is
+// not cleared: with the loads in pairs and 32 clears a flush was longer than a
+// chunk's softmax (one row of 900 / 2000 keys of 8 KV heads of 128 dims as
+// whole items: 10.8 / 18.6 us, now 10.2 / 17.7; 9.1 / 14.4 without runs at all).
 template <int HD>
 struct RunState {
     static constexpr int DT = HD / 16;
     float m, l, mf, lf;
     floatx4 acc[DT], accf[DT];
 
-    __device__ __forceinline__ void reset_run() {
+    __device__ __forceinline__ void reset() {
         m = -INFINITY;
         l = 0.0f;
 #pragma unroll
@@ -369,7 +377,8 @@ struct RunState {
         } else {
             fold_state<HD>(mf, lf, accf, m, l, acc);
         }
-        reset_run();
+        m = -INFINITY;
+        l = 0.0f;
     }
     __device__ __forceinline__ void finish(bool first) {
         if (first) return;
@@ -381,28 +390,25 @@ struct RunState {
     }
     // The same with accf in lds[dt * 64 + lane]; `first`: nothing there yet.
     __device__ __forceinline__ void flush(floatx4 *lds, int lane, bool first) {
-        merge(lds, lane, first);
+        finish(lds, lane, first);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) lds[dt * 64 + lane] = acc[dt];
         mf = m;
         lf = l;
-        reset_run();
+        m = -INFINITY;
+        l = 0.0f;
     }
-    // (m, l, acc) := the runs before it (none if `first`) merged with it.
-    __device__ __forceinline__ void merge(const floatx4 *lds, int lane, bool first) {
-#pragma clang fp contract(off)
+    __device__ __forceinline__ void finish(const floatx4 *lds, int lane, bool first) {
         if (first) return;
-        const float mx = fmaxf(mf, m);
-        const float ef = __builtin_amdgcn_exp2f(mf - mx);
-        const float e = __builtin_amdgcn_exp2f(m - mx);
-        l = lf * ef + l * e;
-        m = mx;
+        floatx4 f[DT];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            const floatx4 f = lds[dt * 64 + lane];
+        for (int dt = 0; dt < DT; ++dt) f[dt] = lds[dt * 64 + lane];
+        __builtin_amdgcn_sched_barrier(0);  // all loads, then one wait
+        fold_state<HD>(mf, lf, f, m, l, acc);
+        m = mf;
+        l = lf;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[dt][j] = __builtin_fmaf(f[j], ef, acc[dt][j] * e);
-        }
+        for (int dt = 0; dt < DT; ++dt) acc[dt] = f[dt];
     }
 };
 
@@ -595,7 +601,7 @@ __device__ __forceinline__ void shared_split(
     auto state = [&](auto w_c) __attribute__((always_inline)) {
         constexpr int w = decltype(w_c)::value;
         RunState<HD> rs;
-        rs.reset_run();
+        rs.reset();
         // One chunk per step: step t waits for its chunk (the DMA of the next
         // two may fly on) and for every wavefront to be done with the step
         // before, refills that stage with the chunk three steps on and
@@ -614,7 +620,7 @@ __device__ __forceinline__ void shared_split(
             read_k(cur, ka, kb);
             chunk_qk<HD>(ka, kb, qv, sa0, sa1);
             read_v(cur, va);
-            chunk_update<HD>(sa0, sa1, va, false, 8, scale_log2, rs.m, rs.l, rs.acc);
+            chunk_update<HD>(sa0, sa1, va, false, 8, scale_log2, rs.m, rs.l, rs.acc, sidx == 0);
         };
         static_assert(kSubChunks == 4, "a run is one turn of the stages");
         for (uint32_t k = 0; k < per; k += 4) {
@@ -825,7 +831,7 @@ __device__ __forceinline__ void shared_split_pairs(
         chunk_qk<HD>(ka, kb, qv, sa0, sa1);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) va[dt] = *reinterpret_cast<const bf16x8 *>(cur + v_rd + 512 * dt);
-        chunk_update<HD, first>(sa0, sa1, va, false, 8, scale_log2, rs.m, rs.l, rs.acc);
+        chunk_update<HD>(sa0, sa1, va, false, 8, scale_log2, rs.m, rs.l, rs.acc, first);
     };
     // Step t stages chunks pair_of(t) and the next: `per` steps (whole runs)
     // for the states 0 and 1, then as many for 2
@@ -848,7 +854,7 @@ __device__ __forceinline__ void shared_split_pairs(
 #pragma unroll 1
     for (uint32_t i = 0; i < 2; ++i) {
         RunState<HD> rs;
-        rs.reset_run();
+        rs.reset();
         auto step = [&](auto s_run, uint32_t k) __attribute__((always_inline)) {
             constexpr int in_run = decltype(s_run)::value;  // k % kSubChunks
             constexpr int sp = in_run % 2;
@@ -1269,9 +1275,11 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
         for (int kk = 0; kk < KK; ++kk) qv[kk] = head_ok ? load_bf16x8(qp + 32 * kk) : bf16x8{};
     }
     // The column's output place (first partial, splits), loaded now so that
-    // the end of the item waits on no load.
-    u32x2 cinfo = {0u, 0u};
-    if (head_ok) cinfo = *reinterpret_cast<const u32x2 *>(row_info + 2 * static_cast<uint64_t>(crow));
+    // the end of the item waits on no load; by every lane (a column without a
+    // row: the item's own row's, not used), as a branch around the load ended
+    // in a wait for it, and for Q, before the first chunk was asked for.
+    const u32x2 cinfo =
+        *reinterpret_cast<const u32x2 *>(row_info + 2 * static_cast<uint64_t>(head_ok ? crow : row));
 
     // The end of an item with a partial, when the row's last workgroup merges
     // (every column is this row's): the workgroup that counts the row's last
@@ -1315,25 +1323,28 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     floatx4 *const run_lds = kStages ? reinterpret_cast<floatx4 *>(
         wave == 0 ? sh0 : (wave == 1 ? sh1 : (wave == 2 ? sh2 : sh3))) : nullptr;
     RunState<HD> rs;
-    rs.reset_run();
+    rs.reset();
 
     // A chunk computed inside the loop has a successor, so it is full: only
     // the chunks computed at the loop's exits can be the split's tail, and
     // only they carry the masking code.
-    auto run = [&](Chunk<HD> &r, uint32_t cc, bool may_tail) {
+    auto run = [&](Chunk<HD> &r, uint32_t cc, bool may_tail, bool first) {
         const uint32_t j0 = k_begin + cc * kChunk;
         if (may_tail && take_new && cc + 1 == nchunks)
             take_new_key<HD>(r, nk - 1 - j0, nk_row, nv_row, lane);
         const bool tail = may_tail && j0 + kChunk > k_end;
         const int nv = max(0, min(8, static_cast<int>(k_end) - static_cast<int>(j0 + 8 * g)));
-        compute_chunk<HD>(r, qv, tail, nv, scale_log2, rs.m, rs.l, rs.acc);
+        compute_chunk<HD>(r, qv, tail, nv, scale_log2, rs.m, rs.l, rs.acc, first);
     };
-    // Before chunk k (even): the runs end every kSubChunks chunks.  (With
-    // another number of wavefronts than a pack's or a fine item's, a tuning
-    // setting, a state is one run.)
+    // Before chunk k (even), true if it begins a run: every kSubChunks chunks.
+    // (With another number of wavefronts than a pack's or a fine item's, a
+    // tuning setting, a state is one run.)  The run before it ends here, ahead
+    // of the next chunk's loads, whose registers it uses.
     auto new_run = [&](uint32_t k) {
+        const bool first = kStages ? k % kSubChunks == 0 : k == 0;
         if constexpr (kStages)
-            if (k != 0 && k % kSubChunks == 0) rs.flush(run_lds, lane, k == kSubChunks);
+            if (first && k != 0) rs.flush(run_lds, lane, k == kSubChunks);
+        return first;
     };
     static_assert(kSubChunks % 2 == 0, "runs start at the first register buffer");
 
@@ -1344,23 +1355,23 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     // loop, the control-flow structurizer routes that exit back through the
     // loop header, where the compiler then waits for every load in flight.
     uint32_t k = 0;
+#pragma unroll 1
     for (; k + 2 < mine; k += 2) {
+        const bool begins = new_run(k);
         load(bufB, chunk(k + 1));
-        new_run(k);
-        run(bufA, chunk(k), false);
+        run(bufA, chunk(k), false, begins);
         load(bufA, chunk(k + 2));
-        run(bufB, chunk(k + 1), false);
+        run(bufB, chunk(k + 1), false, false);
     }
+    const bool first = new_run(k);
     if (k + 1 < mine) {
         load(bufB, chunk(k + 1));
-        new_run(k);
-        run(bufA, chunk(k), false);
-        run(bufB, chunk(k + 1), true);
+        run(bufA, chunk(k), false, first);
+        run(bufB, chunk(k + 1), true, false);
     } else if (k < mine) {
-        new_run(k);
-        run(bufA, chunk(k), true);
+        run(bufA, chunk(k), true, first);
     }
-    if constexpr (kStages) rs.merge(run_lds, lane, mine <= kSubChunks);
+    if constexpr (kStages) rs.finish(run_lds, lane, mine <= kSubChunks);
     float m_run = rs.m;
     float l_run = rs.l;
     floatx4 (&acc)[DT] = rs.acc;
