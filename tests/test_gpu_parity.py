@@ -557,6 +557,39 @@ def test_decode_small_steps_bitwise(vo, monkeypatch, hd, heads, kvh):
     _assert_close(got, W.oracle_attention(orc, wl), f"small steps hd={hd} H={heads}")
 
 
+def test_decode_pool_of_another_shape_than_the_metadata(vo):
+    """Step metadata serves any pool of its block size.  One of more KV heads
+    counts its arrivals inside the metadata's counters (every row of the
+    metadata in use, those past one split at its end); one of a larger head
+    dimension needs larger partials: bitwise the result with metadata of its
+    own where they fit, refused where they do not."""
+    import torch
+    _say("decode: pool and metadata of different shapes")
+    ctx = [40, 3000, 700, 4200, 2100, 9000]
+    tables = sum(-(-(c + 1) // 16) for c in ctx)
+    backend = vo.HipBackend(device=0, max_seqs=8, max_rows=W.FILL_ROWS, max_table_entries=2048,
+                            max_query_heads=32)
+    for kvh, hd, small_kvh, small_hd, entries, fits in ((8, 64, 1, 64, tables, True),
+                                                        (16, 128, 2, 128, tables, True),
+                                                        (8, 128, 8, 64, 16384, True),
+                                                        (8, 128, 8, 64, tables, False)):
+        wl = W.build(vo, backend, kind="decode", heads=32, kv_heads=kvh, head_dim=hd, block_size=16,
+                     num_blocks=tables + 8, context_lens=ctx, seed=kvh + hd)
+        want = _bits(_out(wl, backend))
+        small = backend.alloc_kv_pool(vo.KvLayout(1, 4, 16, small_kvh, small_hd))
+        meta = vo.StepMeta(small, len(ctx), len(ctx), entries, 32)
+        meta.upload(wl.meta)
+        for _ in range(3):
+            out = torch.zeros_like(wl.q)
+            args = (vo._dev_ptr(wl.q), wl.q.shape[0], wl.q.shape[1], wl.pool.handle, 0, meta.handle,
+                    vo._dev_ptr(out), vo._stream_ptr(None))
+            if not fits:
+                assert vo.lib.vo_decode_attention(*args) == vo.VO_ERR_CAPACITY
+                continue
+            vo._check(vo.lib.vo_decode_attention(*args))
+            assert np.array_equal(_bits(out), want), (kvh, hd)
+
+
 def test_decode_batch_invariance_bitwise(vo, gpu_backend):
     """A row's output is identical alone or in a batch (the reference's
     batch-invariance invariant, CLAUDE.md; model.rs:539-584)."""

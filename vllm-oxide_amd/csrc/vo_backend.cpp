@@ -592,6 +592,7 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
     // arithmetic.  Fine items, short chains of work, come last.
     if (rows) std::fill(row_info, row_info + 2 * T, 0u);
     uint64_t n = 0, nred = 0;
+    m->part_end = 0;
     for (uint64_t i = 0; i < R; ++i) {
         const uint64_t r = row_at(i);
         const uint64_t nk = m->row_num_keys[r];
@@ -601,6 +602,7 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
         row_info[2 * r + 1] = static_cast<uint32_t>(ns) | (fr ? kernels::kFineRow : 0u);
         n += fr ? 4 * ns : ns;
         if (ns > 1 || fr) {
+            m->part_end = n;
             uint32_t *rec = reduce_rows + 4 * nred++;
             rec[0] = static_cast<uint32_t>(r);
             rec[1] = row_info[2 * r];
@@ -1008,7 +1010,7 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
                         slots * max_query_heads * 2 * sizeof(float));
     if (err == hipSuccess)
         err = hipMalloc(reinterpret_cast<void **>(&m->d_arrivals),
-                        max_rows * m->kv_heads * sizeof(uint32_t));
+                        max_rows * max_query_heads * sizeof(uint32_t));
     if (err == hipSuccess)
         err = hipMalloc(reinterpret_cast<void **>(&m->d_tokens), max_rows * sizeof(uint32_t));
     if (err == hipSuccess) err = m->tokens_stage.create(max_rows * sizeof(uint32_t));
@@ -1021,7 +1023,7 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
     if (err == hipSuccess) err = hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking);
     // On a stream of its own, as the null stream's work may be under capture.
     if (err == hipSuccess)
-        err = hipMemsetAsync(m->d_arrivals, 0, max_rows * m->kv_heads * sizeof(uint32_t), m->side);
+        err = hipMemsetAsync(m->d_arrivals, 0, max_rows * max_query_heads * sizeof(uint32_t), m->side);
     if (err == hipSuccess) err = hipStreamSynchronize(m->side);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&m->fork, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&m->join, hipEventDisableTiming);
@@ -1345,6 +1347,16 @@ vo_status check_attention(const char *op, const void *queries, uint64_t rows, ui
     return VO_OK;
 }
 
+
+// The partials of the decode plan fit the metadata's buffers, which are sized
+// with the head dimension of the pool it was created for, whatever this
+// pool's.  (The arrival counters are sized for as many KV heads as query
+// heads.)
+vo_status check_partials(const vo_step_meta *m, uint64_t heads, uint64_t head_dim) {
+    const uint64_t room = std::max(m->max_parts, m->fine_slots) * m->max_heads * m->head_dim;
+    const uint64_t need = m->part_end * heads * head_dim;
+    return need <= room ? VO_OK : fail_capacity("split-K partials per step (values)", need, room);
+}
 
 }  // namespace
 
@@ -1790,6 +1802,8 @@ extern "C" int32_t vo_prefill_attention(const void *queries, uint64_t rows, uint
         // fill the wavefront slots the MFMA-bound prefill workgroups leave
         // free.
         const hipStream_t st = static_cast<hipStream_t>(stream);
+        if (m->decode_planned)
+            if (vo_status rc = check_partials(m, heads, L.head_dim)) return rc;
         const bool overlap = m->decode_planned && mixed_overlap_enabled();
         if (overlap) {
             err = hipEventRecord(m->fork, st);
@@ -1839,6 +1853,7 @@ extern "C" int32_t vo_decode_attention(const void *queries, uint64_t rows, uint6
     if (kernels::decode_mfma_supported(static_cast<uint32_t>(L.head_dim),
                                        static_cast<uint32_t>(L.block_size), group) &&
         m->decode_planned) {
+        if (vo_status rc = check_partials(m, heads, L.head_dim)) return rc;
         err = kernels::launch_decode_mfma(pool->layer(layer), m->view, m->plan,
                                           static_cast<const uint16_t *>(queries),
                                           static_cast<uint16_t *>(out), heads, scale,
@@ -1878,6 +1893,7 @@ extern "C" int32_t vo_decode_attention_write_kv(const void *queries, uint64_t ro
         const float scale = 1.0f / std::sqrt(static_cast<float>(L.head_dim));  // attention.rs:88
         const kernels::NewKeys nk{static_cast<const uint16_t *>(keys),
                                   static_cast<const uint16_t *>(values), m->d_write_slots};
+        if (vo_status rc = check_partials(m, heads, L.head_dim)) return rc;
         const hipError_t err = kernels::launch_decode_mfma(
             pool->layer(layer), m->view, m->plan, static_cast<const uint16_t *>(queries),
             static_cast<uint16_t *>(out), heads, scale, decode_waves(),

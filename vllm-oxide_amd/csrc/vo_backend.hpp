@@ -224,7 +224,7 @@ struct vo_step_meta {
     // Split-K partials (fp32).
     float *d_part_acc = nullptr;
     float *d_part_ml = nullptr;
-    // Arrival counters of the rows' work items [max_rows][kv_heads], zero
+    // Arrival counters of the rows' work items [max_rows][max_heads], zero
     // between launches (the decode kernel's in-launch merge).
     uint32_t *d_arrivals = nullptr;
 
@@ -243,6 +243,7 @@ struct vo_step_meta {
     std::vector<uint64_t> seq_keys;    // scratch of plan_decode: keys read per sequence
     std::vector<uint32_t> decode_rows; // rows of a prefill step planned on the decode kernel
     uint64_t decode_parts = 0;         // split-K partials of the plan (work items before packing)
+    uint64_t part_end = 0;             // one past the last partial slot that a launch of it writes
     uint64_t decode_items = 0;         // its work items, a split of fine items counted once
     std::unordered_map<uint64_t, uint32_t> pack_open;  // scratch of plan_decode: open packs by hash
     std::vector<uint32_t> pack_fill;                   // scratch of plan_decode: rows per pack
