@@ -417,7 +417,11 @@ int32_t vo_prefill_attention(const void *queries, uint64_t rows, uint64_t cols,
 
 /* Backend::decode_attention (mod.rs:137-149; CPU: cpu/mod.rs:314-339): one
  * query row per sequence.  Split-K over the keys with an fp32 partial per
- * split and a reduce kernel.  `meta` must hold a decode upload. */
+ * split, merged by the launch itself or by a reduce kernel (same bits).
+ * `meta` must hold a decode upload.  The partials are the metadata's: calls
+ * with one meta whose rows have more than one split must follow one another;
+ * others may overlap, on other streams than the upload's or as replays of a
+ * graph. */
 int32_t vo_decode_attention(const void *queries, uint64_t rows, uint64_t cols,
                             const vo_kv_pool *pool, uint64_t layer, const vo_step_meta *meta,
                             void *out, void *stream);

@@ -590,6 +590,62 @@ def test_decode_pool_of_another_shape_than_the_metadata(vo):
             assert np.array_equal(_bits(out), want), (kvh, hd)
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+def test_decode_launches_on_two_streams_of_one_metadata(vo, hd):
+    """Rows of one split share nothing between launches, so launches of one
+    metadata may overlap: a recorded graph replays on a stream of its own while
+    another stream and the upload's own run eager launches, each bitwise as
+    alone.  Only the launches on the upload's stream, which follow one another,
+    split the longer rows finer."""
+    import torch
+    _say(f"decode: two streams, one metadata, hd={hd}")
+    ctx = [1500, 2046, 1100, 2047, 600]
+    backend = vo.HipBackend(device=0, max_seqs=8, max_rows=W.FILL_ROWS, max_table_entries=2048,
+                            max_query_heads=32)
+    wl = W.build(vo, backend, kind="decode", heads=32, kv_heads=8, head_dim=hd, block_size=16,
+                 num_blocks=700, context_lens=ctx, seed=hd, num_layers=3, fill_layers=[0, 1, 2])
+    gen = torch.Generator(device="cuda:0").manual_seed(hd)
+    qs = [torch.randn(wl.q.shape, generator=gen, device="cuda:0").to(torch.bfloat16) for _ in range(3)]
+    run = lambda layer, out=None: backend.decode_attention(qs[layer], wl.pool, layer, wl.meta, out=out)  # noqa: E731
+
+    def kernels(stream):
+        torch.cuda.synchronize()
+        vo.profile_reset()
+        vo.enable_profiling(True)
+        with torch.cuda.stream(stream):
+            out = run(0)
+        torch.cuda.synchronize()
+        vo.enable_profiling(False)
+        return set(vo.profile()), _bits(out)
+    own, side, replay = torch.cuda.current_stream(), torch.cuda.Stream(), torch.cuda.Stream()
+    want = [_bits(run(layer)) for layer in range(3)]
+    for stream, kernel in ((own, "decode_splitk_fine"), (side, "decode_splitk")):
+        ran, got = kernels(stream)
+        assert ran == {kernel}, (stream, ran)
+        assert np.array_equal(got, want[0])
+    outs = [[torch.zeros_like(wl.q) for _ in range(20)] for _ in range(3)]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for o in outs[2]:
+            run(2, o)
+    for _ in range(3):
+        for o in (o for some in outs for o in some):
+            o.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(replay):
+            for _ in range(5):
+                graph.replay()
+        for a, b in zip(outs[0], outs[1]):
+            run(0, a)
+            with torch.cuda.stream(side):
+                run(1, b)
+        torch.cuda.synchronize()
+        for layer in range(3):
+            for o in outs[layer]:
+                assert np.array_equal(_bits(o), want[layer]), layer
+    assert np.array_equal(_bits(run(0)), want[0])
+
+
 def test_decode_batch_invariance_bitwise(vo, gpu_backend):
     """A row's output is identical alone or in a batch (the reference's
     batch-invariance invariant, CLAUDE.md; model.rs:539-584)."""

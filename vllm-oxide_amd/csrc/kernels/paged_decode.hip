@@ -39,7 +39,9 @@
 // chunks (over 1 us each from HBM) and the number of CUs that read at all.
 // Two rows of 5000-8100 keys of 8 KV heads of 128 dims are 64 whole items: 25.5 us,
 // and 13.8 as 220 fine ones, of a 53 MB read; one row of 8000 keys 27 and
-// 13.8 us a call.
+// 13.8 us a call.  Fine items give rows of one split partials too, so only the
+// launches that the metadata knows to follow one another run them; any other
+// takes the whole items, with the same bits.
 //
 // The merge.  The last workgroup of a row (and KV head) to finish merges the
 // row's partials: they are written and read with
@@ -49,8 +51,10 @@
 // whose workgroups count for each of their rows, 64 rows behind a 4096-key
 // prefix and one of 32768 keys 73.5 -> 72.7 us).  (A release and an acquire fence
 // per workgroup instead are an L2 writeback and invalidate each time, which
-// measured 5-9x slower than the separate launch.)  Packs of one tile and
-// fixed launches keep the reduce kernel.
+// measured 5-9x slower than the separate launch.)  The counters are the
+// upload's, as the plan: zero when it arrives and zero after each launch.
+// Packs of one tile, fixed launches, launches under capture and launches on
+// another stream than the upload's keep the reduce kernel.
 // Workgroups are numbered KV head fastest, so the KV heads of one block are
 // read at about the same time.
 //
@@ -1166,10 +1170,11 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __syncthreads();
     };
-    // Counts one of row r's `expected` items for this KV head.  True for the
-    // last, which leaves the counter at zero for the next launch.
-    auto count_item = [&](uint32_t r, uint32_t expected) {
-        uint32_t *const count = arrivals + static_cast<uint64_t>(r) * kv_heads + kvh;
+    // Counts one of the `expected` items of the row whose partials start at
+    // `first`, for this KV head.  True for the last, which leaves the counter
+    // at zero for the next launch.
+    auto count_item = [&](uint32_t first, uint32_t expected) {
+        uint32_t *const count = arrivals + static_cast<uint64_t>(first) * kv_heads + kvh;
         const uint32_t before =
             __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const bool last = before + 1 == expected;
@@ -1191,8 +1196,10 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
         stored();
         if (threadIdx.x < pack) {
             const uint32_t r = threadIdx.x == 0 ? row : mates[(pack - 1) * item + threadIdx.x - 1];
-            const uint32_t nsplit = r == kNoMate ? 1u : row_info[2 * static_cast<uint64_t>(r) + 1];
-            s_last[threadIdx.x] = nsplit > 1 && count_item(r, nsplit) ? r : kNoMate;
+            const u32x2 info = *reinterpret_cast<const u32x2 *>(
+                row_info + 2 * static_cast<uint64_t>(r == kNoMate ? row : r));
+            s_last[threadIdx.x] =
+                r != kNoMate && info[1] > 1 && count_item(info[0], info[1]) ? r : kNoMate;
         }
         __syncthreads();
         for (uint32_t j = 0; j < pack; ++j) {
@@ -1288,8 +1295,8 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
     auto arrive = [&](uint32_t first, uint32_t nsplit, bool fine_row) {
         stored();
         if (threadIdx.x == 0)
-            s_last[0] = count_item(row, fine_row ? W * (nk / split_keys) + split_states(nk % split_keys)
-                                                 : nsplit);
+            s_last[0] = count_item(first, fine_row ? W * (nk / split_keys) + split_states(nk % split_keys)
+                                                   : nsplit);
         __syncthreads();
         if (s_last[0] != 0) merge(row, first, nsplit, fine_row);
     };
@@ -1540,16 +1547,16 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
 }
 
 // Merges the split-K partials of the rows listed in reduce_rows (those with
-// more than one split, and those of fine items; rows with one whole split
-// were written by the split kernel), where the row's last workgroup does not:
-// plans with one-tile packs and fixed launches.  A wavefront is a workgroup and takes
-// 64 / (HD / 4) query heads of one row, a thread four dims (with four such to
-// a workgroup 65 rows of 64 heads took 5.8 us instead of 5.5).
+// more than one split; rows with one split were written by the split kernel),
+// where the row's last workgroup does not (no arrivals).  A wavefront is a
+// workgroup and takes 64 / (HD / 4) query heads of one row, a thread four dims
+// (with four such to a workgroup 65 rows of 64 heads took 5.8 us instead of
+// 5.5).
 template <int HD>
 __global__ __launch_bounds__(64) void decode_reduce_kernel(
     const uint32_t *__restrict__ reduce_rows, const float *__restrict__ part_acc,
     const float *__restrict__ part_ml, uint16_t *__restrict__ out, uint32_t num_heads,
-    const uint32_t *__restrict__ counts, uint32_t split_keys) {
+    const uint32_t *__restrict__ counts) {
     constexpr uint32_t NQ = HD / 4;    // dim quads of one head
     constexpr uint32_t HPW = 64 / NQ;  // heads per workgroup
     const uint32_t groups = (num_heads + HPW - 1) / HPW;
@@ -1559,8 +1566,8 @@ __global__ __launch_bounds__(64) void decode_reduce_kernel(
     if (blockIdx.x / groups >= counts[1]) return;  // past this step's rows (fixed launch)
     const uint32_t qh = (blockIdx.x % groups) * HPW + threadIdx.x / NQ;
     if (qh >= num_heads) return;
-    merge_row<HD, false>(part_acc, part_ml, rec[1], rec[2] & ~kFineRow, (rec[2] & kFineRow) != 0,
-                         rec[3], split_keys, num_heads, qh, 4 * (threadIdx.x % NQ),
+    merge_row<HD, false>(part_acc, part_ml, rec[1], rec[2], false, 0, 0, num_heads, qh,
+                         4 * (threadIdx.x % NQ),
                          out + (static_cast<uint64_t>(rec[0]) * num_heads + qh) * HD);
 }
 
@@ -1591,7 +1598,7 @@ hipError_t launch_split_kind(const PoolLayer &pool, const MetaView &meta, const 
                             : (2 * W * 16 + static_cast<size_t>(W) * item_pack * group * kAccStride<HD>) * 4;
     const uint64_t grid = static_cast<uint64_t>(plan.launch_work) * pool.kv_heads;
     if (grid > 0x7fffffffull) return hipErrorInvalidValue;
-    KernelTimer timer("decode_splitk", stream);
+    KernelTimer timer(plan.fine ? "decode_splitk_fine" : "decode_splitk", stream);
     hipLaunchKernelGGL((decode_splitk_kernel<HD, W, NT, PACKS>), dim3(static_cast<uint32_t>(grid)),
                        dim3(64 * W), smem, stream, pool.k, pool.v, pool.kv_heads, meta.tables,
                        plan.work, plan.row_info,
@@ -1644,7 +1651,7 @@ hipError_t launch_hd(const PoolLayer &pool, const MetaView &meta, const DecodePl
     KernelTimer timer("decode_reduce", stream);
     hipLaunchKernelGGL((decode_reduce_kernel<HD>), dim3(static_cast<uint32_t>(grid)), dim3(64),
                        0, stream, plan.reduce_rows, plan.part_acc, plan.part_ml, out, num_heads,
-                       plan.counts, plan.split_keys);
+                       plan.counts);
     return hipGetLastError();
 }
 

@@ -191,9 +191,9 @@ struct DecodePlan {
                                   // launch_work records readable; a zero-key row has one item
     const uint32_t *row_info;     // [T][2]: (first partial index, number of splits, kFineRow);
                                   // (0, 0) for rows the plan does not cover
-    const uint32_t *reduce_rows;  // [num_reduce_rows][4]: (row, its row_info, its keys) of the rows
-                                  // with more than one split and the fine rows; 16-byte aligned,
-                                  // launch_reduce records readable
+    const uint32_t *reduce_rows;  // [num_reduce_rows][4]: (row, its row_info, unused) of the rows
+                                  // with more than one split; 16-byte aligned, launch_reduce
+                                  // records readable
     uint32_t num_work;
     uint32_t num_reduce_rows;
     uint32_t split_keys;          // keys per split, a multiple of 32, <= kMaxSplitKeys
@@ -219,12 +219,14 @@ struct DecodePlan {
     // each keeping two of the tile's four softmax states, so pack <= W / 2 *
     // (16 / group) and each wavefront walks half of the split's chunks.
     bool shared_pairs;
-    // With arrivals, [rows][kv_heads] counters that are zero between
-    // launches, the workgroup that finishes a row's last item for a KV head
-    // merges its partials and no reduce kernel runs; only for plans whose
-    // packs, if any, are shared ones, on four wavefronts.  Null: the reduce
+    // With arrivals, [partials][kv_heads] counters (a row's are its first
+    // partial's) that are zero between launches, the workgroup that finishes a
+    // row's last item for a KV head merges its partials and no reduce kernel
+    // runs; only for plans whose packs, if any, are shared ones, on four
+    // wavefronts, and for launches that follow one another.  Null: the reduce
     // kernel.
     uint32_t *arrivals;
+    bool fine;  // rows run as fine items (kFineRow); needs arrivals
 };
 
 constexpr uint32_t kNoMate = 0xffffffffu;

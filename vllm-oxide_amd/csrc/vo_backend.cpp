@@ -146,6 +146,7 @@ vo_status finish_upload(vo_step_meta *m, const Packer &pk, hipStream_t stream, c
         const hipError_t err = m->stage.commit(m->d_buf, pk.used(), stream);
         if (err != hipSuccess) return fail_device(op, err, hipGetErrorString(err));
     }
+    m->upload_stream = stream;
     return VO_OK;
 }
 
@@ -218,8 +219,8 @@ vo_status upload_common(vo_step_meta *m, MetaKind kind, const char *op, uint64_t
 
     const uint32_t *dp;
     // The split-K counts the kernels read; plan_decode_rows fills them.
-    m->h_counts = pk.add(kRegCounts, 2, &dp);
-    m->h_counts[0] = m->h_counts[1] = 0;
+    m->h_counts = pk.add(kRegCounts, 4, &dp);
+    std::fill(m->h_counts, m->h_counts + 4, 0u);
     m->d_counts = dp;
     uint32_t *h = pk.add(kRegTableOff, num_seqs + 1, &dp);
     for (uint64_t s = 0; s <= num_seqs; ++s) h[s] = static_cast<uint32_t>(table_off[s]);
@@ -552,6 +553,83 @@ uint64_t fine_items(uint64_t keys, uint64_t L) {
     return 4 * (keys / L) + std::min<uint64_t>(4, (keys % L + 31) / 32);
 }
 
+// Where the split's block ids start in the tables, and the (leading) row's key
+// count: the rest of each of the n records in `work`.
+void finish_work_records(const vo_step_meta *m, uint32_t *work, uint64_t n, uint64_t L) {
+    for (uint64_t i = 0; i < n; ++i) {
+        const uint32_t row = work[4 * i];
+        const uint64_t split = work[4 * i + 1] & kernels::kSplitMask;
+        work[4 * i + 2] =
+            static_cast<uint32_t>(m->table_off[m->row_seq[row]] + split * L / m->block_size);
+        work[4 * i + 3] = m->row_num_keys[row];
+    }
+}
+
+// The fine plan of a step of few rows, beside m->plan (already made, without
+// packs): the longer rows as fine items, the others as m->plan has them, in an
+// order of their own; fine items, short chains of work, come last.
+void plan_fine_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32_t> *rows,
+                    const uint32_t *whole_work) {
+    const uint64_t T = m->num_rows, L = m->plan.split_keys;
+    const uint64_t R = rows ? rows->size() : T;
+    auto row_at = [&](uint64_t i) -> uint64_t { return rows ? (*rows)[i] : i; };
+    auto fine_row = [](uint64_t keys) { return keys > kFineMinKeys; };
+    uint64_t items = 0;
+    bool any = false;
+    for (uint64_t i = 0; i < R; ++i) {
+        const uint64_t nk = m->row_num_keys[row_at(i)];
+        any |= fine_row(nk);
+        items += fine_row(nk) ? fine_items(nk, L) : row_splits(nk, L);
+    }
+    if (!any) return;
+    kernels::DecodePlan &p = m->fine_plan;
+    p = m->plan;
+    const uint32_t *dp;
+    uint32_t *work = pk.add(kRegFineWork, 4 * items, &dp);
+    p.work = dp;
+    uint32_t *row_info = pk.add(kRegFineRowInfo, 2 * T, &dp);
+    p.row_info = dp;
+    if (rows) std::fill(row_info, row_info + 2 * T, 0u);
+    uint64_t n = 0, f = 0;
+    for (uint64_t i = 0; i < R; ++i) {
+        const uint64_t r = row_at(i);
+        const uint64_t nk = m->row_num_keys[r];
+        const uint64_t ns = row_splits(nk, L);
+        row_info[2 * r] = static_cast<uint32_t>(n);
+        row_info[2 * r + 1] = static_cast<uint32_t>(ns) | (fine_row(nk) ? kernels::kFineRow : 0u);
+        n += fine_row(nk) ? 4 * ns : ns;
+    }
+    for (uint64_t i = 0; i < m->plan.num_work; ++i) {
+        if (fine_row(m->row_num_keys[whole_work[4 * i]])) continue;
+        work[4 * f] = whole_work[4 * i];
+        work[4 * f + 1] = whole_work[4 * i + 1];
+        ++f;
+    }
+    for (uint64_t i = 0; i < R; ++i) {
+        const uint64_t r = row_at(i);
+        const uint64_t nk = m->row_num_keys[r];
+        if (!fine_row(nk)) continue;
+        const uint64_t n_items = fine_items(nk, L);
+        for (uint64_t k = 0; k < n_items; ++k, ++f) {
+            work[4 * f] = static_cast<uint32_t>(r);
+            work[4 * f + 1] = static_cast<uint32_t>(k / 4) |
+                              static_cast<uint32_t>(k % 4 + 1) << kernels::kPartShift;
+        }
+    }
+    finish_work_records(m, work, f, L);
+    uint32_t *counters = pk.add(kRegFineArrivals, n * m->kv_heads, &dp);
+    std::fill(counters, counters + n * m->kv_heads, 0u);
+    p.arrivals = const_cast<uint32_t *>(dp);
+    p.fine = true;
+    p.reduce_rows = nullptr;
+    p.num_work = p.launch_work = static_cast<uint32_t>(f);
+    p.num_reduce_rows = p.launch_reduce = 0;
+    p.part_acc = m->d_part_acc + m->max_parts * m->max_heads * m->head_dim;
+    p.part_ml = m->d_part_ml + m->max_parts * m->max_heads * 2;
+    m->h_counts[2] = static_cast<uint32_t>(f);
+    p.counts = m->d_counts + 2;
+}
+
 // Split-K plan over the rows listed in `rows` (every row of the step when
 // rows is null).  Rows outside the plan get row_info (0, 0).
 vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32_t> *rows) {
@@ -565,20 +643,9 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
 
     const bool streaming = pk.fixed() ? m->fixed.streaming : decode_streaming(m);
     const int waves = decode_waves();
-    // Fine items need four wavefronts, splits they can cover, partial slots,
-    // and no blocks that several rows read (packs serve those).
-    const bool fine = streaming && !pk.fixed() && waves == 4 && L % 128 == 0 &&
-                      L <= kernels::kMaxFineSplit && 4 * parts <= m->fine_slots &&
-                      parts * m->kv_heads < decode_fine_limit(m->num_cus);
-    auto fine_row = [&](uint64_t keys) { return fine && keys > kFineMinKeys; };
-    uint64_t items = 0;
-    for (uint64_t i = 0; i < R; ++i) {
-        const uint64_t nk = m->row_num_keys[row_at(i)];
-        items += fine_row(nk) ? fine_items(nk, L) : row_splits(nk, L);
-    }
 
     const uint32_t *dp;
-    uint32_t *work = pk.add(kRegWork, 4 * items, &dp);
+    uint32_t *work = pk.add(kRegWork, 4 * parts, &dp);
     m->plan.work = dp;
     uint32_t *row_info = pk.add(kRegRowInfo, 2 * T, &dp);
     m->plan.row_info = dp;
@@ -589,25 +656,23 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
     // workgroups out in grid order as slots free up, so the short items fill
     // the gaps at the end instead of a full split starting last and running
     // alone.  Partials are addressed by (row, split), so the order changes no
-    // arithmetic.  Fine items, short chains of work, come last.
+    // arithmetic.
     if (rows) std::fill(row_info, row_info + 2 * T, 0u);
     uint64_t n = 0, nred = 0;
     m->part_end = 0;
     for (uint64_t i = 0; i < R; ++i) {
         const uint64_t r = row_at(i);
-        const uint64_t nk = m->row_num_keys[r];
-        const uint64_t ns = row_splits(nk, L);
-        const bool fr = fine_row(nk);
+        const uint64_t ns = row_splits(m->row_num_keys[r], L);
         row_info[2 * r] = static_cast<uint32_t>(n);
-        row_info[2 * r + 1] = static_cast<uint32_t>(ns) | (fr ? kernels::kFineRow : 0u);
-        n += fr ? 4 * ns : ns;
-        if (ns > 1 || fr) {
-            m->part_end = n;
+        row_info[2 * r + 1] = static_cast<uint32_t>(ns);
+        n += ns;
+        if (ns > 1) {
             uint32_t *rec = reduce_rows + 4 * nred++;
             rec[0] = static_cast<uint32_t>(r);
             rec[1] = row_info[2 * r];
             rec[2] = row_info[2 * r + 1];
-            rec[3] = static_cast<uint32_t>(nk);
+            rec[3] = 0;
+            m->part_end = n;
         }
     }
     m->tail_items.clear();
@@ -634,7 +699,6 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
         uint64_t nf = 0;
         for (uint64_t i = 0; i < R; ++i) {
             const uint64_t r = row_at(i);
-            if (fine_row(m->row_num_keys[r])) continue;
             for (uint64_t sp = 0; sp < m->row_num_keys[r] / L; ++sp, ++nf) {
                 work[4 * nf] = static_cast<uint32_t>(r);
                 work[4 * nf + 1] = static_cast<uint32_t>(sp);
@@ -646,7 +710,6 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
     for (uint64_t i = 0; i < R; ++i) {
         const uint64_t r = row_at(i);
         const uint64_t nk = m->row_num_keys[r];
-        if (fine_row(nk)) continue;
         if (nk % L != 0 || nk == 0)
             m->tail_items.push_back({static_cast<uint32_t>(nk % L), static_cast<uint32_t>(r),
                                      static_cast<uint32_t>(nk / L)});
@@ -675,29 +738,9 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
         if (P > 1) std::fill(mates + (P - 1) * f, mates + (P - 1) * (f + 1), kernels::kNoMate);
         ++f;
     }
-    for (uint64_t i = 0; fine && i < R; ++i) {
-        const uint64_t r = row_at(i);
-        const uint64_t nk = m->row_num_keys[r];
-        if (!fine_row(nk)) continue;
-        const uint64_t n_items = fine_items(nk, L);
-        for (uint64_t k = 0; k < n_items; ++k, ++f) {
-            work[4 * f] = static_cast<uint32_t>(r);
-            work[4 * f + 1] = static_cast<uint32_t>(k / 4) |
-                              static_cast<uint32_t>(k % 4 + 1) << kernels::kPartShift;
-        }
-    }
-    const uint64_t num_work = f;  // = items unless packed
-    // The rest of each record: where the split's block ids start in the
-    // tables, and the (leading) row's key count.
-    for (uint64_t i = 0; i < num_work; ++i) {
-        const uint32_t row = work[4 * i];
-        const uint64_t split = work[4 * i + 1] & kernels::kSplitMask;
-        work[4 * i + 2] =
-            static_cast<uint32_t>(m->table_off[m->row_seq[row]] + split * L / m->block_size);
-        work[4 * i + 3] = m->row_num_keys[row];
-    }
+    const uint64_t num_work = f;  // = parts unless packed
+    finish_work_records(m, work, num_work, L);
     m->decode_parts = parts;
-    m->decode_items = num_work - items + parts;  // a split of fine items counts once
     m->plan.pack = P;
     m->plan.num_work = static_cast<uint32_t>(num_work);
     m->plan.num_reduce_rows = static_cast<uint32_t>(nred);
@@ -705,7 +748,7 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
     m->plan.part_acc = m->d_part_acc;
     m->plan.part_ml = m->d_part_ml;
     m->plan.arrivals = nullptr;
-    if (!pk.fixed() && (P == 1 || m->plan.num_shared != 0) && waves == 4 && decode_arrive()) m->plan.arrivals = m->d_arrivals;
+    m->plan.fine = false;
     m->h_counts[0] = static_cast<uint32_t>(num_work);
     m->h_counts[1] = static_cast<uint32_t>(nred);
     m->plan.counts = m->d_counts;
@@ -720,6 +763,23 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
         m->plan.streaming = streaming || (m->plan.num_shared != 0 && decode_pack_nt());
         m->plan.launch_work = static_cast<uint32_t>(num_work);
         m->plan.launch_reduce = static_cast<uint32_t>(nred);
+    }
+    // What launches that follow one another add (launch_plan): the merge in
+    // the launch, for plans without one-tile packs on four wavefronts, and
+    // fine items, which also need splits they can cover, partial slots, and no
+    // blocks that several rows read (packs serve those).
+    m->arrivals = nullptr;
+    m->fine_plan.fine = false;
+    if (!pk.fixed() && waves == 4 && decode_arrive()) {
+        if (streaming && L % 128 == 0 && L <= kernels::kMaxFineSplit && 4 * parts <= m->fine_slots &&
+            parts * m->kv_heads < decode_fine_limit(m->num_cus))
+            plan_fine_rows(m, pk, rows, work);
+        if (!m->fine_plan.fine && (P == 1 || m->plan.num_shared != 0) && nred != 0) {
+            const uint64_t words = m->part_end * m->kv_heads;
+            uint32_t *counters = pk.add(kRegArrivals, words, &dp);
+            std::fill(counters, counters + words, 0u);
+            m->arrivals = const_cast<uint32_t *>(dp);
+        }
     }
     m->decode_planned = true;
     // New keys cached by the decode launch: a whole decode step without
@@ -987,18 +1047,20 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
     // decode_fine_limit workgroups, and no more than the step can have.
     m->fine_slots = 4 * std::min<uint64_t>(m->max_parts,
                                            decode_fine_limit(m->num_cus) / std::max<uint64_t>(1, m->kv_heads) + 1);
-    const uint64_t slots = std::max(m->max_parts, m->fine_slots);
+    const uint64_t slots = m->max_parts + m->fine_slots;
 
     const uint64_t u32s = (max_seqs + 1) + max_table_entries + 3 * max_rows  // offsets, tables, row arrays
                           + max_rows                                         // write slots
                           + 3 * max_rows                                     // write plan
                           + max_rows                                         // positions
-                          + 4 * slots + 6 * max_rows                         // decode plan
+                          + 2 + 4 * m->max_parts + 6 * max_rows              // decode plan
+                          + 4 * m->fine_slots + 2 * max_rows                 // fine plan
+                          + slots * m->kv_heads                              // arrival counters
                           + 4 * (max_rows + max_seqs)                        // prefill plan
                           + (5 + kernels::kPipeFirstWords) * (max_rows + max_seqs) + 1  // its slot plan
                           + max_seqs                                         // last rows
                           + (decode_pack_limit(m) - 1) * m->max_parts        // row-packing mates
-                          + 10 * 64;                                         // alignment slack
+                          + kNumRegions * 64;                                // alignment slack
     m->buf_bytes = align_up(u32s * sizeof(uint32_t), 4096);
     hipError_t err = hipMalloc(reinterpret_cast<void **>(&m->d_buf), m->buf_bytes);
     if (err == hipSuccess) err = m->stage.create(m->buf_bytes);
@@ -1009,9 +1071,6 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
         err = hipMalloc(reinterpret_cast<void **>(&m->d_part_ml),
                         slots * max_query_heads * 2 * sizeof(float));
     if (err == hipSuccess)
-        err = hipMalloc(reinterpret_cast<void **>(&m->d_arrivals),
-                        max_rows * max_query_heads * sizeof(uint32_t));
-    if (err == hipSuccess)
         err = hipMalloc(reinterpret_cast<void **>(&m->d_tokens), max_rows * sizeof(uint32_t));
     if (err == hipSuccess) err = m->tokens_stage.create(max_rows * sizeof(uint32_t));
     if (err == hipSuccess)
@@ -1021,10 +1080,6 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
     if (err == hipSuccess) err = m->aux_stage.create(max_rows * sizeof(uint32_t));
     // Default priority, like every stream here.
     if (err == hipSuccess) err = hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking);
-    // On a stream of its own, as the null stream's work may be under capture.
-    if (err == hipSuccess)
-        err = hipMemsetAsync(m->d_arrivals, 0, max_rows * max_query_heads * sizeof(uint32_t), m->side);
-    if (err == hipSuccess) err = hipStreamSynchronize(m->side);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&m->fork, hipEventDisableTiming);
     if (err == hipSuccess) err = hipEventCreateWithFlags(&m->join, hipEventDisableTiming);
     if (err != hipSuccess) {
@@ -1038,7 +1093,6 @@ extern "C" int32_t vo_step_meta_create(const vo_kv_pool *pool, uint64_t max_seqs
         m->stage.destroy();
         if (m->d_part_acc) (void)hipFree(m->d_part_acc);
         if (m->d_part_ml) (void)hipFree(m->d_part_ml);
-        if (m->d_arrivals) (void)hipFree(m->d_arrivals);
         if (m->side) (void)hipStreamDestroy(m->side);
         if (m->fork) (void)hipEventDestroy(m->fork);
         if (m->join) (void)hipEventDestroy(m->join);
@@ -1062,7 +1116,6 @@ extern "C" void vo_step_meta_destroy(vo_step_meta *m) {
     (void)hipFree(m->d_buf);
     (void)hipFree(m->d_part_acc);
     (void)hipFree(m->d_part_ml);
-    (void)hipFree(m->d_arrivals);
     if (m->side) {
         (void)hipStreamSynchronize(m->side);
         (void)hipStreamDestroy(m->side);
@@ -1255,8 +1308,8 @@ extern "C" int32_t vo_step_meta_fix_launch(vo_step_meta *m, uint64_t work_headro
     f.streaming = m->plan.streaming;
     const uint64_t S = f.seqs;
     const uint64_t caps[kNumRegions] = {
-        2, S + 1, f.entries_cap, S, S, f.has_positions ? S : 0, S, 3 * S,
-        4 * f.work_cap, 2 * S, 4 * S, S, 0, 0, 0};
+        4, S + 1, f.entries_cap, S, S, f.has_positions ? S : 0, S, 3 * S,
+        4 * f.work_cap, 2 * S, 4 * S, S, 0, 0, 0, 0, 0, 0, 0};
     uint64_t off = 0;
     for (int r = 0; r < kNumRegions; ++r) {
         off = align_up(off, 256);
@@ -1285,7 +1338,7 @@ extern "C" int32_t vo_step_meta_decode_plan(const vo_step_meta *m, uint64_t *wor
                                             uint64_t *partials, uint32_t *pack) {
     if (!m || !work_items || !partials || !pack) return fail_argument("decode_plan", "null argument");
     if (!m->decode_planned) return fail_argument("decode_plan", "the last upload has no decode plan");
-    *work_items = m->decode_items;
+    *work_items = m->plan.num_work;
     *partials = m->decode_parts;
     *pack = m->plan.pack ? m->plan.pack : 1;
     clear_error();
@@ -1348,14 +1401,40 @@ vo_status check_attention(const char *op, const void *queries, uint64_t rows, ui
 }
 
 
-// The partials of the decode plan fit the metadata's buffers, which are sized
-// with the head dimension of the pool it was created for, whatever this
-// pool's.  (The arrival counters are sized for as many KV heads as query
-// heads.)
-vo_status check_partials(const vo_step_meta *m, uint64_t heads, uint64_t head_dim) {
-    const uint64_t room = std::max(m->max_parts, m->fine_slots) * m->max_heads * m->head_dim;
-    const uint64_t need = m->part_end * heads * head_dim;
-    return need <= room ? VO_OK : fail_capacity("split-K partials per step (values)", need, room);
+// The partials of the plan fit the metadata's, whatever the pool's head
+// dimension (they are sized with the one of the pool it was created for).
+vo_status check_partials(const vo_step_meta *m, const kernels::DecodePlan &plan, uint64_t heads,
+                         uint64_t head_dim) {
+    if (plan.fine || m->part_end * heads * head_dim <= m->max_parts * m->max_heads * m->head_dim)
+        return VO_OK;
+    return fail_capacity("split-K partials per step (values)", m->part_end * heads * head_dim,
+                         m->max_parts * m->max_heads * m->head_dim);
+}
+
+// The plan that a decode launch on `stream` takes.  The in-launch merge and
+// fine items share counters and partials between launches, so they are for
+// launches known to follow one another: those on the stream of the upload
+// (`ordered`: on the metadata's own side stream), of a pool with the shape the
+// metadata was created for.  Any other launch, which may overlap with those
+// (another stream, or a graph that replays wherever it is told to), takes the
+// plan that shares nothing for rows of one split.  Same bits.
+kernels::DecodePlan launch_plan(const vo_step_meta *m, const vo_kv_pool *pool, hipStream_t stream,
+                                bool ordered) {
+    const kernels::DecodePlan &best = m->fine_plan.fine ? m->fine_plan : m->plan;
+    if (!m->arrivals && !best.fine) return m->plan;
+    if (pool->layout.kv_heads != m->kv_heads || pool->layout.head_dim != m->head_dim) return m->plan;
+    // hipStreamPerThread is one handle for a stream of each thread.
+    if (!ordered && (stream != static_cast<hipStream_t>(m->upload_stream) || stream == hipStreamPerThread))
+        return m->plan;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+        (void)hipGetLastError();
+        return m->plan;
+    }
+    if (capture != hipStreamCaptureStatusNone) return m->plan;
+    kernels::DecodePlan plan = best;
+    if (!plan.fine) plan.arrivals = m->arrivals;
+    return plan;
 }
 
 }  // namespace
@@ -1802,9 +1881,12 @@ extern "C" int32_t vo_prefill_attention(const void *queries, uint64_t rows, uint
         // fill the wavefront slots the MFMA-bound prefill workgroups leave
         // free.
         const hipStream_t st = static_cast<hipStream_t>(stream);
-        if (m->decode_planned)
-            if (vo_status rc = check_partials(m, heads, L.head_dim)) return rc;
         const bool overlap = m->decode_planned && mixed_overlap_enabled();
+        kernels::DecodePlan plan;
+        if (m->decode_planned) {
+            plan = launch_plan(m, pool, st, overlap);
+            if (vo_status rc = check_partials(m, plan, heads, L.head_dim)) return rc;
+        }
         if (overlap) {
             err = hipEventRecord(m->fork, st);
             if (err == hipSuccess) err = hipStreamWaitEvent(m->side, m->fork, 0);
@@ -1815,7 +1897,7 @@ extern "C" int32_t vo_prefill_attention(const void *queries, uint64_t rows, uint
                                            static_cast<uint16_t *>(out), heads, scale,
                                            pool->num_cus, st);
         if (err == hipSuccess && m->decode_planned)
-            err = kernels::launch_decode_mfma(pool->layer(layer), m->view, m->plan,
+            err = kernels::launch_decode_mfma(pool->layer(layer), m->view, plan,
                                               static_cast<const uint16_t *>(queries),
                                               static_cast<uint16_t *>(out), heads, scale,
                                               decode_waves(), overlap ? m->side : st);
@@ -1853,8 +1935,9 @@ extern "C" int32_t vo_decode_attention(const void *queries, uint64_t rows, uint6
     if (kernels::decode_mfma_supported(static_cast<uint32_t>(L.head_dim),
                                        static_cast<uint32_t>(L.block_size), group) &&
         m->decode_planned) {
-        if (vo_status rc = check_partials(m, heads, L.head_dim)) return rc;
-        err = kernels::launch_decode_mfma(pool->layer(layer), m->view, m->plan,
+        const kernels::DecodePlan plan = launch_plan(m, pool, static_cast<hipStream_t>(stream), false);
+        if (vo_status rc = check_partials(m, plan, heads, L.head_dim)) return rc;
+        err = kernels::launch_decode_mfma(pool->layer(layer), m->view, plan,
                                           static_cast<const uint16_t *>(queries),
                                           static_cast<uint16_t *>(out), heads, scale,
                                           decode_waves(), static_cast<hipStream_t>(stream));
@@ -1893,9 +1976,10 @@ extern "C" int32_t vo_decode_attention_write_kv(const void *queries, uint64_t ro
         const float scale = 1.0f / std::sqrt(static_cast<float>(L.head_dim));  // attention.rs:88
         const kernels::NewKeys nk{static_cast<const uint16_t *>(keys),
                                   static_cast<const uint16_t *>(values), m->d_write_slots};
-        if (vo_status rc = check_partials(m, heads, L.head_dim)) return rc;
+        const kernels::DecodePlan plan = launch_plan(m, pool, static_cast<hipStream_t>(stream), false);
+        if (vo_status rc = check_partials(m, plan, heads, L.head_dim)) return rc;
         const hipError_t err = kernels::launch_decode_mfma(
-            pool->layer(layer), m->view, m->plan, static_cast<const uint16_t *>(queries),
+            pool->layer(layer), m->view, plan, static_cast<const uint16_t *>(queries),
             static_cast<uint16_t *>(out), heads, scale, decode_waves(),
             static_cast<hipStream_t>(stream), &nk);
         return device_status(op, err);

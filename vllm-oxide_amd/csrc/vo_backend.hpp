@@ -62,7 +62,7 @@ enum MetaKind { kNone = 0, kPrefill = 1, kDecode = 2, kSlots = 3 };
 // The arrays of one upload in the metadata buffer.  Ordinary uploads pack
 // them back to back; with fixed launch shapes each has a fixed offset.
 enum Region {
-    kRegCounts = 0,  // [2]: split-K work items, rows to reduce (read by the kernels)
+    kRegCounts = 0,  // [4]: split-K work items, rows to reduce (read by the kernels); the same of fine_plan
     kRegTableOff,
     kRegTables,
     kRegRowSeq,
@@ -77,6 +77,10 @@ enum Region {
     kRegPrefillWork,
     kRegPrefillPipe,
     kRegMates,
+    kRegArrivals,
+    kRegFineWork,
+    kRegFineRowInfo,
+    kRegFineArrivals,
     kNumRegions
 };
 
@@ -193,7 +197,7 @@ struct vo_step_meta {
     uint64_t head_dim = 0;
 
     uint64_t max_seqs = 0, max_rows = 0, max_entries = 0, max_heads = 0, max_parts = 0;
-    uint64_t fine_slots = 0;  // partial slots of a plan of fine decode items (decode_fine_rows)
+    uint64_t fine_slots = 0;  // partial slots of fine_plan
 
     vo::MetaKind kind = vo::kNone;
     uint64_t block_size = 0;
@@ -221,17 +225,24 @@ struct vo_step_meta {
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
 
-    // Split-K partials (fp32).
+    // Split-K partials (fp32): max_parts slots of `plan`, then fine_slots of
+    // `fine_plan`, so that a launch of one leaves the other's alone.
     float *d_part_acc = nullptr;
     float *d_part_ml = nullptr;
-    // Arrival counters of the rows' work items [max_rows][max_heads], zero
-    // between launches (the decode kernel's in-launch merge).
-    uint32_t *d_arrivals = nullptr;
 
     vo::kernels::MetaView view{};
     const uint32_t *d_write_slots = nullptr;  // slots with superseded rows = kSkipSlot
     vo::kernels::WritePlan write_plan{};      // runs of consecutive slots inside one block
+    // The decode plan of any launch: whole splits, merged by the reduce kernel.
     vo::kernels::DecodePlan plan{};
+    // What launches that follow one another take instead (launch_plan): the
+    // same plan with its rows merged in the launch by way of these counters,
+    // or, for a step of few rows, `fine_plan`.  Null and off otherwise.
+    uint32_t *arrivals = nullptr;
+    vo::kernels::DecodePlan fine_plan{};
+    // The stream of the last upload, to compare a launch's with; never used as
+    // a stream.
+    void *upload_stream = nullptr;
     bool decode_planned = false;
     bool slots_repeat = false;  // a slot appears in two rows of the step
     // Decode step whose new keys can be cached by the decode launch itself
@@ -244,7 +255,6 @@ struct vo_step_meta {
     std::vector<uint32_t> decode_rows; // rows of a prefill step planned on the decode kernel
     uint64_t decode_parts = 0;         // split-K partials of the plan (work items before packing)
     uint64_t part_end = 0;             // one past the last partial slot that a launch of it writes
-    uint64_t decode_items = 0;         // its work items, a split of fine items counted once
     std::unordered_map<uint64_t, uint32_t> pack_open;  // scratch of plan_decode: open packs by hash
     std::vector<uint32_t> pack_fill;                   // scratch of plan_decode: rows per pack
     vo::kernels::PrefillPlan prefill_plan{};

@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kPlanThreads) void decode_static_plan_kernel(
             rec[0] = s;
             rec[1] = row_info[2 * s];
             rec[2] = n;
-            rec[3] = nk;
+            rec[3] = 0;
         }
     }
     if (tid == 0) {
