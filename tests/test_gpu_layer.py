@@ -20,6 +20,7 @@ reference's HF check, tests/hf_match.rs).
 """
 import ctypes
 import dataclasses
+import gc
 import math
 
 import numpy as np
@@ -739,6 +740,49 @@ def test_batch_checks(vo, M, gpu_backend):
     assert (e.value.value, e.value.limit) == (65, 64)
     with pytest.raises(vo.ShapeError):
         m.prefill(kv, W.ref_prompt(5, 0), vo.PrefillMeta.new([vo.PrefillSeq(0, 6, table)], 4))
+
+
+def test_no_garbage_collection_while_recording(vo, M, gpu_backend):
+    """Cyclic garbage that would be due while a decode step is recorded (a
+    collection at every allocation) is collected after the recording: a
+    finalizer that frees device memory there breaks it.  The recorded step
+    still equals the eager one."""
+    import torch
+    _say("no collection while recording")
+    cfg, w, prompts, tables, _ = _cfg1_setup(seed=4)
+    lens = [len(p) for p in prompts]
+    model, kv = _gpu_model(vo, M, gpu_backend, cfg, w, 64, 16)
+    pm = vo.PrefillMeta.new([vo.PrefillSeq(0, n, t) for n, t in zip(lens, tables)], 16)
+    toks = model.prefill(kv, sum(prompts, []), pm).tokens
+    meta = vo.DecodeMeta.new([vo.DecodeSeq(c, t[:(c + 16) // 16]) for c, t in zip(lens, tables)], 16)
+    want = model.decode(kv, toks, meta, want_logits=True)
+    seen = []
+
+    class Cycle:
+        def __init__(self):
+            self.me = self
+
+        def __del__(self):
+            seen.append(torch.cuda.is_current_stream_capturing())
+    launch = model._launch
+
+    def launch_and_drop(*args, **kwargs):
+        for _ in range(20):
+            Cycle()
+        return launch(*args, **kwargs)
+    model._launch = launch_and_drop
+    gc.collect()
+    threshold = gc.get_threshold()
+    gc.set_threshold(1, 1, 1)
+    try:
+        graph = model.capture_decode(kv, toks, meta)
+    finally:
+        gc.set_threshold(*threshold)
+        del model._launch
+    gc.collect()
+    assert len(seen) == 40 and not any(seen), seen
+    got = graph.run(toks, meta, want_logits=True)
+    assert got.tokens == want.tokens and np.array_equal(got.logits, want.logits)
 
 
 def test_decode_graph_replays_equal_eager_steps(vo, M, gpu_backend):

@@ -8,6 +8,7 @@ Plus size-independent properties at full BASELINE sizes: batch invariance and
 block-relabelling invariance (bitwise), single key -> V exactly.
 """
 import dataclasses
+import gc
 import os
 
 import numpy as np
@@ -625,9 +626,11 @@ def test_decode_launches_on_two_streams_of_one_metadata(vo, hd):
         assert np.array_equal(got, want[0])
     outs = [[torch.zeros_like(wl.q) for _ in range(20)] for _ in range(3)]
     graph = torch.cuda.CUDAGraph()
+    gc.disable()  # an earlier test's pool is not freed while recording
     with torch.cuda.graph(graph):
         for o in outs[2]:
             run(2, o)
+    gc.enable()
     for _ in range(3):
         for o in (o for some in outs for o in some):
             o.zero_()

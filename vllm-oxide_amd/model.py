@@ -30,7 +30,9 @@ projection add into the residual inside the GEMM (beta = 1).
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import gc
 from dataclasses import dataclass, field
 from typing import List, Optional, Sequence
 
@@ -39,6 +41,22 @@ import numpy as np
 from . import (VO_DTYPE_F32, CapacityError, DecodeMeta, HipBackend, KvLayout,
                KvPool, PrefillMeta, RopeTable, ShapeError, _check, _engine_error, _stream_ptr,
                _vp, lib, VO_ERR_CAPACITY, VO_ERR_SHAPE)
+
+
+@contextlib.contextmanager
+def _no_collection():
+    """No automatic garbage collection inside: the finalizer of a dropped model,
+    pool or metadata frees device memory and its hipBLASLt handle, which must
+    not happen while a stream is recorded (a collection that found an earlier
+    model there ended the process).  What is dropped meanwhile is collected
+    afterwards."""
+    enabled = gc.isenabled()
+    gc.disable()
+    try:
+        yield
+    finally:
+        if enabled:
+            gc.enable()
 
 
 @dataclass(frozen=True)
@@ -251,7 +269,7 @@ class Llama:
         self._argmax_device(S)
         torch.cuda.synchronize()
         graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
+        with _no_collection(), torch.cuda.graph(graph):
             self._launch(pool, m, S, S, False)
             self._argmax_device(S)
         return DecodeGraph(self, pool, m, graph, S)
