@@ -649,6 +649,47 @@ def test_decode_launches_on_two_streams_of_one_metadata(vo, hd):
     assert np.array_equal(_bits(run(0)), want[0])
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("nalias,env", [
+    (0, {}), (0, {"VO_DECODE_FINE": "0"}), (0, {"VO_DECODE_FINE": "0", "VO_DECODE_ARRIVE": "0"}),
+    (0, {"VO_DECODE_WAVES": "8"}), (3, {}), (3, {"VO_DECODE_SHARED_PAIRS": "0"}),
+    (3, {"VO_DECODE_PACK": "1"})])
+def test_decode_keys_scored_minus_infinity(vo, monkeypatch, hd, nalias, env):
+    """Keys whose score is -inf have weight zero wherever they lie: the first
+    chunk of every wavefront, the first chunks of a run, a whole run, a whole
+    split; in whole and fine items and in packs.  Against the softmax in 64
+    bits over the same keys."""
+    import torch
+    for k, v in env.items():
+        monkeypatch.setenv(k, v)
+    _say(f"decode -inf scores hd={hd} alias={nalias} {env}")
+    heads, kvh, prefix = 16, 4, 4096
+    ctx = [prefix + e for e in (40, 700, 2100)] if nalias else [1200, 5000, 2047]
+    backend = vo.HipBackend(device=0, max_seqs=8, max_rows=W.FILL_ROWS, max_table_entries=2048,
+                            max_query_heads=heads)
+    wl = W.build(vo, backend, kind="decode", heads=heads, kv_heads=kvh, head_dim=hd, block_size=16,
+                 num_blocks=1200, context_lens=ctx, seed=hd + nalias,
+                 shared_prefix=prefix if nalias else 0, shared_count=nalias)
+    q = wl.q.clone()
+    q.view(len(ctx), heads, hd)[:, :, 0] = 1.0  # times a key's -inf: its score
+    for s in range(len(ctx)):
+        at = [p for a, b in ((0, 128), (512, 640), (1024, 1100), (1536, 2048), (2048, 4096)) if b < ctx[s]
+              for p in range(a, b)]
+        k, v = backend.read_kv(wl.pool, 0, wl.meta, s, ctx[s])
+        k.view(ctx[s], kvh, hd)[at, :, 0] = float("-inf")
+        slots = np.asarray([int(wl.tables[s][p // 16]) * 16 + p % 16 for p in at], np.uint32)
+        backend.write_kv(wl.pool, 0, k[at].contiguous(), v[at].contiguous(), slots)
+    got = backend.decode_attention(q, wl.pool, 0, wl.meta)
+    for s in range(len(ctx)):
+        k, v = backend.read_kv(wl.pool, 0, wl.meta, s, ctx[s] + 1)
+        for h in range(heads):
+            kh = k.view(-1, kvh, hd)[:, h // (heads // kvh)].double()
+            vh = v.view(-1, kvh, hd)[:, h // (heads // kvh)].double()
+            w = torch.softmax(kh @ q[s].view(heads, hd)[h].double() / hd ** 0.5, 0)
+            _assert_close(got[s].view(heads, hd)[h].float().cpu().numpy(), (w @ vh).cpu().numpy(),
+                          f"sequence {s}, head {h}")
+
+
 def test_decode_batch_invariance_bitwise(vo, gpu_backend):
     """A row's output is identical alone or in a batch (the reference's
     batch-invariance invariant, CLAUDE.md; model.rs:539-584)."""

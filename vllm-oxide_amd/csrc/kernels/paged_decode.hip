@@ -109,6 +109,10 @@ namespace {
 constexpr int kBS = 16;     // block size of the MFMA path
 constexpr int kChunk = 32;  // keys per wavefront iteration
 constexpr uint32_t kSubChunks = 4;  // chunks of one run of a state (see fold_state)
+// The running max before any key: the lowest finite value, not -inf, so that
+// keys scored -inf (weight zero) make no -inf - -inf, wherever they lie; with
+// no other key yet, what is summed is zero.
+constexpr float kNoMax = -3.40282347e38f;
 
 __device__ __forceinline__ floatx4 mfma16x16x32(bf16x8 a, bf16x8 b, floatx4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -269,7 +273,7 @@ __device__ __forceinline__ void chunk_update(const floatx4 &s0, const floatx4 &s
 #pragma unroll
     for (int i = 1; i < 8; ++i) mt = fmaxf(mt, sc[i]);
     mt = column_max(mt);
-    // finite: every chunk has a valid key (and the scale is positive)
+    // at least kNoMax (the scale is positive)
     const float m_new = fmaxf(m_run, mt * scale_log2);
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     // P goes to the MFMA as two bf16 parts, hi = bf16(p) and lo = bf16(p - hi),
@@ -311,7 +315,7 @@ __device__ __forceinline__ void compute_chunk(Chunk<HD> &r, const bf16x8 (&qv)[H
 }
 
 // (mf, lf, accf) := (mf, lf, accf) merged with the run (m, l, acc) after it.
-// Every run holds a chunk, so both maxima are finite.
+// Both maxima are at least kNoMax, so neither difference is -inf - -inf.
 template <int HD>
 __device__ __forceinline__ void fold_state(float &mf, float &lf, floatx4 (&accf)[HD / 16], float m,
                                            float l, const floatx4 (&acc)[HD / 16]) {
@@ -366,7 +370,7 @@ struct RunState {
     floatx4 acc[DT], accf[DT];
 
     __device__ __forceinline__ void reset() {
-        m = -INFINITY;
+        m = kNoMax;
         l = 0.0f;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) acc[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -381,7 +385,7 @@ struct RunState {
         } else {
             fold_state<HD>(mf, lf, accf, m, l, acc);
         }
-        m = -INFINITY;
+        m = kNoMax;
         l = 0.0f;
     }
     __device__ __forceinline__ void finish(bool first) {
@@ -399,7 +403,7 @@ struct RunState {
         for (int dt = 0; dt < DT; ++dt) lds[dt * 64 + lane] = acc[dt];
         mf = m;
         lf = l;
-        m = -INFINITY;
+        m = kNoMax;
         l = 0.0f;
     }
     __device__ __forceinline__ void finish(const floatx4 *lds, int lane, bool first) {
@@ -663,15 +667,12 @@ __device__ __forceinline__ void shared_split(
     for (int dt = 0; dt < DT; ++dt) num[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < W; ++w) {
-        const float mw = ms[w];
-        if (mw != -INFINITY) {
-            const float e = __builtin_amdgcn_exp2f(mw - mx);
+        const float e = __builtin_amdgcn_exp2f(ms[w] - mx);
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) num[dt][j] += e * as[w][dt][j];
-            den += e * ls[w];
-        }
+            for (int j = 0; j < 4; ++j) num[dt][j] += e * as[w][dt][j];
+        den += e * ls[w];
     }
     if (cinfo[1] == 1) {
         uint16_t *op = out + static_cast<uint64_t>(crow) * num_heads * HD +
@@ -941,17 +942,14 @@ __device__ __forceinline__ void shared_split_pairs(
     for (int dt = 0; dt < DT; ++dt) num[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-        const float mw = sm[w];
-        if (mw != -INFINITY) {
-            const float e = __builtin_amdgcn_exp2f(mw - mx);
+        const float e = __builtin_amdgcn_exp2f(sm[w] - mx);
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-                const floatx4 a = (w & 1) ? xa[((w >> 1) * DT + dt) * 64 + lane] : as[w >> 1][dt];
+        for (int dt = 0; dt < DT; ++dt) {
+            const floatx4 a = (w & 1) ? xa[((w >> 1) * DT + dt) * 64 + lane] : as[w >> 1][dt];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) num[dt][j] += e * a[j];
-            }
-            den += e * sl[w];
+            for (int j = 0; j < 4; ++j) num[dt][j] += e * a[j];
         }
+        den += e * sl[w];
     }
     if (cinfo[1] == 1) {
         uint16_t *op = out + static_cast<uint64_t>(crow) * num_heads * HD +
@@ -1520,12 +1518,9 @@ decode_splitk_kernel(const uint16_t *__restrict__ k_pool, const uint16_t *__rest
             float num = 0.0f, den = 0.0f;
 #pragma unroll
             for (int w = 0; w < W; ++w) {
-                const float mw = sm_m[w * 16 + col];
-                if (mw != -INFINITY) {
-                    const float e = __builtin_amdgcn_exp2f(mw - mx);
-                    num += e * sm_acc_w(w)[col * kAccStride<HD> + d];
-                    den += e * sm_l[w * 16 + col];
-                }
+                const float e = __builtin_amdgcn_exp2f(sm_m[w * 16 + col] - mx);
+                num += e * sm_acc_w(w)[col * kAccStride<HD> + d];
+                den += e * sm_l[w * 16 + col];
             }
             const uint32_t qh = kvh * group + (col % group);
             const uint32_t nsplit = s_col[2][col];
