@@ -690,6 +690,45 @@ def test_decode_keys_scored_minus_infinity(vo, monkeypatch, hd, nalias, env):
                           f"sequence {s}, head {h}")
 
 
+@pytest.mark.parametrize("rows,in_launch", [(8, False), (100, True)])
+def test_decode_packs_merge_bitwise(vo, monkeypatch, rows, in_launch):
+    """Rows with shared packs are merged by the launch itself in large steps of
+    packs of four, and by the reduce kernel in others and with
+    VO_DECODE_ARRIVE=0: the same bits on repeated launches, for new queries
+    and after an upload of another step in between (the arrival counters start
+    and end at zero), and within tolerance of the oracle."""
+    import torch
+    _say(f"decode packs merge, {rows} rows")
+    monkeypatch.setenv("VO_DECODE_SPLIT", "512")
+    backend = vo.HipBackend(device=0, max_seqs=128, max_rows=W.FILL_ROWS, max_table_entries=20000,
+                            max_query_heads=64)
+    ctx = [1024 + (37 * i) % 700 for i in range(rows)] + [300]
+    wl = W.build(vo, backend, kind="decode", heads=64, kv_heads=8, head_dim=128, block_size=16,
+                 num_blocks=64 + 48 * (rows + 1), context_lens=ctx, seed=rows, shared_prefix=1024,
+                 shared_count=rows)
+    other = vo.DecodeMeta.new([vo.DecodeSeq(c, t) for c, t in zip(ctx[1:], wl.tables[1:])], 16)
+    gen = torch.Generator(device="cuda:0").manual_seed(rows)
+    qs = [wl.q, torch.randn(wl.q.shape, generator=gen, device="cuda:0").to(torch.bfloat16)]
+    outs = {}
+    for arrive in ("0", "1"):
+        monkeypatch.setenv("VO_DECODE_ARRIVE", arrive)
+        backend.step_meta(wl.pool).holds = None
+        vo.profile_reset()
+        vo.enable_profiling(True)
+        outs[arrive] = [_bits(backend.decode_attention(q, wl.pool, 0, wl.meta)) for q in qs]
+        torch.cuda.synchronize()
+        vo.enable_profiling(False)
+        assert ("decode_reduce" in vo.profile()) != (in_launch and arrive == "1"), arrive
+        for _ in range(3):
+            for q, want in zip(qs, outs[arrive]):
+                assert np.array_equal(_bits(backend.decode_attention(q, wl.pool, 0, wl.meta)), want)
+            backend.decode_attention(qs[1][1:].contiguous(), wl.pool, 0, other)
+    for a, b in zip(outs["0"], outs["1"]):
+        assert np.array_equal(a, b)
+    got = backend.decode_attention(wl.q, wl.pool, 0, wl.meta).float().cpu().numpy()
+    _assert_close(got, W.oracle_attention(orc, wl), f"packs, {rows} rows")
+
+
 def test_decode_batch_invariance_bitwise(vo, gpu_backend):
     """A row's output is identical alone or in a batch (the reference's
     batch-invariance invariant, CLAUDE.md; model.rs:539-584)."""

@@ -48,13 +48,14 @@
 // agent-scope accesses and counted with a relaxed atomic, and no reduce
 // launch follows (3 us of GPU time, and 2.5 us of the host's in a small
 // call: 13.8 -> 11.1 us for one row of 8000 keys of 64 dims; with shared packs,
-// whose workgroups count for each of their rows, 64 rows behind a 4096-key
-// prefix and one of 32768 keys 73.5 -> 72.7 us).  (A release and an acquire fence
+// whose workgroups count for each of their rows, in the plans that the host
+// chooses it for: merge_packs_in_launch).  (A release and an acquire fence
 // per workgroup instead are an L2 writeback and invalidate each time, which
 // measured 5-9x slower than the separate launch.)  The counters are the
 // upload's, as the plan: zero when it arrives and zero after each launch.
-// Packs of one tile, fixed launches, launches under capture and launches on
-// another stream than the upload's keep the reduce kernel.
+// Packs of one tile, most plans with shared packs, fixed launches, launches
+// under capture and launches on another stream than the upload's keep the
+// reduce kernel.
 // Workgroups are numbered KV head fastest, so the KV heads of one block are
 // read at about the same time.
 //

@@ -543,9 +543,24 @@ uint64_t decode_fine_limit(uint64_t num_cus) {
     return env >= 0 ? static_cast<uint64_t>(env) : num_cus * 5 / 8;
 }
 
-// Whether the decode launch merges the partials itself (plans without one-tile packs;
-// VO_DECODE_ARRIVE=0: the reduce kernel does, a tuning knob).
+// Whether the decode launch may merge the partials itself (VO_DECODE_ARRIVE=0:
+// the reduce kernel does, a tuning knob).
 bool decode_arrive() { return env_int("VO_DECODE_ARRIVE", 1) != 0; }
+
+// Plans with shared packs: the last workgroup of a pack merges its rows one
+// after another, about 0.65 us each, at the end of the launch, where the
+// reduce kernel takes all rows at once for a launch of 3 us.  Measured, merge
+// in the launch against the reduce kernel: 8 rows behind a 4096-key prefix at
+// 8 rows to a pack (32 / 8 heads) 44.7 / 39.7 us of 128 dims, 33.9 / 29.1 of
+// 64; at 4 to a pack (64 / 8 heads of 128) 42.4 / 40.0.  Only with packs of 4 and more
+// workgroups than two to a CU run at once do the rest of the workgroups hide
+// it: 880 workgroups 90.2 / 90.7, 904 70.8 / 71.4, 1008 99.8 / 99.5, 1264
+// 137.6 / 144.2, 1536 109.9 / 113.0, 2048 156.7 / 159.9; but 768 57.6 / 56.6
+// (and at 8 to a pack 1152 73.3 / 69.5, 1536 110.4 / 112.8: no line there).
+bool merge_packs_in_launch(const vo_step_meta *m, uint64_t items, uint32_t pack) {
+    return m->head_dim == 128 && pack <= 4 &&
+           items * m->kv_heads > 27 * static_cast<uint64_t>(m->num_cus) / 8;  // 864 of 256 CUs
+}
 
 // States of a row that hold keys, and so its fine items: four per whole
 // split, and one per 32-key chunk of a shorter one.
@@ -582,7 +597,7 @@ void plan_fine_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32_t> *ro
         items += fine_row(nk) ? fine_items(nk, L) : row_splits(nk, L);
     }
     if (!any) return;
-    kernels::DecodePlan &p = m->fine_plan;
+    kernels::DecodePlan &p = m->own_plan;
     p = m->plan;
     const uint32_t *dp;
     uint32_t *work = pk.add(kRegFineWork, 4 * items, &dp);
@@ -765,20 +780,21 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
         m->plan.launch_reduce = static_cast<uint32_t>(nred);
     }
     // What launches that follow one another add (launch_plan): the merge in
-    // the launch, for plans without one-tile packs on four wavefronts, and
-    // fine items, which also need splits they can cover, partial slots, and no
+    // the launch, for plans without one-tile packs on four wavefronts (with
+    // shared packs, merge_packs_in_launch), and fine items, which also need splits they can cover, partial slots, and no
     // blocks that several rows read (packs serve those).
-    m->arrivals = nullptr;
-    m->fine_plan.fine = false;
+    m->own_plan = kernels::DecodePlan{};
     if (!pk.fixed() && waves == 4 && decode_arrive()) {
         if (streaming && L % 128 == 0 && L <= kernels::kMaxFineSplit && 4 * parts <= m->fine_slots &&
             parts * m->kv_heads < decode_fine_limit(m->num_cus))
             plan_fine_rows(m, pk, rows, work);
-        if (!m->fine_plan.fine && (P == 1 || m->plan.num_shared != 0) && nred != 0) {
+        if (!m->own_plan.fine && nred != 0 &&
+            (P == 1 || (m->plan.num_shared != 0 && merge_packs_in_launch(m, num_work, P)))) {
             const uint64_t words = m->part_end * m->kv_heads;
             uint32_t *counters = pk.add(kRegArrivals, words, &dp);
             std::fill(counters, counters + words, 0u);
-            m->arrivals = const_cast<uint32_t *>(dp);
+            m->own_plan = m->plan;
+            m->own_plan.arrivals = const_cast<uint32_t *>(dp);
         }
     }
     m->decode_planned = true;
@@ -1418,11 +1434,11 @@ vo_status check_partials(const vo_step_meta *m, const kernels::DecodePlan &plan,
 // metadata was created for.  Any other launch, which may overlap with those
 // (another stream, or a graph that replays wherever it is told to), takes the
 // plan that shares nothing for rows of one split.  Same bits.
-kernels::DecodePlan launch_plan(const vo_step_meta *m, const vo_kv_pool *pool, hipStream_t stream,
-                                bool ordered) {
-    const kernels::DecodePlan &best = m->fine_plan.fine ? m->fine_plan : m->plan;
-    if (!m->arrivals && !best.fine) return m->plan;
-    if (pool->layout.kv_heads != m->kv_heads || pool->layout.head_dim != m->head_dim) return m->plan;
+const kernels::DecodePlan &launch_plan(const vo_step_meta *m, const vo_kv_pool *pool,
+                                       hipStream_t stream, bool ordered) {
+    if (!m->own_plan.arrivals || pool->layout.kv_heads != m->kv_heads ||
+        pool->layout.head_dim != m->head_dim)
+        return m->plan;
     // hipStreamPerThread is one handle for a stream of each thread.
     if (!ordered && (stream != static_cast<hipStream_t>(m->upload_stream) || stream == hipStreamPerThread))
         return m->plan;
@@ -1431,10 +1447,7 @@ kernels::DecodePlan launch_plan(const vo_step_meta *m, const vo_kv_pool *pool, h
         (void)hipGetLastError();
         return m->plan;
     }
-    if (capture != hipStreamCaptureStatusNone) return m->plan;
-    kernels::DecodePlan plan = best;
-    if (!plan.fine) plan.arrivals = m->arrivals;
-    return plan;
+    return capture == hipStreamCaptureStatusNone ? m->own_plan : m->plan;
 }
 
 }  // namespace
@@ -1882,11 +1895,9 @@ extern "C" int32_t vo_prefill_attention(const void *queries, uint64_t rows, uint
         // free.
         const hipStream_t st = static_cast<hipStream_t>(stream);
         const bool overlap = m->decode_planned && mixed_overlap_enabled();
-        kernels::DecodePlan plan;
-        if (m->decode_planned) {
-            plan = launch_plan(m, pool, st, overlap);
+        const kernels::DecodePlan &plan = m->decode_planned ? launch_plan(m, pool, st, overlap) : m->plan;
+        if (m->decode_planned)
             if (vo_status rc = check_partials(m, plan, heads, L.head_dim)) return rc;
-        }
         if (overlap) {
             err = hipEventRecord(m->fork, st);
             if (err == hipSuccess) err = hipStreamWaitEvent(m->side, m->fork, 0);
@@ -1935,7 +1946,7 @@ extern "C" int32_t vo_decode_attention(const void *queries, uint64_t rows, uint6
     if (kernels::decode_mfma_supported(static_cast<uint32_t>(L.head_dim),
                                        static_cast<uint32_t>(L.block_size), group) &&
         m->decode_planned) {
-        const kernels::DecodePlan plan = launch_plan(m, pool, static_cast<hipStream_t>(stream), false);
+        const kernels::DecodePlan &plan = launch_plan(m, pool, static_cast<hipStream_t>(stream), false);
         if (vo_status rc = check_partials(m, plan, heads, L.head_dim)) return rc;
         err = kernels::launch_decode_mfma(pool->layer(layer), m->view, plan,
                                           static_cast<const uint16_t *>(queries),
@@ -1976,7 +1987,7 @@ extern "C" int32_t vo_decode_attention_write_kv(const void *queries, uint64_t ro
         const float scale = 1.0f / std::sqrt(static_cast<float>(L.head_dim));  // attention.rs:88
         const kernels::NewKeys nk{static_cast<const uint16_t *>(keys),
                                   static_cast<const uint16_t *>(values), m->d_write_slots};
-        const kernels::DecodePlan plan = launch_plan(m, pool, static_cast<hipStream_t>(stream), false);
+        const kernels::DecodePlan &plan = launch_plan(m, pool, static_cast<hipStream_t>(stream), false);
         if (vo_status rc = check_partials(m, plan, heads, L.head_dim)) return rc;
         const hipError_t err = kernels::launch_decode_mfma(
             pool->layer(layer), m->view, plan, static_cast<const uint16_t *>(queries),

@@ -62,7 +62,7 @@ enum MetaKind { kNone = 0, kPrefill = 1, kDecode = 2, kSlots = 3 };
 // The arrays of one upload in the metadata buffer.  Ordinary uploads pack
 // them back to back; with fixed launch shapes each has a fixed offset.
 enum Region {
-    kRegCounts = 0,  // [4]: split-K work items, rows to reduce (read by the kernels); the same of fine_plan
+    kRegCounts = 0,  // [4]: split-K work items, rows to reduce (read by the kernels); the same of own_plan
     kRegTableOff,
     kRegTables,
     kRegRowSeq,
@@ -197,7 +197,7 @@ struct vo_step_meta {
     uint64_t head_dim = 0;
 
     uint64_t max_seqs = 0, max_rows = 0, max_entries = 0, max_heads = 0, max_parts = 0;
-    uint64_t fine_slots = 0;  // partial slots of fine_plan
+    uint64_t fine_slots = 0;  // partial slots of an own_plan with fine items
 
     vo::MetaKind kind = vo::kNone;
     uint64_t block_size = 0;
@@ -225,8 +225,8 @@ struct vo_step_meta {
     hipStream_t side = nullptr;
     hipEvent_t fork = nullptr, join = nullptr;
 
-    // Split-K partials (fp32): max_parts slots of `plan`, then fine_slots of
-    // `fine_plan`, so that a launch of one leaves the other's alone.
+    // Split-K partials (fp32): max_parts slots of `plan`, then fine_slots of a
+    // plan of fine items, so that a launch of one leaves the other's alone.
     float *d_part_acc = nullptr;
     float *d_part_ml = nullptr;
 
@@ -235,11 +235,10 @@ struct vo_step_meta {
     vo::kernels::WritePlan write_plan{};      // runs of consecutive slots inside one block
     // The decode plan of any launch: whole splits, merged by the reduce kernel.
     vo::kernels::DecodePlan plan{};
-    // What launches that follow one another take instead (launch_plan): the
-    // same plan with its rows merged in the launch by way of these counters,
-    // or, for a step of few rows, `fine_plan`.  Null and off otherwise.
-    uint32_t *arrivals = nullptr;
-    vo::kernels::DecodePlan fine_plan{};
+    // What launches that follow one another take instead (launch_plan), if its
+    // arrivals are not null: the same plan with its rows merged in the launch,
+    // or, for a step of few rows, the longer ones as fine items as well.
+    vo::kernels::DecodePlan own_plan{};
     // The stream of the last upload, to compare a launch's with; never used as
     // a stream.
     void *upload_stream = nullptr;
