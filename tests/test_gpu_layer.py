@@ -137,8 +137,38 @@ def test_streaming_matmul_shapes(vo, gpu_backend, rows, n, k):
         assert torch.equal(b16, got.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("rows,n,k,own", [
+    (17, 4096, 4096, True), (33, 4096, 4096, False), (33, 4096, 2048, True), (16, 4112, 1024, True),
+    (17, 4112, 1024, True), (33, 4112, 1024, True), (48, 4112, 4096, True), (49, 4112, 4096, False),
+    (64, 4112, 3072, True), (16, 8192, 1024, True), (32, 8192, 1024, True), (48, 8192, 1024, True),
+    (64, 8192, 1024, True), (16, 8192, 6144, True), (16, 7168, 6144, False), (1, 8208, 6144, False),
+    (1, 16400, 6144, True), (4, 16400, 6144, True), (5, 8208, 6144, False), (4, 8208, 5120, False), (32, 8208, 4096, True),
+    (33, 8208, 4096, False), (16, 16384, 5120, True), (17, 16384, 5120, False), (9, 2048, 8192, False),
+    (8, 2048, 8192, True), (16, 4096, 5120, True), (5, 4096, 6144, False), (4, 4096, 6144, True),
+    (17, 65552, 4096, True), (64, 65552, 4096, True)])
+def test_product_kernel_rule(vo, gpu_backend, rows, n, k, own):
+    """Both sides of each line between the kernels of products of few rows and
+    the library, and the workgroup shapes that meet there: the kernel that
+    runs, and its sums (f32 sums of k products in any order, below 1e-5 of the
+    largest output)."""
+    import torch
+    _say(f"product rule {rows}x{k} . {n}x{k}^T")
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows + n + k)
+    x = torch.randn((rows, k), generator=gen, device="cuda:0").to(torch.bfloat16)
+    w = (0.02 * torch.randn((n, k), generator=gen, device="cuda:0")).to(torch.bfloat16)
+    vo.profile_reset()
+    vo.enable_profiling(True)
+    got = gpu_backend.matmul(x, w, out_dtype=torch.float32)
+    torch.cuda.synchronize()
+    vo.enable_profiling(False)
+    assert ("matmul_skinny" in vo.profile()) == own
+    want = x.double() @ w.double().T
+    assert (got - want).abs().max() < 1e-5 * want.abs().max()
+
+
 @pytest.mark.parametrize("rows", [1, 16, 17, 48, 64, 65])
-@pytest.mark.parametrize("ffn,k", [(16, 512), (24, 512), (2064, 1024), (2576, 1536), (4112, 512),
+@pytest.mark.parametrize("ffn,k", [(16, 512), (24, 512), (2064, 1024), (2576, 1536), (4096, 512), (4112, 512),
                                    (12304, 512), (32784, 512)])
 def test_matmul_silu_mul_shapes(vo, gpu_backend, rows, ffn, k):
     """SwiGLU in the gate/up product: each workgroup shape with a remainder of

@@ -408,8 +408,8 @@ __device__ __forceinline__ floatx4 swiglu4(floatx4 g, floatx4 u) {
     return t;
 }
 
-// Backend::matmul for few rows and a small weight (up to 2^24 values):
-// streaming the weight is the whole cost.  A workgroup owns 16 / P weight rows
+// Backend::matmul for few rows (skinny_kernel has which): streaming the weight
+// is the whole cost.  A workgroup owns 16 / P weight rows
 // (outputs) and splits K over its 8 wavefronts and, within one, over P parts;
 // each wavefront runs v_mfma_f32_16x16x32_bf16 with A = P blocks of 16 / P
 // weight rows, block p from part p of its columns, and B = x^T laid out alike
@@ -425,15 +425,15 @@ __device__ __forceinline__ floatx4 swiglu4(floatx4 g, floatx4 u) {
 // P = 1 (up to 4 rows), 8 steps of loads in flight: here, in the order of one
 // launch and one round of loads, it beats stream_gemm_kernel below (a weight
 // of 3072 x 2048, 4 rows: 5.1 against 5.8 us; 4096 x 4096: 8.7 against 9.4);
-// on larger weights, or with more rows, every workgroup's reads of x from L2
-// make it the slower one.
+// on larger weights of up to 4096 columns, or with more rows, every workgroup's
+// reads of x from L2 make it the slower one.
 // P = 2 (up to 8 rows): weights of at most 2048 rows, whose 128 tiles of 16
 // leave half the 256 CUs idle: a weight of 2048 x 8192, 4 rows, took 13.4 us
 // with P = 1 and takes 9.1 (3.7 TB/s); 2048 x 2048 4.9 and 4.0.  P = 4 adds
 // nothing (10.2, 4.6), and 2 steps in flight do as well as 4 to 16 (9.2-9.5).
 // From 3072 rows on P = 1 is the better one (5.0 against 5.3).
 constexpr int kSkinnyWaves = 8;
-constexpr uint64_t kSkinnyWeight = 1ull << 24;  // largest weight
+constexpr uint64_t kSkinnyWeight = 1ull << 24;  // largest small weight
 constexpr uint32_t kSkinnyHalfN = 2048;         // largest weight rows of P = 2
 
 template <int MODE, int P, int U>
@@ -495,8 +495,10 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(
 //
 // Workgroup b starts its walk over K at chunk b mod (chunks), so that the
 // workgroups do not all read the same lines of x, or the same columns of
-// their weight rows, at once; the order in which an output's products are
-// added depends on the shape and the output's column only.  Weight loads
+// their weight rows, at once.  The order in which an output's products are
+// added depends on the weight's shape, the output's column and which instance
+// runs (launch_stream_rows), so on the number of rows, not on what the
+// other rows hold.  Weight loads
 // are ordinary ones (see skinny_gemm_kernel).
 //
 // MODE 3 is the gate and up projections with SwiGLU: the weight is [gate; up],
@@ -509,7 +511,8 @@ __global__ __launch_bounds__(64 * kSkinnyWaves) void skinny_gemm_kernel(
 // Measured, rows 16 / 40 / 64, against the library product it stands in for:
 // 28672 x 4096: 42.6 / 49.1 / 47.7 us, library 59.6 / 51.1 / 52.2 (5.5 TB/s
 // at 16 rows); 128256 x 2048: 94.8 / 99.9 / 110 us, library 117 / 124 / 130;
-// 6144 x 4096: 13.3 / 16.4 / 18.7 us, library 14.1 / 16.8 / 17.3.
+// 6144 x 4096: 13.3 / 16.4 us, library 14.1 / 16.8 (64 rows 18.7 and 17.3: the
+// library's, see skinny_kernel).
 template <int MODE, int MT, int NW, int KG, int KC>
 __global__ __launch_bounds__(64 * NW * KG) void stream_gemm_kernel(
     const uint16_t *__restrict__ x, const uint16_t *__restrict__ w, uint32_t rows, uint32_t n,
@@ -870,29 +873,29 @@ void launch_stream(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t
 #undef VO_STREAM
 }
 
-// The workgroup's shape, by how many 16-row weight tiles there are: enough
-// workgroups for the 256 CUs, then as many tiles to a workgroup as that
-// leaves (each shares x once more).  Measured over 2048 .. 128256 weight rows:
-// 4 tiles with 256-column chunks from 8192 rows on (the narrower splits of K
-// lose 1-5% there, and 8 tiles leave CUs idle below 24576: 20.9 against 15.6
-// us at 16384 x 2048, 40 rows); 8 tiles for a vocabulary's worth of rows and
-// more than one batch tile (99.9 against 114 us at 128256 x 2048, 40 rows)
-// and for 4 batch tiles from 24576 on (47.7 against 55.2 us at 28672 x
-// 4096); 2 tiles and 4 groups from 5120 on (13.3 against 18.3 us at 6144 x
-// 4096, 16 rows); below that 1 tile and 8 groups, with 2 and 4 where the
-// stages of 3 or 4 batch tiles would not fit, or where tiles come in pairs.
+// The workgroup's shape, by how many 16-row weight tiles there are.  While they
+// last, a workgroup to each of the 256 CUs and no second round: 1 tile and 8
+// groups up to 4096 weight rows, 2 tiles and 4 groups up to 8192 (16 rows of
+// x, 4608 x 4096: 13.0 us, with 1 tile 15.2; 8192 x 8192: 31.4, with 4 tiles
+// 38.6; 10240 x 8192: 47.2, with 4 tiles 41.0).  Past that 4 tiles with 256-column chunks (each
+// shares x once more); 8 for a vocabulary's worth of rows and more than one
+// batch tile (99.9 against 114 us at 128256 x 2048, 40 rows; 348 against 392
+// at 128256 x 8192, 32 rows; but rows of 8 KiB want 4: 128256 x 4096, 17 rows 227 with 8 and
+// 183 with 4, 3584 and 4608 columns not) and for 4 batch tiles from 24576
+// on (47.7 against 55.2 us at 28672 x 4096).  3 and 4 batch tiles, whose stages
+// would not fit 8 groups, and tiles in pairs run 2 and 4 below 8192 too.
 template <int MT>
 void launch_stream_rows(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
                         uint32_t k, void *out, int mode, hipStream_t stream) {
-    if (n >= 8192) {
+    if (n > 8192) {
         if constexpr (MT > 1)
-            if (n >= 65536) return launch_stream<MT, 8, 1, 256>(x, w, rows, n, k, out, mode, stream);
+            if (n >= 65536 && k != 4096) return launch_stream<MT, 8, 1, 256>(x, w, rows, n, k, out, mode, stream);
         if constexpr (MT == 4)
             if (n >= 24576) return launch_stream<MT, 8, 1, 128>(x, w, rows, n, k, out, mode, stream);
         return launch_stream<MT, 4, 1, 256>(x, w, rows, n, k, out, mode, stream);
     }
     if constexpr (MT <= 2) {
-        if (n >= 5120) return launch_stream<MT, 2, 4, 128>(x, w, rows, n, k, out, mode, stream);
+        if (n > 4096) return launch_stream<MT, 2, 4, 128>(x, w, rows, n, k, out, mode, stream);
         if (mode != 3) return launch_stream<MT, 1, 8, 64>(x, w, rows, n, k, out, mode, stream);
     }
     return launch_stream<MT, 2, 4, 64>(x, w, rows, n, k, out, mode, stream);
@@ -1041,24 +1044,81 @@ hipError_t launch_matmul_generic(const uint16_t *x, const uint16_t *w, uint32_t 
 namespace vo {
 namespace kernels {
 
-// The weight-streaming kernels take up to 64 rows.  Past 16 rows a weight
-// with more than twice as many columns as rows stays with the library: each
-// workgroup then reads more of x than of the weight (4096 x 14336: 32.5 / 49 us at
-// 32 / 40 rows, library 30.7 / 35.3; at 16 rows 26.5 against 25.9, and the
-// call costs the host 6 us less).
+namespace {
+
+enum SkinnyKernel { kLibrary, kHalves, kWhole, kStream };
+
+// Which kernel runs a product of few rows, from times of weights of 1024 to
+// 128256 rows and 2048 to 28672 columns (GPU us a call, replayed from a graph
+// over weights that are not cached; own kernels / library):
+//  - skinny_gemm_kernel: small weights (above), and up to 4 rows of weights of
+//    more than 4096 columns and 16384 to 65536 rows: 16384 x 8192, 1 row 51.8,
+//    stream 64.7, library 65.5; 57344 x 8192 162, 187, 178; but 8192 x 28672
+//    92.8, 85.6, 88.4, 10240 x 8192 38.1, 42.0, 36.0, 128256 x 8192, 4 rows 388,
+//    360, 363.
+//  - up to 16 rows stream: 4096 x 4096 9.9 / 12.7, 6144 x 4096 13.7 / 14.5, 16384 x
+//    2048 14.9 / 17.7, 28672 x 4096 45.0 / 63.0, 8192 x 14336 45.9 / 51.7.  Not
+//    past 5120 columns where the tiles leave CUs idle (2048 x 8192 15.1 / 13.1,
+//    4096 x 14336 27.8 / 27.0, 6144 x 8192 24.8 / 23.2), or 4096 below 16384 rows
+//    (10240 x 8192 40.9 / 35.6) and past 32768 (128256 x 8192 372 / 359).
+//  - 17 to 64 rows, where every workgroup stages more of x: the line is at
+//    fewer columns the more rows there are.  4096 x 2048, 64 rows 10.9 / 12.0; 4096 x
+//    4096, 32 rows 11.6 / 13.1, 33 rows 15.8 / 13.3; 6144 x 3072, 64 rows 16.6 / 17.5;
+//    6144 x 4096, 48 rows 17.4 / 17.3, 64 rows 19.0 / 17.9; 8192 x 8192, 32 rows 31.7 /
+//    30.2; 12288 x 4096, 32 rows 23.3 / 23.6, 48 rows 25.6 / 24.9; 28672 x 4096, 64 rows
+//    50.9 / 56.0; 32768 x 5120, 32 rows 66.8 / 60.5; 128256 x 8192, 32 rows 349 / 381.
+// The library costs the host 6 us more a call, which decides where both are
+// within 3% (5120 .. 7168 x 4096 at 24 and 32 rows).
+SkinnyKernel skinny_kernel(uint64_t rows, uint64_t n, uint64_t k) {
+    if (rows < 1 || rows > 64 || n < 16 || n % 16 != 0 || n / 16 > 0x7fffffffull || k < 512 ||
+        k % 512 != 0 || k > (1u << 24))
+        return kLibrary;
+    const bool small = n * k <= kSkinnyWeight;
+    if (small && rows <= 8 && n <= kSkinnyHalfN && k % (kSkinnyWaves * 2 * 32 * 2) == 0) return kHalves;
+    if (rows <= 4 && k % (kSkinnyWaves * 32 * 8) == 0 && (small || (n >= 16384 && n <= 65536 && k > 4096)))
+        return kWhole;
+    bool stream;
+    if (rows <= 16) {
+        if (n <= 4096)
+            stream = k <= 5120 || (rows <= 4 && k % 2048 == 0);
+        else if (n <= 8192)
+            stream = k <= 5120 || n > 7168 || rows <= 4;
+        else
+            stream = k <= 4096 || (n >= 16384 && n <= 32768 && k <= 8192);
+    } else if (k > 2 * n) {
+        stream = false;
+    } else if (n <= 4096) {
+        stream = k <= (rows <= 32 ? 4096 : 2048);
+    } else if (n <= 8192) {
+        stream = k <= (rows <= 48 ? 4096 : 3072);
+    } else if (n < 16384) {
+        stream = k <= (rows <= 32 ? 4096 : 2048);
+    } else {
+        stream = k <= 4096 || n >= 98304;
+    }
+    return stream ? kStream : kLibrary;
+}
+
+}  // namespace
+
 bool skinny_gemm_supported(uint64_t rows, uint64_t n, uint64_t k) {
-    return rows >= 1 && rows <= 64 && n >= 16 && n % 16 == 0 && k >= 512 && k % 512 == 0 &&
-           k <= (1u << 24) && n / 16 <= 0x7fffffffull && (rows <= 16 || k <= 2 * n);
+    return skinny_kernel(rows, n, k) != kLibrary;
+}
+
+bool swiglu_gemm_supported(uint64_t rows, uint64_t ffn, uint64_t k) {
+    const SkinnyKernel kernel = skinny_kernel(rows, 2 * ffn, k);
+    return ffn % 16 == 0 && kernel != kLibrary && (kernel != kWhole || 2 * ffn * k <= kSkinnyWeight);
 }
 
 hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
                               uint32_t k, void *out, bool out_f32, bool accumulate,
                               hipStream_t stream) {
-    if (!skinny_gemm_supported(rows, n, k)) return hipErrorInvalidValue;
+    const SkinnyKernel kernel = skinny_kernel(rows, n, k);
+    if (kernel == kLibrary) return hipErrorInvalidValue;
     KernelTimer timer("matmul_skinny", stream);
     const int mode = !out_f32 ? 0 : (accumulate ? 2 : 1);
-    if (static_cast<uint64_t>(n) * k <= kSkinnyWeight) {
-        const dim3 block(64 * kSkinnyWaves);
+    if (kernel == kStream) return launch_stream_any(x, w, rows, n, k, out, mode, stream);
+    const dim3 block(64 * kSkinnyWaves);
 #define VO_SKINNY(P, U)                                                                          \
     do {                                                                                         \
         const dim3 grid(n / 16 * P);                                                             \
@@ -1071,13 +1131,13 @@ hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t row
         else                                                                                     \
             hipLaunchKernelGGL((skinny_gemm_kernel<2, P, U>), grid, block, 0, stream, x, w, rows, \
                                n, k, out);                                                       \
-        return hipGetLastError();                                                                \
     } while (0)
-        if (rows <= 8 && n <= kSkinnyHalfN && k % (kSkinnyWaves * 2 * 32 * 2) == 0) VO_SKINNY(2, 2);
-        if (rows <= 4 && k % (kSkinnyWaves * 32 * 8) == 0) VO_SKINNY(1, 8);
+    if (kernel == kHalves)
+        VO_SKINNY(2, 2);
+    else
+        VO_SKINNY(1, 8);
 #undef VO_SKINNY
-    }
-    return launch_stream_any(x, w, rows, n, k, out, mode, stream);
+    return hipGetLastError();
 }
 
 // Up to 8 rows of 2048 values, 4 for a weight of 8192 rows and more, where
@@ -1127,7 +1187,7 @@ hipError_t launch_norm_qkv_rope(const float *x, const uint16_t *norm, float eps,
 
 hipError_t launch_swiglu_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t ffn,
                               uint32_t k, uint16_t *out, hipStream_t stream) {
-    if (ffn % 16 != 0 || !skinny_gemm_supported(rows, 2ull * ffn, k)) return hipErrorInvalidValue;
+    if (!swiglu_gemm_supported(rows, ffn, k)) return hipErrorInvalidValue;
     KernelTimer timer("matmul_swiglu", stream);
     return launch_stream_any(x, w, rows, 2 * ffn, k, out, 3, stream);
 }

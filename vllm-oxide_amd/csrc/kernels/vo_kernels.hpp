@@ -138,14 +138,15 @@ hipError_t launch_silu_mul(const uint16_t *gate, uint32_t gate_ld, const uint16_
                            uint32_t out_ld, bool vec8, hipStream_t stream);
 hipError_t launch_argmax(const void *logits, bool f32, uint32_t rows, uint32_t cols, uint32_t *ids,
                          hipStream_t stream);
-// Weight-streaming GEMM for 1..64 rows (decode batches): n % 16 == 0,
-// k % 512 == 0, and past 16 rows k <= 2 n.
+// Weight-streaming GEMM for 1..64 rows (decode batches): n % 16 == 0 and
+// k % 512 == 0, where it is faster than the library (skinny_kernel).
 bool skinny_gemm_supported(uint64_t rows, uint64_t n, uint64_t k);
 hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
                               uint32_t k, void *out, bool out_f32, bool accumulate,
                               hipStream_t stream);
 // The same for a weight [gate; up] of 2 * ffn rows (ffn % 16 == 0) with SwiGLU:
 // out [rows, ffn] = silu(x . gate^T) * (x . up^T).
+bool swiglu_gemm_supported(uint64_t rows, uint64_t ffn, uint64_t k);
 hipError_t launch_swiglu_gemm(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t ffn,
                               uint32_t k, uint16_t *out, hipStream_t stream);
 // RMSNorm of x [rows, k] f32 by norm, then the product with w [n, k], out bf16

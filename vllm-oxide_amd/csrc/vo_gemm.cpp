@@ -360,9 +360,9 @@ extern "C" int32_t vo_matmul_silu_mul(vo_gemm *g, const void *x, uint64_t rows, 
     // The decode-sized batches of whole tiles: one launch, nothing in gate_up.
     // Every other form, and every argument the two steps refuse, goes to them.
     const uint64_t ob = rows * ffn * 2;
-    if (skinny_on() && x && weight && out && in_features == x_cols && ffn % 16 == 0 &&
+    if (skinny_on() && x && weight && out && in_features == x_cols &&
         aligned16(x) && aligned16(weight) && aligned16(out) &&
-        kernels::skinny_gemm_supported(rows, 2 * ffn, in_features) &&
+        kernels::swiglu_gemm_supported(rows, ffn, in_features) &&
         !overlaps(out, ob, x, rows * x_cols * 2) &&
         !overlaps(out, ob, weight, 2 * ffn * in_features * 2)) {
         DeviceGuard guard(g->device);
