@@ -729,6 +729,48 @@ def test_decode_packs_merge_bitwise(vo, monkeypatch, rows, in_launch):
     _assert_close(got, W.oracle_attention(orc, wl), f"packs, {rows} rows")
 
 
+@pytest.mark.parametrize("hd,prefix,ctx,fine", [
+    (128, 0, [500, 511], False), (128, 0, [500, 512], True), (64, 0, [900, 1023], False),
+    (64, 0, [900, 1024], True), (128, 0, [700] * 17, False), (128, 0, [700] * 16, True),
+    (128, 1024, [1100, 1324, 1536], True), (64, 1024, [1100, 1324, 1536], True),
+    (128, 2048, [2100, 2324], False)])
+def test_decode_fine_item_rule(vo, monkeypatch, hd, prefix, ctx, fine):
+    """Which steps run their longer rows as fine items (the launch's name tells):
+    both sides of the row length of each head dimension, of the number of
+    workgroups that run at once (8 KV heads), behind a shared prefix without
+    packs (shorter than a split) and with them.  Bitwise what whole splits
+    and the reduce kernel give, write_kv in the launch too.  With the merge in
+    the launch off, neither runs."""
+    import torch
+    _say(f"decode fine rule hd={hd} prefix={prefix} ctx={ctx}")
+    backend = vo.HipBackend(device=0, max_seqs=32, max_rows=W.FILL_ROWS, max_table_entries=4096,
+                            max_query_heads=32)
+    wl = W.build(vo, backend, kind="decode", heads=32, kv_heads=8, head_dim=hd, block_size=16,
+                 num_blocks=1400, context_lens=ctx, seed=hd + len(ctx), shared_prefix=prefix,
+                 shared_count=len(ctx) if prefix else 0)
+    outs = []
+    for fine_env, arrive_env in (("", ""), ("0", ""), ("", "0"), ("0", "0")):
+        for key, value in (("VO_DECODE_FINE", fine_env), ("VO_DECODE_ARRIVE", arrive_env)):
+            monkeypatch.setenv(key, value)
+        backend.step_meta(wl.pool).holds = None
+        vo.profile_reset()
+        vo.enable_profiling(True)
+        outs.append(_bits(_out(wl, backend)))
+        torch.cuda.synchronize()
+        vo.enable_profiling(False)
+        expect = "decode_splitk_fine" if fine and not fine_env and not arrive_env else "decode_splitk"
+        reduced = max(ctx) >= 2048 and (arrive_env or prefix >= 2048)
+        assert set(vo.profile()) == {expect} | ({"decode_reduce"} if reduced else set())
+    for got in outs[1:]:
+        assert np.array_equal(got, outs[0])
+    monkeypatch.delenv("VO_DECODE_FINE")
+    monkeypatch.delenv("VO_DECODE_ARRIVE")
+    backend.step_meta(wl.pool).holds = None
+    fused = backend.decode_attention_write_kv(wl.q, wl.k_new, wl.v_new, wl.pool, 0, wl.meta)
+    assert np.array_equal(_bits(fused), outs[0])
+    _assert_close(fused.float().cpu().numpy(), W.oracle_attention(orc, wl), f"fine rule {ctx}")
+
+
 def test_decode_batch_invariance_bitwise(vo, gpu_backend):
     """A row's output is identical alone or in a batch (the reference's
     batch-invariance invariant, CLAUDE.md; model.rs:539-584)."""

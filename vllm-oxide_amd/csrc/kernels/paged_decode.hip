@@ -38,7 +38,7 @@
 // either way and batch invariance holds.  Bound: a wavefront's chain of
 // chunks (over 1 us each from HBM) and the number of CUs that read at all.
 // Two rows of 5000-8100 keys of 8 KV heads of 128 dims are 64 whole items: 25.5 us,
-// and 13.8 as 220 fine ones, of a 53 MB read; one row of 8000 keys 27 and
+// and 13.9 as 220 fine ones, of a 53 MB read; one row of 8000 keys 27 and
 // 13.8 us a call.  Fine items give rows of one split partials too, so only the
 // launches that the metadata knows to follow one another run them; any other
 // takes the whole items, with the same bits.

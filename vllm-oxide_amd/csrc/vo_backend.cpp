@@ -526,17 +526,23 @@ bool canonical_decode_rows(vo_step_meta *m) {
     return true;
 }
 
-// Fine items (one state of a split per workgroup, paged_decode.hip): for
-// plans of fewer than decode_fine_limit workgroups, the rows of more than
-// kFineMinKeys keys.  Measured a call, whole / fine: 8 rows of 1000-2000 keys
-// of 128 dims (64 workgroups) 24.2 / 17.2 us, 16 of 1500-2000 (128) 28.5 /
-// 25.5, but 24 of them (192) 32.9 / 37.1 and 16 of 1100-4000 (200) 36.0 /
-// 36.7: past five eighths of the CUs the whole items already draw what the
-// HBM gives, and the fine ones only add partials.  One row of 1100 keys:
-// 14.4 / 11.1 us at 128 dims, 11.0 / 11.2 at 64, where a split's chain of
-// chunks is as short as the merge is long.  VO_DECODE_FINE overrides the
-// limit (0: off; a tuning knob, read per plan and at creation).
-constexpr uint64_t kFineMinKeys = 1024;
+// Fine items (one state of a split per workgroup, paged_decode.hip): in plans of
+// fewer than decode_fine_limit workgroups, the longer rows.  Measured (GPU us a
+// call, replayed from a graph; whole / fine): 16 rows of 1200-2000 keys of 8 KV heads
+// of 128 dims (128 workgroups) 23.7 / 19.3, 19 of them (152) 25.0 / 24.0, but
+// 24 (192) 32.9 / 37.1 a call: past five eighths of the CUs the whole items
+// already draw what the HBM gives, and the fine ones only add partials.
+// VO_DECODE_FINE overrides the limit (0: off; a tuning knob, read per plan and
+// at creation).
+//
+// How long a row, by the head dimension: a whole item's chain of chunks is
+// twice as long at 128 dims.  At 64 a row of 600 / 900 / 1100 keys takes 5.4 /
+// 6.6 / 7.2 whole and 6.2 / 6.3 / 6.3 fine, 12 rows of 600-1000 7.6 / 7.8: past 1024 keys.
+// At 128 7.9 / 10.0 / 11.4 and 7.2 / 7.3 / 7.5, one of 500 6.7 / 7.1, 16 of 600-1000 13.4 / 11.6:
+// past 512, as long as all items run at once (two workgroups to a CU): 19
+// rows of 600-1000 14.8 / 16.4, and 13.8 with only those past 1024 fine.
+constexpr uint64_t kFineKeys = 1024;
+constexpr uint64_t kFineKeys128 = 512;
 
 uint64_t decode_fine_limit(uint64_t num_cus) {
     const int env = env_int("VO_DECODE_FINE", -1);
@@ -581,20 +587,31 @@ void finish_work_records(const vo_step_meta *m, uint32_t *work, uint64_t n, uint
 }
 
 // The fine plan of a step of few rows, beside m->plan (already made, without
-// packs): the longer rows as fine items, the others as m->plan has them, in an
+// packs; 4 rows of 1100-1300 keys behind a shared prefix of 1024, 128 dims: 12.3 us
+// whole, 7.8 fine): the longer rows as fine items, the others as m->plan has them, in an
 // order of their own; fine items, short chains of work, come last.
 void plan_fine_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32_t> *rows,
                     const uint32_t *whole_work) {
     const uint64_t T = m->num_rows, L = m->plan.split_keys;
     const uint64_t R = rows ? rows->size() : T;
     auto row_at = [&](uint64_t i) -> uint64_t { return rows ? (*rows)[i] : i; };
-    auto fine_row = [](uint64_t keys) { return keys > kFineMinKeys; };
+    uint64_t min_keys = m->head_dim == 128 ? kFineKeys128 : kFineKeys;
+    auto fine_row = [&](uint64_t keys) { return keys > min_keys; };
     uint64_t items = 0;
     bool any = false;
-    for (uint64_t i = 0; i < R; ++i) {
-        const uint64_t nk = m->row_num_keys[row_at(i)];
-        any |= fine_row(nk);
-        items += fine_row(nk) ? fine_items(nk, L) : row_splits(nk, L);
+    auto count = [&]() {
+        items = 0;
+        any = false;
+        for (uint64_t i = 0; i < R; ++i) {
+            const uint64_t nk = m->row_num_keys[row_at(i)];
+            any |= fine_row(nk);
+            items += fine_row(nk) ? fine_items(nk, L) : row_splits(nk, L);
+        }
+    };
+    count();
+    if (items * m->kv_heads > 2 * static_cast<uint64_t>(m->num_cus) && min_keys < kFineKeys) {
+        min_keys = kFineKeys;
+        count();
     }
     if (!any) return;
     kernels::DecodePlan &p = m->own_plan;
@@ -781,11 +798,12 @@ vo_status plan_decode_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32
     }
     // What launches that follow one another add (launch_plan): the merge in
     // the launch, for plans without one-tile packs on four wavefronts (with
-    // shared packs, merge_packs_in_launch), and fine items, which also need splits they can cover, partial slots, and no
-    // blocks that several rows read (packs serve those).
+    // shared packs, merge_packs_in_launch), and fine items, which also need
+    // splits they can cover, partial slots and no packs (a kernel of packs has
+    // no fine items).
     m->own_plan = kernels::DecodePlan{};
     if (!pk.fixed() && waves == 4 && decode_arrive()) {
-        if (streaming && L % 128 == 0 && L <= kernels::kMaxFineSplit && 4 * parts <= m->fine_slots &&
+        if (P == 1 && L % 128 == 0 && L <= kernels::kMaxFineSplit && 4 * parts <= m->fine_slots &&
             parts * m->kv_heads < decode_fine_limit(m->num_cus))
             plan_fine_rows(m, pk, rows, work);
         if (!m->own_plan.fine && nred != 0 &&
