@@ -143,8 +143,8 @@ def test_streaming_matmul_shapes(vo, gpu_backend, rows, n, k):
     (64, 4112, 3072, True), (16, 8192, 1024, True), (32, 8192, 1024, True), (48, 8192, 1024, True),
     (64, 8192, 1024, True), (16, 8192, 6144, True), (16, 7168, 6144, False), (1, 8208, 6144, False),
     (1, 16400, 6144, True), (4, 16400, 6144, True), (5, 8208, 6144, False), (4, 8208, 5120, False), (32, 8208, 4096, True),
-    (33, 8208, 4096, False), (16, 16384, 5120, True), (17, 16384, 5120, False), (9, 2048, 8192, False),
-    (8, 2048, 8192, True), (16, 4096, 5120, True), (5, 4096, 6144, False), (4, 4096, 6144, True),
+    (33, 8208, 4096, False), (16, 16384, 5120, True), (17, 16384, 5120, False), (9, 2048, 8192, True),
+    (8, 2048, 8192, True), (16, 4096, 8192, True), (12, 4096, 8704, True), (13, 4096, 8704, False),
     (17, 65552, 4096, True), (64, 65552, 4096, True)])
 def test_product_kernel_rule(vo, gpu_backend, rows, n, k, own):
     """Both sides of each line between the kernels of products of few rows and

@@ -1058,17 +1058,21 @@ enum SkinnyKernel { kLibrary, kHalves, kWhole, kStream };
 //    360, 363.
 //  - up to 16 rows stream: 4096 x 4096 9.9 / 12.7, 6144 x 4096 13.7 / 14.5, 16384 x
 //    2048 14.9 / 17.7, 28672 x 4096 45.0 / 63.0, 8192 x 14336 45.9 / 51.7.  Not
-//    past 5120 columns where the tiles leave CUs idle (2048 x 8192 15.1 / 13.1,
-//    4096 x 14336 27.8 / 27.0, 6144 x 8192 24.8 / 23.2), or 4096 below 16384 rows
-//    (10240 x 8192 40.9 / 35.6) and past 32768 (128256 x 8192 372 / 359).
+//    past 5120 columns where the tiles leave CUs idle (6144 x 8192 24.8 / 23.2),
+//    or 4096 below 16384 rows (10240 x 8192 40.9 / 35.6) and past 32768 (128256 x
+//    8192 372 / 359).  Up to 4096 weight rows the library's 6 us more of host
+//    time a call count: an MLP of 2048 x 8192 and 9 to 16 rows takes 45.8 us with
+//    this kernel (15.1 alone, the library 13.1) and 54.6; 4096 x 14336, 12 rows 26.5 / 26.4,
+//    the MLP 73.2 and 74.0, 16 rows 27.8 / 27.0, 75.2 and 74.6 (4096 x 11264, 12
+//    rows, 21.7 / 20.1 is on the wrong side of that line).
 //  - 17 to 64 rows, where every workgroup stages more of x: the line is at
 //    fewer columns the more rows there are.  4096 x 2048, 64 rows 10.9 / 12.0; 4096 x
 //    4096, 32 rows 11.6 / 13.1, 33 rows 15.8 / 13.3; 6144 x 3072, 64 rows 16.6 / 17.5;
 //    6144 x 4096, 48 rows 17.4 / 17.3, 64 rows 19.0 / 17.9; 8192 x 8192, 32 rows 31.7 /
 //    30.2; 12288 x 4096, 32 rows 23.3 / 23.6, 48 rows 25.6 / 24.9; 28672 x 4096, 64 rows
 //    50.9 / 56.0; 32768 x 5120, 32 rows 66.8 / 60.5; 128256 x 8192, 32 rows 349 / 381.
-// The library costs the host 6 us more a call, which decides where both are
-// within 3% (5120 .. 7168 x 4096 at 24 and 32 rows).
+// The host time also decides 5120 .. 7168 x 4096 at 24 and 32 rows, where both
+// are within 3%.
 SkinnyKernel skinny_kernel(uint64_t rows, uint64_t n, uint64_t k) {
     if (rows < 1 || rows > 64 || n < 16 || n % 16 != 0 || n / 16 > 0x7fffffffull || k < 512 ||
         k % 512 != 0 || k > (1u << 24))
@@ -1080,7 +1084,7 @@ SkinnyKernel skinny_kernel(uint64_t rows, uint64_t n, uint64_t k) {
     bool stream;
     if (rows <= 16) {
         if (n <= 4096)
-            stream = k <= 5120 || (rows <= 4 && k % 2048 == 0);
+            stream = k <= 8192 || rows <= 12;
         else if (n <= 8192)
             stream = k <= 5120 || n > 7168 || rows <= 4;
         else
