@@ -9,7 +9,7 @@ disjoint slices of a seeded permutation of a 20000-block pool.
 One step = what the engine does per layer for this batch
 (crates/engine/src/model.rs:309-319): write_kv of the 64 new tokens
 (reshape_and_cache), then decode_attention over ctx + 1 keys per sequence
-(split-K kernel + reduce kernel).  Steps alternate between two pool layers
+(split-K, its partials merged in the launch).  Steps alternate between two pool layers
 (2.6 GB) so that the 256 MB MALL cannot serve one step's KV from the last.
 
 value = algorithmic decode bytes per step / step time, in GB/s, where the
@@ -222,7 +222,7 @@ def bench_decode(vo, W, orc, args, cfg):
             "seqs": S, "query_heads": heads, "kv_heads": kvh, "head_dim": hd, "block_size": bs,
             "pool_blocks": cfg["num_blocks"], "context": cfg["ctx_desc"],
             "keys_total": int(wl.row_num_keys().sum()),
-            "step": ("write_kv(new tokens) + decode_attention (split-K + reduce)" +
+            "step": ("write_kv(new tokens) + decode_attention (split-K, partials merged)" +
                      (", two calls" if args.unfused else
                       ", one call: vo_decode_attention_write_kv")),
             "layers_rotated": layers,

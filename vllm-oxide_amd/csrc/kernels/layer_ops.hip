@@ -730,30 +730,26 @@ __global__ __launch_bounds__(64 * NW * KG) void norm_gemm_kernel(
     // the row's last 8, not used).
     floatx4 v[2 * KJ];
     u32x4 g[KJ];
-    auto load_row = [&](uint32_t row) __attribute__((always_inline)) {
-        const float *p = x + static_cast<uint64_t>(row) * k;
-#pragma unroll
-        for (int j = 0; j < KJ; ++j) {
-            const uint32_t c = min(512 * j + 8 * lane, k - 8);
-            v[2 * j] = *reinterpret_cast<const floatx4 *>(p + c);
-            v[2 * j + 1] = *reinterpret_cast<const floatx4 *>(p + c + 4);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
     uint32_t pos = 0, slot = 0;
     if constexpr (ROPE) {
         pos = to.positions[min(r, rows - 1)];
         slot = to.slots[min(r, rows - 1)];
     }
-    load_row(min(wave, rows - 1));
+    const float *xr = x + static_cast<uint64_t>(min(wave, rows - 1)) * k;
+#pragma unroll
+    for (int j = 0; j < KJ; ++j) {
+        const uint32_t c = min(512 * j + 8 * lane, k - 8);
+        v[2 * j] = *reinterpret_cast<const floatx4 *>(xr + c);
+        v[2 * j + 1] = *reinterpret_cast<const floatx4 *>(xr + c + 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < KJ; ++j)
         g[j] = *reinterpret_cast<const u32x4 *>(norm + min(512 * j + 8 * lane, k - 8));
     __builtin_amdgcn_sched_barrier(0);
     u32x4 a0[U], a1[U];
     load_w(a0, 0);
-    for (uint32_t row = wave; row < rows; row += W) {
-        if (row != wave) load_row(row);
+    if (wave < rows) {  // a wavefront for each row (norm_gemm_supported)
         float ss = 0.0f;
 #pragma unroll
         for (int j = 0; j < KJ; ++j)
@@ -775,7 +771,7 @@ __global__ __launch_bounds__(64 * NW * KG) void norm_gemm_kernel(
                     o[e] = wf[e] * (v[2 * j][e] * inv_rms);
                     o[4 + e] = wf[4 + e] * (v[2 * j + 1][e] * inv_rms);
                 }
-                *reinterpret_cast<u32x4 *>(xs + (row * upr + ((64 * j + lane) ^ (row & 15))) * 16) =
+                *reinterpret_cast<u32x4 *>(xs + (wave * upr + ((64 * j + lane) ^ (wave & 15))) * 16) =
                     pack8(o);
             }
     }
@@ -873,17 +869,18 @@ void launch_stream(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t
 #undef VO_STREAM
 }
 
-// The workgroup's shape, by how many 16-row weight tiles there are.  While they
-// last, a workgroup to each of the 256 CUs and no second round: 1 tile and 8
-// groups up to 4096 weight rows, 2 tiles and 4 groups up to 8192 (16 rows of
+// The workgroup's shape, by how many 16-row weight tiles there are.  While
+// they last, a workgroup to each of the 256 CUs and no second round: 1 tile and
+// 8 groups up to 4096 weight rows, 2 tiles and 4 groups up to 8192 (16 rows of
 // x, 4608 x 4096: 13.0 us, with 1 tile 15.2; 8192 x 8192: 31.4, with 4 tiles
-// 38.6; 10240 x 8192: 47.2, with 4 tiles 41.0).  Past that 4 tiles with 256-column chunks (each
-// shares x once more); 8 for a vocabulary's worth of rows and more than one
-// batch tile (99.9 against 114 us at 128256 x 2048, 40 rows; 348 against 392
-// at 128256 x 8192, 32 rows; but rows of 8 KiB want 4: 128256 x 4096, 17 rows 227 with 8 and
-// 183 with 4, 3584 and 4608 columns not) and for 4 batch tiles from 24576
-// on (47.7 against 55.2 us at 28672 x 4096).  3 and 4 batch tiles, whose stages
-// would not fit 8 groups, and tiles in pairs run 2 and 4 below 8192 too.
+// 38.6; 10240 x 8192: 47.2, with 4 tiles 41.0).  Past that 4 tiles with
+// 256-column chunks (each shares x once more); 8 for a vocabulary's worth of
+// rows and more than one batch tile (99.9 against 114 us at 128256 x 2048, 40
+// rows; 348 against 392 at 128256 x 8192, 32 rows; but weight rows of 8 KiB
+// want 4: 128256 x 4096, 17 rows 227 with 8 and 183 with 4, 3584 and 4608
+// columns not) and for 4 batch tiles from 24576 on (47.7 against 55.2 us at
+// 28672 x 4096).  3 and 4 batch tiles, whose stages would not fit 8 groups,
+// and tiles in pairs run 2 and 4 below 4096 too.
 template <int MT>
 void launch_stream_rows(const uint16_t *x, const uint16_t *w, uint32_t rows, uint32_t n,
                         uint32_t k, void *out, int mode, hipStream_t stream) {
@@ -1050,27 +1047,30 @@ enum SkinnyKernel { kLibrary, kHalves, kWhole, kStream };
 
 // Which kernel runs a product of few rows, from times of weights of 1024 to
 // 128256 rows and 2048 to 28672 columns (GPU us a call, replayed from a graph
-// over weights that are not cached; own kernels / library):
+// over weights that are not cached; own kernel / library):
 //  - skinny_gemm_kernel: small weights (above), and up to 4 rows of weights of
 //    more than 4096 columns and 16384 to 65536 rows: 16384 x 8192, 1 row 51.8,
 //    stream 64.7, library 65.5; 57344 x 8192 162, 187, 178; but 8192 x 28672
-//    92.8, 85.6, 88.4, 10240 x 8192 38.1, 42.0, 36.0, 128256 x 8192, 4 rows 388,
-//    360, 363.
-//  - up to 16 rows stream: 4096 x 4096 9.9 / 12.7, 6144 x 4096 13.7 / 14.5, 16384 x
-//    2048 14.9 / 17.7, 28672 x 4096 45.0 / 63.0, 8192 x 14336 45.9 / 51.7.  Not
-//    past 5120 columns where the tiles leave CUs idle (6144 x 8192 24.8 / 23.2),
-//    or 4096 below 16384 rows (10240 x 8192 40.9 / 35.6) and past 32768 (128256 x
-//    8192 372 / 359).  Up to 4096 weight rows the library's 6 us more of host
-//    time a call count: an MLP of 2048 x 8192 and 9 to 16 rows takes 45.8 us with
-//    this kernel (15.1 alone, the library 13.1) and 54.6; 4096 x 14336, 12 rows 26.5 / 26.4,
-//    the MLP 73.2 and 74.0, 16 rows 27.8 / 27.0, 75.2 and 74.6 (4096 x 11264, 12
-//    rows, 21.7 / 20.1 is on the wrong side of that line).
+//    92.8, 85.6, 88.4, 10240 x 8192 38.1, 42.0, 36.0, 128256 x 8192, 4 rows
+//    388, 360, 363.
+//  - up to 16 rows stream_gemm_kernel: 4096 x 4096 9.9 / 12.7, 6144 x 4096
+//    13.7 / 14.5, 16384 x 2048 14.9 / 17.7, 28672 x 4096 45.0 / 63.0, 8192 x
+//    14336 45.9 / 51.7.  Not past 5120 columns where the tiles leave CUs idle
+//    (6144 x 8192 24.8 / 23.2), or 4096 below 16384 rows (10240 x 8192 40.9 /
+//    35.6) and past 32768 (128256 x 8192 372 / 359).  Up to 4096 weight rows
+//    the library's 6 us more of host time a call count: an MLP, op by op, of
+//    2048 x 8192 and 9 to 16 rows takes 45.8 us with this kernel (15.1 alone,
+//    the library 13.1) and 54.6, though a whole decode step of 9 or 12
+//    sequences, bound by the GPU, 1229 and 1165; 4096 x 14336, 12 rows 26.5 /
+//    26.4, the MLP 73.2 and 74.0, 16 rows 27.8 / 27.0, 75.2 and 74.6.  (4096 x
+//    11264, 12 rows, 21.7 / 20.1, is on the wrong side of that line.)
 //  - 17 to 64 rows, where every workgroup stages more of x: the line is at
-//    fewer columns the more rows there are.  4096 x 2048, 64 rows 10.9 / 12.0; 4096 x
-//    4096, 32 rows 11.6 / 13.1, 33 rows 15.8 / 13.3; 6144 x 3072, 64 rows 16.6 / 17.5;
-//    6144 x 4096, 48 rows 17.4 / 17.3, 64 rows 19.0 / 17.9; 8192 x 8192, 32 rows 31.7 /
-//    30.2; 12288 x 4096, 32 rows 23.3 / 23.6, 48 rows 25.6 / 24.9; 28672 x 4096, 64 rows
-//    50.9 / 56.0; 32768 x 5120, 32 rows 66.8 / 60.5; 128256 x 8192, 32 rows 349 / 381.
+//    fewer columns the more rows there are.  4096 x 2048, 64 rows 10.9 / 12.0;
+//    4096 x 4096, 32 rows 11.6 / 13.1, 33 rows 15.8 / 13.3; 6144 x 3072, 64
+//    rows 16.6 / 17.5; 6144 x 4096, 48 rows 17.4 / 17.3, 64 rows 19.0 / 17.9;
+//    8192 x 8192, 32 rows 31.7 / 30.2; 12288 x 4096, 32 rows 23.3 / 23.6, 48
+//    rows 25.6 / 24.9; 28672 x 4096, 64 rows 50.9 / 56.0; 32768 x 5120, 32
+//    rows 66.8 / 60.5; 128256 x 8192, 32 rows 349 / 381.
 // The host time also decides 5120 .. 7168 x 4096 at 24 and 32 rows, where both
 // are within 3%.
 SkinnyKernel skinny_kernel(uint64_t rows, uint64_t n, uint64_t k) {
@@ -1145,10 +1145,11 @@ hipError_t launch_skinny_gemm(const uint16_t *x, const uint16_t *w, uint32_t row
 }
 
 // Up to 8 rows of 2048 values, 4 for a weight of 8192 rows and more, where
-// the product's own time hides less of them (figures at norm_gemm_kernel);
-// longer rows lose: 6144 x 4096, 1 and 4 rows, 19.3 and 20.2 us against 15.4 and
-// 15.8 as two launches, 28672 x 4096 with SwiGLU 46.0 and 45.2 against 46.2
-// and 46.3.
+// the product's own time hides less of them (figures at norm_gemm_kernel): as
+// many as the workgroup has wavefronts.  Longer rows lose or gain nothing:
+// 6144 x 4096, 1 and 4 rows, 19.3 and 20.2 us against 15.4 and 15.8 as two
+// launches; 28672 x 4096 with SwiGLU 46.0 and 45.2 against 46.2 and 46.3, no
+// more than runs differ.
 bool norm_gemm_supported(uint64_t rows, uint64_t n, uint64_t k, bool swiglu) {
     const uint32_t kg = n >= 8192 ? 1 : swiglu ? 4 : 8;
     return rows >= 1 && rows <= (n >= 8192 ? 4 : kNormGemmRows) && k >= 512 && k <= kNormGemmK &&

@@ -526,21 +526,22 @@ bool canonical_decode_rows(vo_step_meta *m) {
     return true;
 }
 
-// Fine items (one state of a split per workgroup, paged_decode.hip): in plans of
-// fewer than decode_fine_limit workgroups, the longer rows.  Measured (GPU us a
-// call, replayed from a graph; whole / fine): 16 rows of 1200-2000 keys of 8 KV heads
-// of 128 dims (128 workgroups) 23.7 / 19.3, 19 of them (152) 25.0 / 24.0, but
-// 24 (192) 32.9 / 37.1 a call: past five eighths of the CUs the whole items
-// already draw what the HBM gives, and the fine ones only add partials.
-// VO_DECODE_FINE overrides the limit (0: off; a tuning knob, read per plan and
-// at creation).
+// Fine items (one state of a split per workgroup, paged_decode.hip): in plans
+// of fewer than decode_fine_limit workgroups, the longer rows.  Measured (GPU
+// us a call, replayed from a graph; whole / fine): 16 rows of 1200-2000 keys
+// of 8 KV heads of 128 dims (128 workgroups) 23.7 / 19.3, 19 of them (152)
+// 25.0 / 24.0, but 24 (192) 32.9 / 37.1: past five eighths of the CUs the
+// whole items already draw what the HBM gives, and the fine ones only add
+// partials.  VO_DECODE_FINE overrides the limit (0: off; a tuning knob, read
+// per plan and at creation).
 //
 // How long a row, by the head dimension: a whole item's chain of chunks is
-// twice as long at 128 dims.  At 64 a row of 600 / 900 / 1100 keys takes 5.4 /
-// 6.6 / 7.2 whole and 6.2 / 6.3 / 6.3 fine, 12 rows of 600-1000 7.6 / 7.8: past 1024 keys.
-// At 128 7.9 / 10.0 / 11.4 and 7.2 / 7.3 / 7.5, one of 500 6.7 / 7.1, 16 of 600-1000 13.4 / 11.6:
-// past 512, as long as all items run at once (two workgroups to a CU): 19
-// rows of 600-1000 14.8 / 16.4, and 13.8 with only those past 1024 fine.
+// longer at 128 dims.  At 64 a row of 600 / 900 / 1100 keys takes 5.4 / 6.6 /
+// 7.2 whole and 6.2 / 6.3 / 6.3 fine, 12 rows of 600-1000 7.6 / 7.8: past 1024
+// keys.  At 128 they take 7.9 / 10.0 / 11.4 and 7.2 / 7.3 / 7.5, one of 500
+// 6.7 / 7.1, 16 rows of 600-1000 13.4 / 11.6: past 512, as long as all items
+// run at once (two workgroups to a CU): 19 rows of 600-1000 14.8 / 16.4, and
+// 13.8 with only those past 1024 fine.
 constexpr uint64_t kFineKeys = 1024;
 constexpr uint64_t kFineKeys128 = 512;
 
@@ -558,8 +559,8 @@ bool decode_arrive() { return env_int("VO_DECODE_ARRIVE", 1) != 0; }
 // reduce kernel takes all rows at once for a launch of 3 us.  Measured, merge
 // in the launch against the reduce kernel: 8 rows behind a 4096-key prefix at
 // 8 rows to a pack (32 / 8 heads) 44.7 / 39.7 us of 128 dims, 33.9 / 29.1 of
-// 64; at 4 to a pack (64 / 8 heads of 128) 42.4 / 40.0.  Only with packs of 4 and more
-// workgroups than two to a CU run at once do the rest of the workgroups hide
+// 64; at 4 to a pack (64 / 8 heads of 128) 42.4 / 40.0.  Only with packs of 4
+// and more workgroups than two to a CU run at once do the rest of them hide
 // it: 880 workgroups 90.2 / 90.7, 904 70.8 / 71.4, 1008 99.8 / 99.5, 1264
 // 137.6 / 144.2, 1536 109.9 / 113.0, 2048 156.7 / 159.9; but 768 57.6 / 56.6
 // (and at 8 to a pack 1152 73.3 / 69.5, 1536 110.4 / 112.8: no line there).
@@ -586,10 +587,10 @@ void finish_work_records(const vo_step_meta *m, uint32_t *work, uint64_t n, uint
     }
 }
 
-// The fine plan of a step of few rows, beside m->plan (already made, without
-// packs; 4 rows of 1100-1300 keys behind a shared prefix of 1024, 128 dims: 12.3 us
-// whole, 7.8 fine): the longer rows as fine items, the others as m->plan has them, in an
-// order of their own; fine items, short chains of work, come last.
+// The own plan of a step of few rows, beside m->plan (already made, without
+// packs): the longer rows as fine items, the others as m->plan has them; fine
+// items, short chains of work, come last.  (4 rows of 1100-1300 keys behind a
+// shared prefix of 1024, 128 dims: 12.3 us whole, 7.8 fine.)
 void plan_fine_rows(vo_step_meta *m, Packer &pk, const std::vector<uint32_t> *rows,
                     const uint32_t *whole_work) {
     const uint64_t T = m->num_rows, L = m->plan.split_keys;
