@@ -748,7 +748,9 @@ def test_decode_fine_item_rule(vo, monkeypatch, hd, prefix, ctx, fine):
     wl = W.build(vo, backend, kind="decode", heads=32, kv_heads=8, head_dim=hd, block_size=16,
                  num_blocks=1400, context_lens=ctx, seed=hd + len(ctx), shared_prefix=prefix,
                  shared_count=len(ctx) if prefix else 0)
-    outs = []
+    outs, others = [], []
+    gen = torch.Generator(device="cuda:0").manual_seed(hd)
+    q2 = torch.randn(wl.q.shape, generator=gen, device="cuda:0").to(torch.bfloat16)
     for fine_env, arrive_env in (("", ""), ("0", ""), ("", "0"), ("0", "0")):
         for key, value in (("VO_DECODE_FINE", fine_env), ("VO_DECODE_ARRIVE", arrive_env)):
             monkeypatch.setenv(key, value)
@@ -761,8 +763,14 @@ def test_decode_fine_item_rule(vo, monkeypatch, hd, prefix, ctx, fine):
         expect = "decode_splitk_fine" if fine and not fine_env and not arrive_env else "decode_splitk"
         reduced = max(ctx) >= 2048 and (arrive_env or prefix >= 2048)
         assert set(vo.profile()) == {expect} | ({"decode_reduce"} if reduced else set())
+        for _ in range(3):  # other queries in between: no partial is left over
+            others.append(_bits(backend.decode_attention(q2, wl.pool, 0, wl.meta)))
+            assert np.array_equal(_bits(_out(wl, backend)), outs[-1])
     for got in outs[1:]:
         assert np.array_equal(got, outs[0])
+    for got in others[1:]:
+        assert np.array_equal(got, others[0])
+    assert not np.array_equal(others[0], outs[0])
     monkeypatch.delenv("VO_DECODE_FINE")
     monkeypatch.delenv("VO_DECODE_ARRIVE")
     backend.step_meta(wl.pool).holds = None
